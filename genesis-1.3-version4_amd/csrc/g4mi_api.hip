@@ -30,6 +30,33 @@ namespace g4mi {
 thread_local std::string g_last_error;
 void set_error(const std::string &msg) { g_last_error = msg; }
 
+// The ADI's tables for one step size on one grid: Thomas factors, and the
+// banded inverse where a kernel's half width holds it.
+struct AdiPlan {
+    double cstep = 0;
+    int tile = 0;     // 8 or 16: window of the fused recurrence kernel; 0: not eligible
+    int band_m = 0;   // 7, 8, 12 or 16: half width of the banded-inverse kernel; 0: not eligible
+    int klo = 0, khi = -1;  // rows sharing the central band row
+    double2 *fac = nullptr, *band = nullptr;  // one allocation: c | cbet | cwet, then the band
+};
+// The spectral solver's tables for one step size: the convolution's kernel
+// transform and, once a GEMM needs it, the propagator matrix.
+struct FftPlan {
+    double2 *hk = nullptr, *m = nullptr;
+};
+// Tables by step size.  A line has a few distinct step sizes (its modules,
+// quadrupoles and drift pieces) that alternate, so each is built once per
+// context; the oldest goes when the cache is full (plans_room).
+template <class Plan>
+struct PlanCache {
+    std::vector<std::pair<double, Plan>> plans;
+    Plan *find(double delz) {
+        for (auto &e : plans)
+            if (e.first == delz) return &e.second;
+        return nullptr;
+    }
+};
+
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -48,7 +75,6 @@ struct Ctx {
            *d_rmax = nullptr, *d_efield = nullptr;
     double2 *d_field = nullptr, *d_work = nullptr, *d_src = nullptr;
     int4 *d_box = nullptr;
-    double2 *d_fac = nullptr;  // c | cbet | cwet, ngrid each
     int nblk = 0, blk_cap = 0;
     int *d_blk_slice = nullptr;
     long long *d_blk_begin = nullptr;
@@ -63,12 +89,10 @@ struct Ctx {
     // space charge
     int longrange = 0, sc_nz = 0, sc_nphi = 0, sc_ng = 100;
     double sc_rmax = 0;
-    // ADI factor cache and the kernels eligible for it
-    double adi_delz = 0, cstep = 0;
-    int adi_tile = 0;  // 8 or 16: window of the fused recurrence kernel; 0: not eligible
-    int adi_band_m = 0;  // 7, 8, 12 or 16: half width of the banded-inverse kernel; 0: not eligible
-    int adi_klo = 0, adi_khi = -1;  // rows sharing the central band row
-    double2 *d_band = nullptr;
+    // ADI tables per step size and the current step's
+    PlanCache<AdiPlan> adi_plans;
+    double adi_delz = std::nan("");
+    AdiPlan adi;
     double *d_tilediag = nullptr;
     // field diagnostics sums written by the fused ADI of the last field
     // step, and the storage slices slippage has zeroed since then
@@ -90,13 +114,12 @@ struct Ctx {
     // picks the faster); the convolution's length and tables per delz
     int fft_prop = -1, fft_conv_L = 0;
     float fft_conv_ms = -1.f;
-    double2 *d_fft_hk = nullptr, *d_fft_tw = nullptr;
+    double2 *d_fft_tw = nullptr;
     // Bluestein DFT tables (forward, inverse): [L] kernel transform, then [ng] chirp
     double2 *d_fft_bf = nullptr, *d_fft_bi = nullptr;
     double fft_xc = 1, fft_yc = 1, fft_sig = 1;
-    bool fft_ready = false;
-    double fft_delz = 0;
-    double2 *d_fft_m = nullptr, *d_fft_w = nullptr, *d_fft_wc = nullptr, *d_fft_u = nullptr,
+    PlanCache<FftPlan> fft_plans;
+    double2 *d_fft_w = nullptr, *d_fft_wc = nullptr, *d_fft_u = nullptr,
             *d_fft_v = nullptr;
     double *d_fft_sig = nullptr, *d_fft_mom = nullptr, *d_fft_mompart = nullptr;
     // incoherent synchrotron radiation (Incoherent): the host's uniform
@@ -115,10 +138,9 @@ struct Ctx {
     struct HField {
         int harm = 1, ng = 0;
         double gridmax = 0, dgrid = 0, xks = 0;
-        double2 *d_field = nullptr, *d_work = nullptr, *d_src = nullptr, *d_fac = nullptr;
+        double2 *d_field = nullptr, *d_work = nullptr, *d_src = nullptr;
         int4 *d_box = nullptr;
-        double fac_delz = 0, cstep = 0;
-        bool fac_ready = false;
+        PlanCache<AdiPlan> plans;
     };
     std::vector<HField> hf;
     // records of g4mi_run waiting for the host: their per-slice sums sit in
@@ -291,73 +313,110 @@ static void build_block_table(const std::vector<long long> &off, std::vector<int
         }
 }
 
-static int ensure_factors(Ctx *c, double delz) {
-    if (delz == c->adi_delz) return G4MI_OK;  // FieldSolverADI::init caching on delz
-    c->adi_delz = delz;
-    std::vector<double> h(6 * (size_t)c->ng);
-    c->cstep = adi_factors(c->ng, delz, c->dgrid, c->xks, h.data(), h.data() + 2 * c->ng,
-                           h.data() + 4 * c->ng);
+constexpr size_t kPlanBytes = 64u << 20;  // of one cache of plans
+constexpr size_t kPlanMax = 32;
+
+static void plan_free(AdiPlan &p) { (void)hipFree(p.fac); }
+static void plan_free(FftPlan &p) {
+    (void)hipFree(p.hk);
+    (void)hipFree(p.m);
+}
+template <class Plan>
+static void plans_free(PlanCache<Plan> &pc) {
+    for (auto &e : pc.plans) plan_free(e.second);
+    pc.plans.clear();
+}
+// Room for a plan of `bytes`: the oldest plans go, once the stream no longer
+// reads them.
+template <class Plan>
+static int plans_room(Ctx *c, PlanCache<Plan> &pc, size_t bytes) {
+    const size_t cap = std::min(kPlanMax, std::max<size_t>(2, kPlanBytes / std::max<size_t>(1, bytes)));
+    while (pc.plans.size() >= cap) {
+        G4_HIP(hipStreamSynchronize(c->stream));
+        plan_free(pc.plans.front().second);
+        pc.plans.erase(pc.plans.begin());
+    }
+    return G4MI_OK;
+}
+
+// FieldSolverADI::init for one grid and step size, kept in `pc`.
+static int adi_plan(Ctx *c, PlanCache<AdiPlan> &pc, int ng, double dgrid, double xks, double delz, AdiPlan *out) {
+    if (const AdiPlan *have = pc.find(delz)) {
+        *out = *have;
+        return G4MI_OK;
+    }
+    AdiPlan p;
+    std::vector<double> h(6 * (size_t)ng);
+    p.cstep = adi_factors(ng, delz, dgrid, xks, h.data(), h.data() + 2 * ng, h.data() + 4 * ng);
     // Window of the fused kernel: a back-substitution started T cells early
     // is off by at most max|cwet|^(T+1) relative; accept it below 2^-66.
     double wmax = 0;
-    for (int i = 0; i < c->ng; i++)
-        wmax = std::max(wmax, std::hypot(h[4 * c->ng + 2 * i], h[4 * c->ng + 2 * i + 1]));
+    for (int i = 0; i < ng; i++) wmax = std::max(wmax, std::hypot(h[4 * ng + 2 * i], h[4 * ng + 2 * i + 1]));
     const double bound = std::ldexp(1.0, -66);
-    c->adi_tile = 0;
-    if (c->ng <= 256) {
-        if (std::pow(wmax, 9) < bound) c->adi_tile = 8;
-        else if (std::pow(wmax, 17) < bound) c->adi_tile = 16;
+    if (ng <= 256) {
+        if (std::pow(wmax, 9) < bound) p.tile = 8;
+        else if (std::pow(wmax, 17) < bound) p.tile = 16;
     }
     // banded inverse: accept the narrowest band whose dropped entries are
     // all below 2^-60 of the diagonal (1/128 ulp of the result)
-    c->adi_band_m = 0;
+    const AdiInverse inv(ng, h.data(), h.data() + 2 * ng, h.data() + 4 * ng);
+    const double tiny = std::ldexp(1.0, -60);
     for (int m : {7, 8, 12, 16}) {
-        std::vector<double> band(2 * (size_t)c->ng * (2 * m + 1));
-        const double worst = adi_band(c->ng, h.data(), h.data() + 2 * c->ng,
-                                      h.data() + 4 * c->ng, m, band.data());
-        if (worst < std::ldexp(1.0, -60)) {
-            // interior rows whose band equals the central row's to 2^-60
-            const int W = 2 * m + 1, kc = c->ng / 2;
-            auto same = [&](int k) {
-                double d = 0, dia = std::hypot(band[2 * ((size_t)kc * W + m)], band[2 * ((size_t)kc * W + m) + 1]);
-                for (int q = 0; q < W; q++)
-                    d = std::max(d, std::hypot(band[2 * ((size_t)k * W + q)] - band[2 * ((size_t)kc * W + q)],
-                                               band[2 * ((size_t)k * W + q) + 1] - band[2 * ((size_t)kc * W + q) + 1]));
-                return d <= std::ldexp(1.0, -60) * dia;
-            };
-            int lo = kc, hi = kc;
-            while (lo > 0 && same(lo - 1)) lo--;
-            while (hi < c->ng - 1 && same(hi + 1)) hi++;
-            // the kernel takes the band of row (klo+khi)/2: keep the range centred
-            const int half = std::min(kc - lo, hi - kc);
-            c->adi_klo = kc - half;
-            c->adi_khi = kc + half;
-            if (c->d_band) (void)hipFree(c->d_band);
-            c->d_band = nullptr;
-            G4_HIP(hipMalloc(&c->d_band, band.size() * sizeof(double)));
-            G4_HIP(hipMemcpy(c->d_band, band.data(), band.size() * sizeof(double),
-                             hipMemcpyHostToDevice));
-            if (!c->d_tilediag)
-                G4_HIP(hipMalloc(&c->d_tilediag,
-                                 (size_t)c->ns * adi_band_tiles(c->ng) * 8 * sizeof(double)));
-            c->adi_band_m = m;
-            break;
-        }
+        if (!(inv.beyond(m) < tiny)) continue;
+        std::vector<double> band(2 * (size_t)ng * (2 * m + 1));
+        inv.band(m, band.data());
+        // interior rows whose band equals the central row's to 2^-60
+        const int W = 2 * m + 1, kc = ng / 2;
+        const double dia = std::hypot(band[2 * ((size_t)kc * W + m)], band[2 * ((size_t)kc * W + m) + 1]);
+        auto same = [&](int k) {
+            double d = 0;
+            for (int q = 0; q < W; q++)
+                d = std::max(d, std::hypot(band[2 * ((size_t)k * W + q)] - band[2 * ((size_t)kc * W + q)],
+                                           band[2 * ((size_t)k * W + q) + 1] - band[2 * ((size_t)kc * W + q) + 1]));
+            return d <= tiny * dia;
+        };
+        int lo = kc, hi = kc;
+        while (lo > 0 && same(lo - 1)) lo--;
+        while (hi < ng - 1 && same(hi + 1)) hi++;
+        // the kernel takes the band of row (klo+khi)/2: keep the range centred
+        const int half = std::min(kc - lo, hi - kc);
+        p.klo = kc - half;
+        p.khi = kc + half;
+        p.band_m = m;
+        h.insert(h.end(), band.begin(), band.end());
+        break;
     }
+    G4_TRY(plans_room(c, pc, h.size() * sizeof(double)));
+    G4_HIP(hipMalloc(&p.fac, h.size() * sizeof(double)));
+    if (hipMemcpy(p.fac, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
+        plan_free(p);
+        set_error("copying the ADI tables failed");
+        return G4MI_E_HIP;
+    }
+    p.band = p.band_m ? p.fac + 3 * (size_t)ng : nullptr;
+    pc.plans.emplace_back(delz, p);
+    *out = p;
+    return G4MI_OK;
+}
+
+static int ensure_factors(Ctx *c, double delz) {
+    if (delz == c->adi_delz) return G4MI_OK;
+    c->adi_delz = std::nan("");  // until the new plan is there
+    G4_TRY(adi_plan(c, c->adi_plans, c->ng, c->dgrid, c->xks, delz, &c->adi));
+    c->adi_delz = delz;
+    if (c->adi.band_m && !c->d_tilediag)
+        G4_HIP(hipMalloc(&c->d_tilediag, (size_t)c->ns * adi_band_tiles(c->ng) * 8 * sizeof(double)));
     if (!c->adi_fixed) {
         // the tuner's choice for this step size, or tune it at the next field step
         auto it = c->adi_choice.find(delz);
         c->adi_kernel = it != c->adi_choice.end() ? it->second : -1;
     } else if (c->adi_kernel == 1 || c->adi_kernel == 2) {
-        if (!c->adi_tile) c->adi_kernel = -1;      // re-tune if no longer eligible
-    } else if (c->adi_kernel == 3 && !c->adi_band_m) {
+        if (!c->adi.tile) c->adi_kernel = -1;      // re-tune if no longer eligible
+    } else if (c->adi_kernel == 3 && !c->adi.band_m) {
         c->adi_kernel = -1;
-    } else if (c->adi_kernel == 4 && !adi_wide64_ok(c->ng, c->adi_band_m, c->adi_klo, c->adi_khi)) {
+    } else if (c->adi_kernel == 4 && !adi_wide64_ok(c->ng, c->adi.band_m, c->adi.klo, c->adi.khi)) {
         c->adi_kernel = -1;
     }
-    G4_HIP(hipMemcpyAsync(c->d_fac, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice,
-                          c->stream));
-    G4_HIP(hipStreamSynchronize(c->stream));
     return G4MI_OK;
 }
 
@@ -483,15 +542,15 @@ static int beam_track(Ctx *c, const g4mi_step_params &st, double gamma0, double 
 // writes `fout`, the others work in place using `fout` as scratch).
 static void adi_launch(Ctx *c, int kind, const AdiFactors &f, double2 *fin, double2 *fout) {
     if (kind == 4)
-        (void)launch_adi_wide64(c->stream, c->ns, fin, fout, c->d_src, c->d_box, c->d_band, c->cstep, c->ng,
-                                c->first, c->adi_band_m, c->adi_klo, c->adi_khi, c->d_diag_f);
+        (void)launch_adi_wide64(c->stream, c->ns, fin, fout, c->d_src, c->d_box, c->adi.band, c->adi.cstep, c->ng,
+                                c->first, c->adi.band_m, c->adi.klo, c->adi.khi, c->d_diag_f);
     else if (kind == 3)
-        launch_adi_band(c->stream, c->ns, fin, fout, c->d_src, c->d_box, c->d_band, c->cstep,
-                        c->ng, c->first, c->adi_band_m, c->adi_klo, c->adi_khi, c->d_tilediag,
+        launch_adi_band(c->stream, c->ns, fin, fout, c->d_src, c->d_box, c->adi.band, c->adi.cstep,
+                        c->ng, c->first, c->adi.band_m, c->adi.klo, c->adi.khi, c->d_tilediag,
                         c->d_diag_f);
     else if (kind == 1 || kind == 2)
         launch_adi_fused(c->stream, c->ns, fin, fout, c->d_src, c->d_box, f, c->first,
-                         c->d_diag_f, c->adi_tile, kind == 2);
+                         c->d_diag_f, c->adi.tile, kind == 2);
     else
         launch_adi(c->stream, c->ns, fin, fout, c->d_src, c->d_box, f, c->first);
 }
@@ -512,9 +571,9 @@ static int tune_adi(Ctx *c, const AdiFactors &f) {
     float best_ms = 1e30f;
     for (int kind = 0; kind < 5; kind++) {
         c->adi_ms[kind] = -1.f;
-        if ((kind == 1 || kind == 2) && !c->adi_tile) continue;
-        if (kind == 3 && !c->adi_band_m) continue;
-        if (kind == 4 && !adi_wide64_ok(c->ng, c->adi_band_m, c->adi_klo, c->adi_khi)) continue;
+        if ((kind == 1 || kind == 2) && !c->adi.tile) continue;
+        if (kind == 3 && !c->adi.band_m) continue;
+        if (kind == 4 && !adi_wide64_ok(c->ng, c->adi.band_m, c->adi.klo, c->adi.khi)) continue;
         adi_launch(c, kind, f, scratch, c->d_work);  // warm-up
         float best = 1e30f;
         for (int rep = 0; rep < 3; rep++) {
@@ -547,7 +606,7 @@ static int tune_adi(Ctx *c, const AdiFactors &f) {
 // Tuner of the complex GEMM: each variant runs the row product E M^T of the
 // current field into the work buffer (which the step overwrites anyway)
 // and the fastest is kept for both products of every later step.
-static int tune_fft(Ctx *c) {
+static int tune_fft(Ctx *c, const FftPlan &p) {
     hipEvent_t e0, e1;
     G4_HIP(hipEventCreate(&e0));
     G4_HIP(hipEventCreate(&e1));
@@ -557,7 +616,7 @@ static int tune_fft(Ctx *c) {
     g.nrows = (long long)c->ns * c->ng;
     g.scale = 1.0;
     g.a = c->d_field;
-    g.mat = c->d_fft_m;
+    g.mat = p.m;
     g.c = c->d_work;
     int best = c->fft_variant;
     float best_ms = 1e30f;
@@ -589,7 +648,7 @@ static int tune_fft(Ctx *c) {
             ConvArgs a{};
             a.in = c->d_field;
             a.out = c->d_work;
-            a.hk = c->d_fft_hk;
+            a.hk = p.hk;
             a.tw = c->d_fft_tw;
             a.nrows = (long long)c->ns * c->ng;
             a.ng = c->ng;
@@ -618,38 +677,63 @@ static int tune_fft(Ctx *c) {
 static int ensure_bluestein(Ctx *c);
 static ConvArgs bluestein_pass(const Ctx *c, int sign, const double2 *in, double2 *out);
 
+static int ensure_twiddles(Ctx *c) {
+    if (c->d_fft_tw) return G4MI_OK;
+    const int L = fft_conv_length(c->ng);
+    std::vector<double> tw(2 * (size_t)L);
+    fft_twiddles(L, tw.data());
+    double2 *d = nullptr;
+    G4_TRY(dalloc(c, &d, L));
+    G4_HIP(hipMemcpy(d, tw.data(), tw.size() * sizeof(double), hipMemcpyHostToDevice));
+    c->d_fft_tw = d;
+    return G4MI_OK;
+}
+
+// FieldSolverFFT::init for a step size, kept in the context; the propagator
+// matrix is built only when the GEMMs run or are to be timed.
+static int fft_plan(Ctx *c, double delz, bool matrix, FftPlan *out) {
+    const size_t nn = (size_t)c->ng * c->ng;
+    FftPlan *have = c->fft_plans.find(delz);
+    if (have && (have->hk || !c->fft_conv_L) && (have->m || !matrix)) {
+        *out = *have;
+        return G4MI_OK;
+    }
+    const auto md = propagator_kernel(c->ng, c->dgrid, c->xks, delz);
+    if (!have) {
+        G4_TRY(plans_room(c, c->fft_plans, nn * sizeof(double2)));
+        c->fft_plans.plans.emplace_back(delz, FftPlan{});
+        have = &c->fft_plans.plans.back().second;
+    }
+    const int L = c->fft_conv_L;
+    if (L && !have->hk) {
+        std::vector<double> hk(2 * (size_t)L);
+        fft_conv_kernel(md, L, hk.data());
+        G4_HIP(hipMalloc(&have->hk, hk.size() * sizeof(double)));
+        G4_HIP(hipMemcpy(have->hk, hk.data(), hk.size() * sizeof(double), hipMemcpyHostToDevice));
+    }
+    if (matrix) {
+        std::vector<double> m(2 * nn);
+        fft_propagator(md, m.data());
+        G4_HIP(hipMalloc(&have->m, m.size() * sizeof(double)));
+        G4_HIP(hipMemcpy(have->m, m.data(), m.size() * sizeof(double), hipMemcpyHostToDevice));
+    }
+    *out = *have;
+    return G4MI_OK;
+}
+
 static int fft_field_step(Ctx *c, double delz) {
     const int ng = c->ng;
     const size_t nn = (size_t)ng * ng;
-    if (!c->d_fft_m) G4_TRY(dalloc(c, &c->d_fft_m, nn));
-    if (!c->fft_ready || delz != c->fft_delz) {  // FieldSolverFFT::init keeps delz per call
-        std::vector<double> m(2 * nn);
-        fft_propagator(ng, c->dgrid, c->xks, delz, m.data());
-        G4_HIP(hipMemcpyAsync(c->d_fft_m, m.data(), m.size() * sizeof(double), hipMemcpyHostToDevice,
-                              c->stream));
-        G4_HIP(hipStreamSynchronize(c->stream));
-        c->fft_conv_L = fft_conv_length(ng);
-        if (c->fft_conv_L) {
-            if (!c->d_fft_hk) {
-                G4_TRY(dalloc(c, &c->d_fft_hk, 512));
-                G4_TRY(dalloc(c, &c->d_fft_tw, 512));
-            }
-            std::vector<double> hk(2 * (size_t)c->fft_conv_L), tw(2 * (size_t)c->fft_conv_L);
-            fft_conv_tables(ng, c->dgrid, c->xks, delz, hk.data(), tw.data());
-            G4_HIP(hipMemcpyAsync(c->d_fft_hk, hk.data(), hk.size() * sizeof(double), hipMemcpyHostToDevice,
-                                  c->stream));
-            G4_HIP(hipMemcpyAsync(c->d_fft_tw, tw.data(), tw.size() * sizeof(double), hipMemcpyHostToDevice,
-                                  c->stream));
-            G4_HIP(hipStreamSynchronize(c->stream));
-        }
-        c->fft_delz = delz;
-        c->fft_ready = true;
-    }
+    c->fft_conv_L = fft_conv_length(ng);
+    if (c->fft_conv_L) G4_TRY(ensure_twiddles(c));
     if (c->fft_prop == 1 && !c->fft_conv_L) {
         set_error("fft_propagation 1: the FFT convolution supports ngrid <= 256");
         return G4MI_E_ARG;
     }
-    if (c->fft_variant < 0 || c->fft_prop < 0) G4_TRY(tune_fft(c));
+    const bool tune = c->fft_variant < 0 || c->fft_prop < 0;
+    FftPlan p;
+    G4_TRY(fft_plan(c, delz, tune || c->fft_prop != 1, &p));
+    if (tune) G4_TRY(tune_fft(c, p));
     CgemmArgs g{};
     g.ng = ng;
     g.ns = c->ns;
@@ -694,7 +778,7 @@ static int fft_field_step(Ctx *c, double delz) {
     }
     if (c->fft_prop == 1) {  // the same two products as FFT convolutions of every line
         ConvArgs a{};
-        a.hk = c->d_fft_hk;
+        a.hk = p.hk;
         a.tw = c->d_fft_tw;
         a.nrows = (long long)c->ns * ng;
         a.ng = ng;
@@ -715,7 +799,7 @@ static int fft_field_step(Ctx *c, double delz) {
         return launch_fft_conv_cols(c->stream, a);
     }
     g.a = c->d_field;  // T = E M^T
-    g.mat = c->d_fft_m;
+    g.mat = p.m;
     g.c = c->d_work;
     G4_TRY(launch_cgemm_rows(c->stream, g));
     g.b = c->d_work;  // E = M T + 2 (S or Y) of beam slice (s - first) mod Ns
@@ -735,14 +819,8 @@ static int fft_field_step(Ctx *c, double delz) {
 // and the two-kernel Thomas ADI with the field's own factors.
 static int harmonics_track(Ctx *c, const g4mi_step_params &st, double delz) {
     for (Ctx::HField &h : c->hf) {
-        if (!h.fac_ready || delz != h.fac_delz) {  // FieldSolverADI::init for this field
-            std::vector<double> f(6 * (size_t)h.ng);
-            h.cstep = adi_factors(h.ng, delz, h.dgrid, h.xks, f.data(), f.data() + 2 * h.ng, f.data() + 4 * h.ng);
-            G4_HIP(hipMemcpyAsync(h.d_fac, f.data(), f.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
-            G4_HIP(hipStreamSynchronize(c->stream));
-            h.fac_delz = delz;
-            h.fac_ready = true;
-        }
+        AdiPlan p;
+        G4_TRY(adi_plan(c, h.plans, h.ng, h.dgrid, h.xks, delz, &p));
         DepositParams d{};
         d.enabled = (st.aw > 0 && (h.harm % 2 == 1)) ? 1 : 0;
         d.harm = (double)h.harm;
@@ -759,7 +837,7 @@ static int harmonics_track(Ctx *c, const g4mi_step_params &st, double delz) {
         d.grady = st.grady;
         d.ngrid = h.ng;
         launch_deposit(c->stream, c->ns, c->d_off, c->d_g, c->d_th, c->d_x, c->d_y, c->d_cur, h.d_src, h.d_box, d);
-        AdiFactors f{h.d_fac, h.d_fac + h.ng, h.d_fac + 2 * h.ng, h.cstep, h.ng};
+        AdiFactors f{p.fac, p.fac + h.ng, p.fac + 2 * h.ng, p.cstep, h.ng};
         launch_adi(c->stream, c->ns, h.d_field, h.d_work, h.d_src, h.d_box, f, c->first);
     }
     G4_HIP(hipGetLastError());
@@ -800,7 +878,7 @@ static int field_track(Ctx *c, const g4mi_step_params &st, double delz, bool dep
         if (c->ev) G4_HIP(hipEventRecord(c->ev[7], c->stream));
         return G4MI_OK;
     }
-    AdiFactors f{c->d_fac, c->d_fac + c->ng, c->d_fac + 2 * c->ng, c->cstep, c->ng};
+    AdiFactors f{c->adi.fac, c->adi.fac + c->ng, c->adi.fac + 2 * c->ng, c->adi.cstep, c->ng};
     if (c->adi_kernel < 0) G4_TRY(tune_adi(c, f));
     adi_launch(c, c->adi_kernel, f, c->d_field, c->d_work);
     if (c->adi_kernel >= 3) std::swap(c->d_field, c->d_work);  // result is in the other buffer
@@ -1039,13 +1117,7 @@ static int ensure_bluestein(Ctx *c) {
     const int L = fft_conv_length(c->ng);
     if (!L) return G4MI_E_ARG;
     if (c->d_fft_bf) return G4MI_OK;
-    if (!c->d_fft_tw) {
-        G4_TRY(dalloc(c, &c->d_fft_hk, 512));
-        G4_TRY(dalloc(c, &c->d_fft_tw, 512));
-        std::vector<double> hk(2 * (size_t)L), tw(2 * (size_t)L);
-        (void)fft_conv_tables(c->ng, c->dgrid, c->xks, 1.0, hk.data(), tw.data());  // twiddles only
-        G4_HIP(hipMemcpy(c->d_fft_tw, tw.data(), tw.size() * sizeof(double), hipMemcpyHostToDevice));
-    }
+    G4_TRY(ensure_twiddles(c));
     double2 *bf = nullptr, *bi = nullptr;
     G4_TRY(dalloc(c, &bf, 512 + 256));
     G4_TRY(dalloc(c, &bi, 512 + 256));
@@ -1462,19 +1534,16 @@ static int mix_band(Ctx *c, double delz, int *band) {
     const double rtmp = adi_factors(ng, delz, c->dgrid, c->xks, h.data(), h.data() + 2 * ng,
                                     h.data() + 4 * ng);
     int need = -1, tm = 0;
-    for (int m = 1; m <= 12 && need < 0; m++) {
-        std::vector<double> tmp(2 * (size_t)ng * (2 * m + 1));
-        if (adi_band(ng, h.data(), h.data() + 2 * ng, h.data() + 4 * ng, m, tmp.data()) <
-            std::ldexp(1.0, -28))
-            need = m;
-    }
+    const AdiInverse inv(ng, h.data(), h.data() + 2 * ng, h.data() + 4 * ng);
+    for (int m = 1; m <= 12 && need < 0; m++)
+        if (inv.beyond(m) < std::ldexp(1.0, -28)) need = m;
     if (need < 0 || !mix_band_supported(need, &tm)) {
         set_error("mixed form: the step size needs a band wider than 12 cells");
         return G4MI_E_ARG;
     }
     const int W = 2 * tm + 1;
     std::vector<double> bd(2 * (size_t)ng * W);
-    (void)adi_band(ng, h.data(), h.data() + 2 * ng, h.data() + 4 * ng, tm, bd.data());
+    inv.band(tm, bd.data());
     // interior rows whose band equals the central row's to 2^-30 (FP32)
     const int kc = ng / 2;
     auto same = [&](int k) {
@@ -2296,7 +2365,7 @@ int g4mi_create(g4mi_ctx **out, int device, int nslice, const long long *off, in
         (rc = dalloc(c, &c->d_dr, ns)) || (rc = dalloc(c, &c->d_rmax, 1)) ||
         (rc = dalloc(c, &c->d_efield, ns)) || (rc = dalloc(c, &c->d_field, ns * cells)) ||
         (rc = dalloc(c, &c->d_work, ns * cells)) || (rc = dalloc(c, &c->d_src, ns * cells)) ||
-        (rc = dalloc(c, &c->d_box, ns)) || (rc = dalloc(c, &c->d_fac, 3 * (size_t)ngrid)) ||
+        (rc = dalloc(c, &c->d_box, ns)) || 
         (rc = dalloc(c, &c->d_diag_b, 8 * ns)) || (rc = dalloc(c, &c->d_diag_f, 8 * ns)) ||
         (rc = dalloc(c, &c->d_count, 1)) || (rc = dalloc(c, &c->d_beamsum, 8 * ns)) ||
         (rc = dalloc(c, &c->d_pbox, ns)) || (rc = dalloc(c, &c->d_pmaxf, ns)))
@@ -2330,7 +2399,9 @@ int g4mi_destroy(g4mi_ctx *h) {
     Ctx *c = &h->c;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (void *p : c->allocs) (void)hipFree(p);
-    if (c->d_band) (void)hipFree(c->d_band);
+    plans_free(c->adi_plans);
+    plans_free(c->fft_plans);
+    for (Ctx::HField &h : c->hf) plans_free(h.plans);
     if (c->d_tilediag) (void)hipFree(c->d_tilediag);
     if (c->m_steps) (void)hipFree(c->m_steps);
     mix_clear_graphs(c);
@@ -2437,7 +2508,6 @@ int g4mi_add_harmonic(g4mi_ctx *hc, int harm, int ngrid, double gridmax, int *in
     G4_TRY(dalloc(c, &h.d_field, cells));
     G4_TRY(dalloc(c, &h.d_work, cells));
     G4_TRY(dalloc(c, &h.d_src, cells));
-    G4_TRY(dalloc(c, &h.d_fac, 3 * (size_t)ngrid));
     G4_TRY(dalloc(c, &h.d_box, (size_t)c->ns));
     G4_HIP(hipMemsetAsync(h.d_field, 0, cells * sizeof(double2), c->stream));
     G4_HIP(hipStreamSynchronize(c->stream));
@@ -2640,7 +2710,6 @@ int g4mi_set_field_solver(g4mi_ctx *h, int fft, int filter, double xcut, double 
     c->fft_xc = xcut;
     c->fft_yc = ycut;
     c->fft_sig = sigmoid;
-    c->fft_ready = false;
     c->field_diag_fresh = false;
     if (c->fft_filter) {
         const size_t nn = (size_t)c->ng * c->ng;
@@ -3124,8 +3193,8 @@ int g4mi_get_schedule(g4mi_ctx *h, char *buf, int len) {
              "{\"field_solver\": \"adi\", \"adi_kernel\": %d, \"adi\": \"%s\", \"adi_window\": %d, "
              "\"adi_band_m\": %d, \"adi_tuned_ms\": [%.4f, %.4f, %.4f, %.4f, %.4f], \"adi_by_delz\": %s, "
              "\"fp64_fused\": %d}",
-             c->adi_kernel, c->adi_kernel >= 0 ? names[c->adi_kernel] : "untuned", c->adi_tile,
-             c->adi_band_m, c->adi_ms[0], c->adi_ms[1], c->adi_ms[2], c->adi_ms[3], c->adi_ms[4], bydz.c_str(),
+             c->adi_kernel, c->adi_kernel >= 0 ? names[c->adi_kernel] : "untuned", c->adi.tile,
+             c->adi.band_m, c->adi_ms[0], c->adi_ms[1], c->adi_ms[2], c->adi_ms[3], c->adi_ms[4], bydz.c_str(),
              fp64_fuse_on(c) ? 1 : 0);
     snprintf(buf, (size_t)len, "%s", tmp);
     return G4MI_OK;

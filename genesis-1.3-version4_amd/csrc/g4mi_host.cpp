@@ -152,41 +152,46 @@ double adi_factors(int ngrid, double delz, double dgrid, double xks, double *c, 
     return rtmp;
 }
 
-double adi_band(int ngrid, const double *c, const double *cbet, const double *cwet, int M,
-                double *band) {
+AdiInverse::AdiInverse(int ngrid, const double *c, const double *cbet, const double *cwet)
+    : n_(ngrid), inv_((size_t)ngrid * ngrid), rel_(ngrid, 0.0) {
     typedef std::complex<double> cd;
-    const int n = ngrid, W = 2 * M + 1;
-    std::vector<cd> C(n), B(n), Wt(n), col(n);
+    const int n = ngrid;
+    std::vector<cd> C(n), B(n), Wt(n);
     for (int i = 0; i < n; i++) {
         C[i] = cd(c[2 * i], c[2 * i + 1]);
         B[i] = cd(cbet[2 * i], cbet[2 * i + 1]);
         Wt[i] = cd(cwet[2 * i], cwet[2 * i + 1]);
     }
-    std::vector<cd> inv((size_t)n * n);
-    for (int j = 0; j < n; j++) {  // column j of A^-1: Thomas on e_j
-        for (int i = 0; i < n; i++) {
-            const cd r = (i == j) ? cd(1, 0) : cd(0, 0);
-            col[i] = (i == 0) ? r * B[0] : (r - C[i] * col[i - 1]) * B[i];
-        }
+    for (int j = 0; j < n; j++) {  // column j of A^-1: Thomas on e_j, zero above row j going down
+        cd *col = inv_.data() + (size_t)j * n;
+        col[j] = B[j];
+        for (int i = j + 1; i < n; i++) col[i] = (cd(0, 0) - C[i] * col[i - 1]) * B[i];
         for (int i = n - 2; i >= 0; i--) col[i] -= Wt[i + 1] * col[i + 1];
-        for (int i = 0; i < n; i++) inv[(size_t)i * n + j] = col[i];
     }
-    double worst = 0;
-    for (int k = 0; k < n; k++) {
-        const double diag = std::abs(inv[(size_t)k * n + k]);
-        for (int j = 0; j < n; j++) {
-            const int m = j - k + M;
-            if (m >= 0 && m < W) continue;
-            worst = std::max(worst, std::abs(inv[(size_t)k * n + j]) / diag);
+    std::vector<double> diag(n);
+    for (int k = 0; k < n; k++) diag[k] = std::abs(inv_[(size_t)k * n + k]);
+    for (int j = 0; j < n; j++)
+        for (int k = 0; k < n; k++) {
+            double &r = rel_[std::abs(j - k)];
+            r = std::max(r, std::abs(inv_[(size_t)j * n + k]) / diag[k]);
         }
+}
+
+double AdiInverse::beyond(int M) const {
+    double worst = 0;
+    for (int q = M + 1; q < n_; q++) worst = std::max(worst, rel_[q]);
+    return worst;
+}
+
+void AdiInverse::band(int M, double *band) const {
+    const int W = 2 * M + 1;
+    for (int k = 0; k < n_; k++)
         for (int m = 0; m < W; m++) {
             const int j = k + m - M;
-            const cd v = (j >= 0 && j < n) ? inv[(size_t)k * n + j] : cd(0, 0);
+            const std::complex<double> v = (j >= 0 && j < n_) ? inv_[(size_t)j * n_ + k] : 0.0;
             band[2 * ((size_t)k * W + m)] = v.real();
             band[2 * ((size_t)k * W + m) + 1] = v.imag();
         }
-    }
-    return worst;
 }
 
 namespace {
@@ -199,10 +204,26 @@ double fft_offset(int n, int k) {
 }  // namespace
 
 namespace {
+typedef std::complex<long double> cl;
+// a += b c without the library product's test for infinities
+inline void mul_add(cl &a, const cl &b, const cl &c) {
+    a += cl(b.real() * c.real() - b.imag() * c.imag(), b.real() * c.imag() + b.imag() * c.real());
+}
+// exp(sign 2 pi i k / n), k = 0 .. n-1
+std::vector<cl> unit_roots(int n, int sign) {
+    const long double twopi = 8.0L * atanl(1.0L);
+    std::vector<cl> w(n);
+    for (int k = 0; k < n; k++) {
+        const long double a = twopi * (long double)k / (long double)n;
+        w[k] = cl(cosl(a), sign * sinl(a));
+    }
+    return w;
+}
+}  // namespace
+
 // m[d] = (1/n) sum_k p_k exp(2 pi i k d / n), p_k = exp(i K2_1(k) delz), in
 // long double with the DFT exponents reduced mod n exactly
 std::vector<std::complex<long double>> propagator_kernel(int n, double dgrid, double xks, double delz) {
-    typedef std::complex<long double> cl;
     const double dk = 4. * asin(1.) / ((double)n * dgrid);
     std::vector<cl> p(n), md(n);
     for (int k = 0; k < n; k++) {
@@ -210,22 +231,17 @@ std::vector<std::complex<long double>> propagator_kernel(int n, double dgrid, do
         const double ph = -(dx * dx) * dk * dk / 2. / xks * delz;
         p[k] = cl(cos(ph), sin(ph));
     }
-    const long double twopi = 8.0L * atanl(1.0L);
+    const std::vector<cl> w = unit_roots(n, 1);
     for (int d = 0; d < n; d++) {
         cl acc(0, 0);
-        for (int k = 0; k < n; k++) {
-            const long double a = twopi * (long double)(((long long)k * d) % n) / (long double)n;
-            acc += p[k] * cl(cosl(a), sinl(a));
-        }
+        for (int k = 0; k < n; k++) mul_add(acc, p[k], w[((long long)k * d) % n]);
         md[d] = acc / (long double)n;
     }
     return md;
 }
-}  // namespace
 
-void fft_propagator(int n, double dgrid, double xks, double delz, double *m) {
-    typedef std::complex<long double> cl;
-    const std::vector<cl> md = propagator_kernel(n, dgrid, xks, delz);
+void fft_propagator(const std::vector<cl> &md, double *m) {
+    const int n = (int)md.size();
     for (int j = 0; j < n; j++)
         for (int l = 0; l < n; l++) {
             const cl v = md[((j - l) % n + n) % n];
@@ -240,37 +256,33 @@ int fft_conv_length(int n) {
     return (n >= 2 && L <= 512) ? L : 0;
 }
 
-int fft_conv_tables(int n, double dgrid, double xks, double delz, double *hk, double *tw) {
-    typedef std::complex<long double> cl;
-    const int L = fft_conv_length(n);
-    if (!L) return 0;
-    const std::vector<cl> md = propagator_kernel(n, dgrid, xks, delz);
-    const long double twopi = 8.0L * atanl(1.0L);
-    std::vector<cl> w(L);
+void fft_twiddles(int L, double *tw) {
+    const std::vector<cl> w = unit_roots(L, -1);
     for (int k = 0; k < L; k++) {
-        const long double a = twopi * (long double)k / (long double)L;
-        w[k] = cl(cosl(a), -sinl(a));
         tw[2 * k] = (double)w[k].real();
         tw[2 * k + 1] = (double)w[k].imag();
     }
+}
+
+void fft_conv_kernel(const std::vector<cl> &md, int L, double *hk) {
+    const int n = (int)md.size();
+    const std::vector<cl> w = unit_roots(L, -1);
     for (int k = 0; k < L; k++) {  // (1/L) sum over |d| < n of m[d mod n] exp(-2 pi i k d / L)
         cl acc(0, 0);
         for (int d = -(n - 1); d < n; d++) {
             const int dl = (d % L + L) % L;
-            acc += md[(d % n + n) % n] * w[(int)(((long long)k * dl) % L)];
+            mul_add(acc, md[(d % n + n) % n], w[(int)(((long long)k * dl) % L)]);
         }
         acc /= (long double)L;
         hk[2 * k] = (double)acc.real();
         hk[2 * k + 1] = (double)acc.imag();
     }
-    return L;
 }
 
 int fft_chirp_tables(int n, int sign, double *hk, double *chirp) {
     // Bluestein: sum_j x_j exp(sign 2 pi i j k / n) = w_k sum_j (x_j w_j) conj(w_(k-j)),
     // w_m = exp(sign i pi m^2 / n), as jk = (j^2 + k^2 - (k - j)^2) / 2; the
     // exponent m^2 is reduced mod 2n exactly
-    typedef std::complex<long double> cl;
     const int L = fft_conv_length(n);
     if (!L) return 0;
     const long double pi = 4.0L * atanl(1.0L);
@@ -284,17 +296,14 @@ int fft_chirp_tables(int n, int sign, double *hk, double *chirp) {
         chirp[2 * j] = (double)c.real();
         chirp[2 * j + 1] = (double)c.imag();
     }
-    const long double twopi = 8.0L * atanl(1.0L);
-    std::vector<cl> tw(L);
-    for (int k = 0; k < L; k++) {
-        const long double a = twopi * (long double)k / (long double)L;
-        tw[k] = cl(cosl(a), -sinl(a));
-    }
+    std::vector<cl> wd(n);
+    for (int d = 0; d < n; d++) wd[d] = std::conj(w(d));
+    const std::vector<cl> tw = unit_roots(L, -1);
     for (int k = 0; k < L; k++) {  // (1/L) DFT_L of conj(w_d) placed at d mod L, |d| < n
         cl acc(0, 0);
         for (int d = -(n - 1); d < n; d++) {
             const int dl = (d % L + L) % L;
-            acc += std::conj(w(d < 0 ? -d : d)) * tw[(int)(((long long)k * dl) % L)];
+            mul_add(acc, wd[d < 0 ? -d : d], tw[(int)(((long long)k * dl) % L)]);
         }
         acc /= (long double)L;
         hk[2 * k] = (double)acc.real();
@@ -304,12 +313,12 @@ int fft_chirp_tables(int n, int sign, double *hk, double *chirp) {
 }
 
 void dft_matrix(int n, int sign, double *w) {
-    const long double twopi = 8.0L * atanl(1.0L);
+    const std::vector<cl> r = unit_roots(n, sign);
     for (int j = 0; j < n; j++)
         for (int l = 0; l < n; l++) {
-            const long double a = twopi * (long double)(((long long)j * l) % n) / (long double)n;
-            w[2 * ((size_t)j * n + l)] = (double)cosl(a);
-            w[2 * ((size_t)j * n + l) + 1] = (double)(sign * sinl(a));
+            const cl v = r[((long long)j * l) % n];
+            w[2 * ((size_t)j * n + l)] = (double)v.real();
+            w[2 * ((size_t)j * n + l) + 1] = (double)v.imag();
         }
 }
 

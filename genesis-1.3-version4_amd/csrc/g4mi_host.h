@@ -6,6 +6,7 @@
 // host, in FP64 with the reference's operation order.
 #pragma once
 
+#include <complex>
 #include <string>
 #include <vector>
 
@@ -26,13 +27,23 @@ double bessel_j(int n, double x);
 double adi_factors(int ngrid, double delz, double dgrid, double xks, double *c, double *cbet,
                    double *cwet);
 
-// Band of the inverse of the ADI tridiagonal matrix: band[k][m] =
-// (A^-1)[k][k+m-M] (interleaved complex, ngrid*(2M+1) entries, zero where
-// k+m-M is off the grid), computed column by column with the Thomas factors
-// of adi_factors.  Returns the largest entry outside the band relative to
-// its row's diagonal entry.
-double adi_band(int ngrid, const double *c, const double *cbet, const double *cwet, int M,
-                double *band);
+// The inverse of the ADI tridiagonal matrix, column by column with the
+// Thomas factors of adi_factors, built once for every band width asked of it.
+class AdiInverse {
+  public:
+    AdiInverse(int ngrid, const double *c, const double *cbet, const double *cwet);
+    // The largest entry more than M columns off the diagonal relative to its
+    // row's diagonal entry.
+    double beyond(int M) const;
+    // band[k][m] = (A^-1)[k][k+m-M] (interleaved complex, ngrid*(2M+1)
+    // entries, zero where k+m-M is off the grid).
+    void band(int M, double *band) const;
+
+  private:
+    int n_;
+    std::vector<std::complex<double>> inv_;  // column after column
+    std::vector<double> rel_;                // largest relative entry q columns off the diagonal
+};
 
 // Spectral solver matrices (FieldSolverFFT, src/Core/FieldSolverFFT.cpp),
 // interleaved complex, row-major n x n.
@@ -40,15 +51,17 @@ double adi_band(int ngrid, const double *c, const double *cbet, const double *cw
 // m[d] = (1/n) sum_k p_k exp(2 pi i k d / n) and p_k = exp(i K2_1(k) delz),
 // K2_1(k) = -dx(k)^2 dk^2 / (2 xks) the one-dimensional part of K2 (:139)
 // at FFT index k.  exp(K2 delz) = p_ky p_kx, so the 2-D step
-// IDFT(exp(K2 delz) DFT(E)) / n^2 equals M E M^T.
-void fft_propagator(int n, double dgrid, double xks, double delz, double *m);
+// IDFT(exp(K2 delz) DFT(E)) / n^2 equals M E M^T.  propagator_kernel gives m.
+std::vector<std::complex<long double>> propagator_kernel(int n, double dgrid, double xks, double delz);
+void fft_propagator(const std::vector<std::complex<long double>> &md, double *m);
 // The same step as a circular convolution of every line with m, run as a
 // zero-padded FFT of length L = fft_conv_length(n) (the power of two >= 2n-1,
 // at least 128; 0 when n > 256): hk[k] = (1/L) sum_{|d|<n} m[d mod n]
 // exp(-2 pi i k d / L) and tw[k] = exp(-2 pi i k / L), L interleaved complex
-// entries each.  Returns L (0: not supported for this n).
+// entries each.  fft_conv_length returns 0 where n is not supported.
 int fft_conv_length(int n);
-int fft_conv_tables(int n, double dgrid, double xks, double delz, double *hk, double *tw);
+void fft_twiddles(int L, double *tw);
+void fft_conv_kernel(const std::vector<std::complex<long double>> &md, int L, double *hk);
 // A length-n DFT with exp(sign 2 pi i j k / n) as the same convolution
 // (Bluestein): chirp[j] = exp(sign i pi j^2 / n) multiplies the line before
 // and after, hk = (1/L) DFT_L of conj(chirp) placed at d mod L for |d| < n.
