@@ -134,13 +134,14 @@ struct Ctx {
     double *d_wake = nullptr, *d_wake_dg = nullptr, *d_wake_buf = nullptr;
     std::vector<double> h_wake, wake_applied;
     // fields at harmonics of the fundamental (FP64 form): own grid and
-    // wavenumber, the fundamental's ring offset, Thomas ADI per field
+    // wavenumber, the fundamental's ring offset, ADI tables per field
     struct HField {
         int harm = 1, ng = 0;
         double gridmax = 0, dgrid = 0, xks = 0;
         double2 *d_field = nullptr, *d_work = nullptr, *d_src = nullptr;
         int4 *d_box = nullptr;
         PlanCache<AdiPlan> plans;
+        std::map<double, int> choice;  // the tuner's kernel per step size
     };
     std::vector<HField> hf;
     // records of g4mi_run waiting for the host: their per-slice sums sit in
@@ -538,54 +539,68 @@ static int beam_track(Ctx *c, const g4mi_step_params &st, double gamma0, double 
     return G4MI_OK;
 }
 
-// One ADI launch of kernel `kind` on field buffer `fin` (the banded kernel
-// writes `fout`, the others work in place using `fout` as scratch).
-static void adi_launch(Ctx *c, int kind, const AdiFactors &f, double2 *fin, double2 *fout) {
+// One field's ADI: its grid, tables and sources, and where its sums go (null
+// for a harmonic field, whose diagnostics read the field itself).
+struct AdiField {
+    int ng;
+    const AdiPlan *p;
+    const double2 *src;
+    const int4 *box;
+    double *tilediag, *diag;
+};
+
+static bool adi_eligible(const AdiField &a, int kind) {
+    if (kind == 1 || kind == 2) return a.p->tile != 0 && a.diag;
+    if (kind == 3) return a.p->band_m != 0;
+    if (kind == 4) return adi_wide64_ok(a.ng, a.p->band_m, a.p->klo, a.p->khi);
+    return kind == 0;
+}
+
+// One ADI launch of kernel `kind` on field buffer `fin` (the banded kernels
+// write `fout`, the others work in place using `fout` as scratch).
+static void adi_launch(Ctx *c, int kind, const AdiField &a, double2 *fin, double2 *fout) {
+    const AdiPlan &p = *a.p;
+    const AdiFactors f{p.fac, p.fac + a.ng, p.fac + 2 * a.ng, p.cstep, a.ng};
     if (kind == 4)
-        (void)launch_adi_wide64(c->stream, c->ns, fin, fout, c->d_src, c->d_box, c->adi.band, c->adi.cstep, c->ng,
-                                c->first, c->adi.band_m, c->adi.klo, c->adi.khi, c->d_diag_f);
+        (void)launch_adi_wide64(c->stream, c->ns, fin, fout, a.src, a.box, p.band, p.cstep, a.ng, c->first,
+                                p.band_m, p.klo, p.khi, a.diag);
     else if (kind == 3)
-        launch_adi_band(c->stream, c->ns, fin, fout, c->d_src, c->d_box, c->adi.band, c->adi.cstep,
-                        c->ng, c->first, c->adi.band_m, c->adi.klo, c->adi.khi, c->d_tilediag,
-                        c->d_diag_f);
+        launch_adi_band(c->stream, c->ns, fin, fout, a.src, a.box, p.band, p.cstep, a.ng, c->first, p.band_m,
+                        p.klo, p.khi, a.tilediag, a.diag);
     else if (kind == 1 || kind == 2)
-        launch_adi_fused(c->stream, c->ns, fin, fout, c->d_src, c->d_box, f, c->first,
-                         c->d_diag_f, c->adi.tile, kind == 2);
+        launch_adi_fused(c->stream, c->ns, fin, fout, a.src, a.box, f, c->first, a.diag, p.tile, kind == 2);
     else
-        launch_adi(c->stream, c->ns, fin, fout, c->d_src, c->d_box, f, c->first);
+        launch_adi(c->stream, c->ns, fin, fout, a.src, a.box, f, c->first);
 }
 
 // Autotuner of the ADI: run each eligible kernel on a scratch copy of the
-// current field (same sources and boxes) and keep the fastest.  Runs
-// before the first field step of a context and after a step-size change
-// that alters eligibility.
-static int tune_adi(Ctx *c, const AdiFactors &f) {
-    const size_t bytes = (size_t)c->ns * c->ng * c->ng * sizeof(double2);
+// current field (same sources and boxes) and return the fastest.  Runs
+// before a field's first step of each step size; ms[5] receives the timings.
+static int tune_adi(Ctx *c, const AdiField &a, const double2 *field, double2 *work, int *choice, float *ms) {
+    const size_t bytes = (size_t)c->ns * a.ng * a.ng * sizeof(double2);
     double2 *scratch = nullptr;
     G4_HIP(hipMalloc(&scratch, bytes));
     hipEvent_t e0, e1;
     G4_HIP(hipEventCreate(&e0));
     G4_HIP(hipEventCreate(&e1));
-    G4_HIP(hipMemcpyAsync(scratch, c->d_field, bytes, hipMemcpyDeviceToDevice, c->stream));
+    G4_HIP(hipMemcpyAsync(scratch, field, bytes, hipMemcpyDeviceToDevice, c->stream));
     int best_kind = 0;
     float best_ms = 1e30f;
     for (int kind = 0; kind < 5; kind++) {
-        c->adi_ms[kind] = -1.f;
-        if ((kind == 1 || kind == 2) && !c->adi.tile) continue;
-        if (kind == 3 && !c->adi.band_m) continue;
-        if (kind == 4 && !adi_wide64_ok(c->ng, c->adi.band_m, c->adi.klo, c->adi.khi)) continue;
-        adi_launch(c, kind, f, scratch, c->d_work);  // warm-up
+        ms[kind] = -1.f;
+        if (!adi_eligible(a, kind)) continue;
+        adi_launch(c, kind, a, scratch, work);  // warm-up
         float best = 1e30f;
         for (int rep = 0; rep < 3; rep++) {
             G4_HIP(hipEventRecord(e0, c->stream));
-            adi_launch(c, kind, f, scratch, c->d_work);
+            adi_launch(c, kind, a, scratch, work);
             G4_HIP(hipEventRecord(e1, c->stream));
             G4_HIP(hipEventSynchronize(e1));
-            float ms = 0;
-            G4_HIP(hipEventElapsedTime(&ms, e0, e1));
-            best = std::min(best, ms);
+            float t = 0;
+            G4_HIP(hipEventElapsedTime(&t, e0, e1));
+            best = std::min(best, t);
         }
-        c->adi_ms[kind] = best;
+        ms[kind] = best;
         if (best < best_ms) {
             best_ms = best;
             best_kind = kind;
@@ -595,8 +610,7 @@ static int tune_adi(Ctx *c, const AdiFactors &f) {
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     G4_HIP(hipFree(scratch));
-    c->adi_kernel = best_kind;
-    c->adi_choice[c->adi_delz] = best_kind;
+    *choice = best_kind;
     return G4MI_OK;
 }
 
@@ -816,7 +830,9 @@ static int fft_field_step(Ctx *c, double delz) {
 
 // Field::track of every harmonic field (FieldSolverADI per field, Field.cpp
 // :177-185): the source at harmonic h (odd h only, FieldSolverADI.cpp:19-22)
-// and the two-kernel Thomas ADI with the field's own factors.
+// and the ADI with the field's own tables, in the fastest of its kernels
+// (97 slices at 151^2: 48 us a step in the banded tiles, 317 us in the
+// two Thomas sweeps that every harmonic field ran before).
 static int harmonics_track(Ctx *c, const g4mi_step_params &st, double delz) {
     for (Ctx::HField &h : c->hf) {
         AdiPlan p;
@@ -837,8 +853,22 @@ static int harmonics_track(Ctx *c, const g4mi_step_params &st, double delz) {
         d.grady = st.grady;
         d.ngrid = h.ng;
         launch_deposit(c->stream, c->ns, c->d_off, c->d_g, c->d_th, c->d_x, c->d_y, c->d_cur, h.d_src, h.d_box, d);
-        AdiFactors f{p.fac, p.fac + h.ng, p.fac + 2 * h.ng, p.cstep, h.ng};
-        launch_adi(c->stream, c->ns, h.d_field, h.d_work, h.d_src, h.d_box, f, c->first);
+        const AdiField a{h.ng, &p, h.d_src, h.d_box, nullptr, nullptr};
+        // the fundamental's rules: a fixed kernel where it is eligible, the
+        // tuner's choice for the step size otherwise
+        int kind = c->adi_fixed && adi_eligible(a, c->adi_kernel) ? c->adi_kernel : -1;
+        if (kind < 0) {
+            auto it = h.choice.find(delz);
+            if (it == h.choice.end()) {
+                float ms[5];
+                G4_TRY(tune_adi(c, a, h.d_field, h.d_work, &kind, ms));
+                h.choice[delz] = kind;
+            } else {
+                kind = it->second;
+            }
+        }
+        adi_launch(c, kind, a, h.d_field, h.d_work);
+        if (kind >= 3) std::swap(h.d_field, h.d_work);  // result is in the other buffer
     }
     G4_HIP(hipGetLastError());
     return G4MI_OK;
@@ -878,9 +908,12 @@ static int field_track(Ctx *c, const g4mi_step_params &st, double delz, bool dep
         if (c->ev) G4_HIP(hipEventRecord(c->ev[7], c->stream));
         return G4MI_OK;
     }
-    AdiFactors f{c->adi.fac, c->adi.fac + c->ng, c->adi.fac + 2 * c->ng, c->adi.cstep, c->ng};
-    if (c->adi_kernel < 0) G4_TRY(tune_adi(c, f));
-    adi_launch(c, c->adi_kernel, f, c->d_field, c->d_work);
+    const AdiField a{c->ng, &c->adi, c->d_src, c->d_box, c->d_tilediag, c->d_diag_f};
+    if (c->adi_kernel < 0) {
+        G4_TRY(tune_adi(c, a, c->d_field, c->d_work, &c->adi_kernel, c->adi_ms));
+        c->adi_choice[c->adi_delz] = c->adi_kernel;
+    }
+    adi_launch(c, c->adi_kernel, a, c->d_field, c->d_work);
     if (c->adi_kernel >= 3) std::swap(c->d_field, c->d_work);  // result is in the other buffer
     c->field_diag_fresh = c->adi_kernel != 0;
     c->zeroed_since_adi.clear();
@@ -3081,7 +3114,10 @@ int g4mi_set_schedule(g4mi_ctx *h, const char *name, int value) {
     if (std::string(name) == "adi_kernel" && value >= -1 && value <= 4) {
         c->adi_kernel = value;
         c->adi_fixed = value >= 0;
-        if (value < 0) c->adi_choice.clear();
+        if (value < 0) {
+            c->adi_choice.clear();
+            for (Ctx::HField &hf : c->hf) hf.choice.clear();
+        }
         return G4MI_OK;
     }
     if (std::string(name) == "fft_variant" && value >= -1 && value < kCgemmVariants) {

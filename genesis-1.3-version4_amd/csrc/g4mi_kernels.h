@@ -85,14 +85,15 @@ int launch_adi_fused(hipStream_t s, int ns, double2 *field, double2 *work, const
 // reads field `fin`, writes `fout` (the host swaps the buffers), band =
 // [ngrid][2M+1] complex rows of A^-1 around the diagonal, a = Im(cstep).
 // m: 7, 8 or 12.  Rows [klo, khi] of the band equal row (klo+khi)/2 to
-// 2^-60.  tilediag: scratch [ns][adi_band_tiles(ngrid)][8].
+// 2^-60.  tilediag: scratch [ns][adi_band_tiles(ngrid)][8], or null: no
+// field sums.
 int adi_band_tiles(int ng);
 int launch_adi_band(hipStream_t s, int ns, const double2 *fin, double2 *fout, const double2 *src,
                     const int4 *box, const double2 *band, double a, int ng, int first, int m,
                     int klo, int khi, double *tilediag, double *diag);
 // The banded operator as a whole-width stream (one workgroup per slice, one
 // lane per column; the products of launch_adi_band as four partial sums,
-// diagnostics straight into diag[8 ns]).  Eligible for band half widths 7 and 8, grids up to 512
+// diagnostics straight into diag[8 ns], none where it is null).  Eligible for band half widths 7 and 8, grids up to 512
 // columns whose rows [klo, khi] share the central band except in the first
 // and last 32 columns; returns -1 otherwise.
 bool adi_wide64_ok(int ng, int m, int klo, int khi);

@@ -1818,6 +1818,7 @@ __global__ void __launch_bounds__(256) k_adi_band(const double2 *__restrict__ fi
             }
         }
     }
+    if (!tilediag) return;
     double *red = (double *)sm;
     block_sum_waves<NT, 8>(dg, red);
     if (t == 0) {
@@ -2014,6 +2015,7 @@ __global__ void __launch_bounds__(512, 3) k_adi_wide64(const double2 *__restrict
             }
         }
     }
+    if (!diag) return;
     const double dx = (double)x + shift;
     double dg[8] = {s_w, dx * s_w, dx * dx * s_w, s_yw, s_yyw, s_re, s_im, s_cen};
     if (!xin)
@@ -2387,8 +2389,9 @@ static void launch_adi_band_t(hipStream_t s, int ns, const double2 *fin, double2
     const unsigned nblocks = (unsigned)(((ns + 7) / 8) * 8) * (unsigned)(ntx * ntx);
     hipLaunchKernelGGL(k_adi_band<M>, dim3(nblocks), dim3(256), lds, s, fin, fout, src, box,
                        band, a, ng, first, ns, ntx, klo, khi, tilediag);
-    hipLaunchKernelGGL(k_adi_tile_diag, dim3((ns + 63) / 64), dim3(64), 0, s, tilediag,
-                       ntx * ntx, ns, diag);
+    if (tilediag)
+        hipLaunchKernelGGL(k_adi_tile_diag, dim3((ns + 63) / 64), dim3(64), 0, s, tilediag,
+                           ntx * ntx, ns, diag);
 }
 
 int adi_band_tiles(int ng) {

@@ -31,3 +31,31 @@ def test_more_step_sizes_than_kept(solver, ngrid):
     print(f"  {solver} {ngrid}^2, 36 step sizes twice: {err:.2e}", flush=True)
     assert err < 1e-11  # 74 steps of the single step's 1e-13 bar
     ctx.close()
+
+
+@pytest.mark.parametrize("kernel", [-1, 0, 3, 4])
+@pytest.mark.parametrize("ngrid", [31, 32, 65, 97])
+def test_harmonic_field_in_each_adi_kernel(kernel, ngrid):
+    """A third-harmonic field on its own grid (at, below and above the edges
+    of the 32-cell tiles and 64-column wavefronts) in the tuned and in each
+    fixed ADI kernel, over three step sizes with other band widths; a kernel
+    that does not take a step size falls back to the tuner's."""
+    sim = H.make_state([256] * 9, ngrid=41, gridmax=0.3e-3, seed_power=1e6, timerun=False)
+    # bunched at the harmonic: an unmodulated quiet beam's source is rounding noise
+    sim.theta[:] += 0.2 * np.sin(3 * sim.theta)
+    sim.add_harmonics([(3, ngrid, 0.25e-3)])
+    rng = np.random.default_rng(ngrid)
+    sim.hfields[0][:] = rng.normal(size=sim.hfields[0].shape) * 1e10
+    ctx = H.to_gpu(sim)
+    ctx.add_harmonic(3, ngrid, 0.25e-3)
+    ctx.upload_harmonic(0, sim.hfields[0])
+    ctx.set_schedule("adi_kernel", kernel)
+    st = H.steps(1, 2)
+    one = H.gsteps(st)[0]
+    for delz in (0.015, 0.4, 0.015, 3.0):
+        ctx.field_track(one, delz)
+        H.oracle_call("orc_field_advance", sim, C.byref(st[0]), C.c_double(delz))
+    e = np.max(np.abs(ctx.download_harmonic(0) - sim.hfields[0])) / np.max(np.abs(sim.hfields[0]))
+    print(f"  harmonic {ngrid}^2, kernel {kernel}: {e:.2e}", flush=True)
+    assert e < 4e-13  # four steps of the single step's 1e-13 bar
+    ctx.close()
