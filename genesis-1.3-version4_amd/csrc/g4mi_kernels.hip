@@ -56,6 +56,83 @@ __device__ __forceinline__ double2 cpow_int(double2 z, int n) {
     return y;
 }
 
+// ---------------------------------------------------------------------------
+// FP64 quotients, square roots, sines and cosines of the particle kernels.
+//
+// These kernels are bound by FP64 issue, and most of their instructions were
+// the compiler's general divide (12 of them), square root (21) and sincos
+// (~100 on its near path).  The operands here are normal numbers far from
+// overflow, so the scaling and fix-up steps of the general forms go:
+//  * quot(a, recip(b)) is the correctly rounded quotient of the general form
+//    (Newton on v_rcp_f64, then one correction with the exact remainder:
+//    Markstein, IBM J. Res. Dev. 34 (1990) 111), and one reciprocal serves
+//    every division by the same b;
+//  * root(a) is the correctly rounded square root (Goldschmidt on v_rsq_f64
+//    with two exact-remainder corrections) of a normal a > 0;
+//  * sincos64 reduces by Cody and Waite's two-part pi/2 (exact products by
+//    FMA), carries the remainder's rounding along, and evaluates degree-5
+//    polynomials in r^2 interpolated at the Chebyshev nodes of [0, (pi/4)^2]
+//    (errors 1.3e-17 and 5e-19).  At most 0.93 ulp off, 2.8e-17 rms (a
+//    correctly rounded result: 2.7e-17) over |x| up to 5e8.  From 2^45 on,
+//    where neighbouring doubles lie 0.008 rad apart, the phase is first
+//    taken modulo the double nearest 2 pi: off by less than that spacing.
+// ---------------------------------------------------------------------------
+struct Recip {
+    double b, y;  // y = 1/b to an ulp
+};
+__device__ __forceinline__ Recip recip(double b) {
+    double y = __builtin_amdgcn_rcp(b);
+    y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+    y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+    return {b, y};
+}
+// 1/b^2 from 1/b: the square is a few ulp off, one Newton step repairs it
+__device__ __forceinline__ Recip recip_sq(const Recip &r) {
+    const double b = r.b * r.b;
+    double y = r.y * r.y;
+    y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+    return {b, y};
+}
+__device__ __forceinline__ double quot(double a, const Recip &r) {
+    const double q = a * r.y;
+    return __builtin_fma(__builtin_fma(-r.b, q, a), r.y, q);
+}
+__device__ __forceinline__ double root(double a) {
+    const double y = __builtin_amdgcn_rsq(a);
+    double g = a * y, h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    g = __builtin_fma(__builtin_fma(-g, g, a), h, g);
+    return __builtin_fma(__builtin_fma(-g, g, a), h, g);
+}
+__device__ __forceinline__ void sincos64(double x, double *s, double *c) {
+    if (__builtin_expect(!(fabs(x) < 0x1p45), 0)) x = fmod(x, 0x1.921fb54442d18p+2);
+    const double kb = x * 0x1.45f306dc9c883p-1 + 0x1.8p52;  // the multiple in the low bits
+    const double k = kb - 0x1.8p52;
+    const double u = __builtin_fma(-k, 0x1.921fb54442d18p+0, x);
+    const double r = __builtin_fma(-k, 0x1.1a62633145c07p-54, u);
+    const double tail = __builtin_fma(-k, 0x1.1a62633145c07p-54, u - r);
+    const double z = r * r;
+    double p = __builtin_fma(0x1.5e0b19ee56c63p-33, z, -0x1.ae600b0299686p-26);
+    double q = __builtin_fma(-0x1.907da35d467bfp-37, z, 0x1.1eeb68e92d026p-29);
+    p = __builtin_fma(p, z, 0x1.71de379689f47p-19);
+    q = __builtin_fma(q, z, -0x1.27e4fa17d9fc1p-22);
+    p = __builtin_fma(p, z, -0x1.a01a019e83aadp-13);
+    q = __builtin_fma(q, z, 0x1.a01a019f4eb00p-16);
+    p = __builtin_fma(p, z, 0x1.1111111110bb2p-7);
+    q = __builtin_fma(q, z, -0x1.6c16c16c16967p-10);
+    p = __builtin_fma(p, z, -0x1.5555555555555p-3);
+    q = __builtin_fma(q, z, 0x1.5555555555555p-5);
+    const double sn = r + __builtin_fma(r * z, p, tail);
+    const double w = __builtin_fma(-0.5, z, 1.0);
+    const double cs = w + __builtin_fma(z * z, q, __builtin_fma(-r, tail, __builtin_fma(-0.5, z, 1.0 - w)));
+    const int n = __double2loint(kb);
+    const double a = (n & 1) ? cs : sn, b = (n & 1) ? sn : cs;
+    *s = __hiloint2double(__double2hiint(a) ^ ((n << 30) & (int)0x80000000), __double2loint(a));
+    *c = __hiloint2double(__double2hiint(b) ^ (((n + 1) << 30) & (int)0x80000000), __double2loint(b));
+}
+
 // Deterministic block reduction of K doubles (fixed tree order).
 template <int NT, int K>
 __device__ __forceinline__ void block_sum(double (&v)[K], double *lds) {
@@ -81,27 +158,30 @@ __device__ __forceinline__ void block_sum(double (&v)[K], double *lds) {
 // with applyDrift/FQuad/DQuad (:84-116), corrector (:118-128) and the
 // chicane matrix application (:223-236).
 // ---------------------------------------------------------------------------
+// DEFOC: lines that defocus (quadrupoles) are among them
+template <bool DEFOC = true>
 __device__ __forceinline__ void line_map(int kind, double delz, double q, double &x, double &px,
-                                         double gz, double d) {
+                                         const Recip &gz, double d) {
     if (kind == 0) {
-        x += px * delz / gz;
+        x += quot(px * delz, gz);
     } else if (kind > 0) {
-        double foc = sqrt(q / gz), omg = foc * delz;
+        double foc = root(quot(q, gz)), omg = foc * delz;
         double s, c;
-        sincos(omg, &s, &c);
-        double a1 = c, a2 = s / foc, a3 = -a2 * foc * foc;
+        sincos64(omg, &s, &c);
+        double a1 = c, a2 = quot(s, recip(foc)), a3 = -a2 * foc * foc;
         double xtmp = x - d;
-        x = a1 * xtmp + a2 * px / gz + d;
-        px = a3 * xtmp * gz + a1 * px;
-    } else {
-        double foc = sqrt(-q / gz), omg = foc * delz;
-        double a1 = cosh(omg), a2 = sinh(omg) / foc, a3 = a2 * foc * foc;
+        x = a1 * xtmp + quot(a2 * px, gz) + d;
+        px = a3 * xtmp * gz.b + a1 * px;
+    } else if (DEFOC) {
+        double foc = root(quot(-q, gz)), omg = foc * delz;
+        double a1 = cosh(omg), a2 = quot(sinh(omg), recip(foc)), a3 = a2 * foc * foc;
         double xtmp = x - d;
-        x = a1 * xtmp + a2 * px / gz + d;
-        px = a3 * xtmp * gz + a1 * px;
+        x = a1 * xtmp + quot(a2 * px, gz) + d;
+        px = a3 * xtmp * gz.b + a1 * px;
     }
 }
 
+template <bool DEFOC = true>
 __device__ __forceinline__ void transverse_one(const TransParams &p, double gi, double &xi, double &yi,
                                                double &pxi, double &pyi) {
     if (p.corrector) {
@@ -117,9 +197,9 @@ __device__ __forceinline__ void transverse_one(const TransParams &p, double gi, 
         yi = p.m22 * t + p.m23 * pyi / gz;
         pyi = p.m32 * t * gz + p.m33 * pyi;
     }
-    double gammaz = sqrt(gi * gi - 1 - p.aw * p.aw - pxi * pxi - pyi * pyi);
-    line_map(p.kindx, p.delz, p.qx, xi, pxi, gammaz, p.xoff);
-    line_map(p.kindy, p.delz, p.qy, yi, pyi, gammaz, p.yoff);
+    const Recip gammaz = recip(root(gi * gi - 1 - p.aw * p.aw - pxi * pxi - pyi * pyi));
+    line_map<DEFOC>(p.kindx, p.delz, p.qx, xi, pxi, gammaz, p.xoff);
+    line_map<DEFOC>(p.kindy, p.delz, p.qy, yi, pyi, gammaz, p.yoff);
 }
 
 __global__ void __launch_bounds__(256) k_transverse(long long n, const double *__restrict__ g,
@@ -333,7 +413,7 @@ __global__ void __launch_bounds__(256) k_sc_solve(
                 int bin = (int)floor(radi / dr);
                 bin = (bin >= 0 && bin < ngr) ? bin : (bin >= ngr ? ngr - 1 : 0);
                 double s, c;
-                sincos(l * th[i], &s, &c);
+                sincos64(l * th[i], &s, &c);
                 double2 v = make_double2(c, -s);
                 if (m != 0)  // cwork^0 is exactly 1: the azimuthal factor only for m != 0
                     v = cmul(cpow_int(make_double2(tx / radi, ty / radi), -m), v);
@@ -380,7 +460,7 @@ __global__ void __launch_bounds__(256) k_sc_solve(
                 int bin = (int)floor(radi / dr);
                 bin = (bin >= 0 && bin < ngr) ? bin : (bin >= ngr ? ngr - 1 : 0);
                 double s, c;
-                sincos(l * th[i], &s, &c);
+                sincos64(l * th[i], &s, &c);
                 double2 ct = make_double2(c, s);
                 if (m != 0) ct = cmul(cpow_int(make_double2(tx / radi, ty / radi), m), ct);
                 ez[i] += 2 * cmul(ct, celm[bin]).x;
@@ -402,20 +482,25 @@ struct Ode {
     double hh[NH > 0 ? NH : 1];
     double k2gg, k2pp;
     __device__ __forceinline__ void eval(double tgam, double tthet) {
-        double ztemp1 = -2. / xks;
         double s, c;
-        sincos(1.0 * tthet, &s, &c);
+        sincos64(tthet, &s, &c);
+        eval(tgam, tthet, s, c);
+    }
+    // s, c: sine and cosine of tthet
+    __device__ __forceinline__ void eval(double tgam, double tthet, double s, double c) {
+        double ztemp1 = -2. / xks;
         double2 ctmp = cmul(rpart, make_double2(c, -s));
 #pragma unroll
         for (int k = 0; k < NH; k++) {  // the harmonic fields, in field order
             double sh, ch;
-            sincos(hh[k] * tthet, &sh, &ch);
+            sincos64(hh[k] * tthet, &sh, &ch);
             ctmp = cadd(ctmp, cmul(rph[k], make_double2(ch, -sh)));
         }
         double btper0 = btpar + ztemp1 * ctmp.x;
-        double btpar0 = sqrt(1. - btper0 / (tgam * tgam));
-        k2pp += xks * (1. - 1. / btpar0) + xku;
-        k2gg += ctmp.y / btpar0 / tgam - ez;
+        const Recip rg = recip(tgam);
+        const Recip rb = recip(root(1. - quot(btper0, recip_sq(rg))));
+        k2pp += xks * (1. - quot(1.0, rb)) + xku;
+        k2gg += quot(quot(ctmp.y, rb), rg) - ez;
     }
 };
 
@@ -635,7 +720,7 @@ __global__ void __launch_bounds__(1024) k_deposit(const long long *__restrict__ 
                     double faw2 = (1 + p.kx * ddx * ddx + p.ky * ddy * ddy + 2 * (p.gradx * ddx + p.grady * ddy));
                     double part = sqrt(faw2) * scl / g[i];
                     double s, c;
-                    sincos(p.harm * th[i], &s, &c);
+                    sincos64(p.harm * th[i], &s, &c);
                     const double2 cp = make_double2(s * part, c * part);
                     const double wgt[4] = {wx * wy, (1 - wx) * wy, wx * (1 - wy), (1 - wx) * (1 - wy)};
 #pragma unroll
@@ -863,7 +948,14 @@ __global__ void __launch_bounds__(kFrontNT) k_fp64_front(const long long *__rest
 }
 
 
-__global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restrict__ off, double *__restrict__ g,
+// GEN: the second half step defocuses in a plane (quadrupoles) or the
+// short-range solver has azimuthal modes.  The other form, which nearly every
+// step takes, is small enough for four wavefronts per SIMD (two workgroups
+// per CU, what the LDS allows): 1024 x 8192 particles with space charge
+// 433 us against 498 us at the two its 170 registers would give by
+// themselves, and 678 us with the general divide, square root and sincos.
+template <bool GEN>
+__global__ void __launch_bounds__(kFuseNT, GEN ? 2 : 4) k_fp64_main(const long long *__restrict__ off, double *__restrict__ g,
                                                        double *__restrict__ th, double *__restrict__ x,
                                                        double *__restrict__ y, double *__restrict__ px,
                                                        double *__restrict__ py, const double2 *__restrict__ field,
@@ -884,8 +976,10 @@ __global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restri
     const PushParams &p = f.p;
     const DepositParams &d = f.d;
     const int ngr = f.ngr, ng = p.ngrid;
+    const Recip rgrid = {p.dgrid, 1 / p.dgrid};  // the deposit's grid is the push's
     const bool sc = f.use_sc && npart > 0;
-    double xc = 0, yc = 0, dr = 1;
+    double xc = 0, yc = 0;
+    Recip rdr = {1, 1};
     if (t == 0 && f.use_sc) efield[is] = 0;
     // ---- short-range space charge (k_sc_solve): every mode's solution into celm
     if (sc) {
@@ -893,7 +987,8 @@ __global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restri
         double2 *gam = work + kFuseNW * kScMaxNg, *rhs = gam + kScMaxNg;
         double *vol = (double *)(rhs + kScMaxNg), *ldig = vol + kScMaxNg, *rlog = ldig + kScMaxNg + 1;
         double *cupp = rlog + kScMaxNg, *clow = cupp + kScMaxNg, *cmid = clow + kScMaxNg;
-        dr = dr_arr[is];
+        const double dr = dr_arr[is];
+        rdr = {dr, 1 / dr};
         xc = cen[2 * is];
         yc = cen[2 * is + 1];
         const double pi = 2 * asin(1.0);
@@ -914,7 +1009,7 @@ __global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restri
         const double econst = kVacimp / kEev * cur[is] / f.ks / (double)npart;
         const double hs = fx_scale((double)npart);
         int mode = 0;
-        for (int m = -f.nphi; m <= f.nphi; m++) {
+        for (int m = GEN ? -f.nphi : 0; m <= (GEN ? f.nphi : 0); m++) {
             for (int l = 1; l <= f.nz; l++, mode++) {
                 __syncthreads();
                 for (int k = t; k < kFuseNW * kScMaxNg; k += kFuseNT)
@@ -923,12 +1018,12 @@ __global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restri
                 for (long long i = a + t; i < b; i += kFuseNT) {
                     double tx = x[i] - xc, ty = y[i] - yc;
                     double radi = sqrt(tx * tx + ty * ty);
-                    int bin = (int)floor(radi / dr);
+                    int bin = (int)floor(quot(radi, rdr));
                     bin = (bin >= 0 && bin < ngr) ? bin : (bin >= ngr ? ngr - 1 : 0);
                     double s, c;
-                    sincos(l * th[i], &s, &c);
+                    sincos64(l * th[i], &s, &c);
                     double2 v = make_double2(c, -s);
-                    if (m != 0) v = cmul(cpow_int(make_double2(tx / radi, ty / radi), -m), v);
+                    if (GEN && m != 0) v = cmul(cpow_int(make_double2(tx / radi, ty / radi), -m), v);
                     fx_add(&hist[w][bin][0], fx(v.x, hs));
                     fx_add(&hist[w][bin][1], fx(v.y, hs));
                 }
@@ -1010,24 +1105,29 @@ __global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restri
         double xi = x[i], yi = y[i], pxi = px[i], pyi = py[i];
         // short-range field of the particle (k_sc_solve's gather, mode order)
         double ez = 0;
+        double s0, c0;
+        sincos64(theta, &s0, &c0);
         if (sc) {
             const double tx = xi - xc, ty = yi - yc;
             const double radi = sqrt(tx * tx + ty * ty);
-            int bin = (int)floor(radi / dr);
+            int bin = (int)floor(quot(radi, rdr));
             bin = (bin >= 0 && bin < ngr) ? bin : (bin >= ngr ? ngr - 1 : 0);
             int mode = 0;
-            for (int m = -f.nphi; m <= f.nphi; m++) {
+            for (int m = GEN ? -f.nphi : 0; m <= (GEN ? f.nphi : 0); m++) {
                 for (int l = 1; l <= f.nz; l++, mode++) {
-                    double s, c;
-                    sincos(l * theta, &s, &c);
+                    double s = s0, c = c0;
+                    if (l > 1) sincos64(l * theta, &s, &c);
                     double2 ct = make_double2(c, s);
-                    if (m != 0) ct = cmul(cpow_int(make_double2(tx / radi, ty / radi), m), ct);
+                    if (GEN && m != 0) ct = cmul(cpow_int(make_double2(tx / radi, ty / radi), m), ct);
                     ez += 2 * cmul(ct, celm[mode * ngr + bin]).x;
                 }
             }
         }
         // push (k_push)
-        theta += p.autophase;
+        if (p.autophase != 0) {  // uniform: else the first evaluation is at the same phase
+            theta += p.autophase;
+            sincos64(theta, &s0, &c0);
+        }
         const double dx = xi - p.ax, dy = yi - p.ay;
         const double awloc = (1 + 0.5 * (p.kx * dx * dx + p.ky * dy * dy) + p.gradx * dx + p.grady * dy);
         Ode<0> o;
@@ -1036,8 +1136,8 @@ __global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restri
         o.btpar = 1 + pxi * pxi + pyi * pyi + p.aw * p.aw * awloc * awloc;
         o.ez = (p.use_sc ? ez : 0.0) + eloss;
         if ((xi > -p.gridmax) && (xi < p.gridmax) && (yi > -p.gridmax) && (yi < p.gridmax)) {
-            double wx = (xi + p.gridmax) / p.dgrid;
-            double wy = (yi + p.gridmax) / p.dgrid;
+            double wx = quot(xi + p.gridmax, rgrid);
+            double wy = quot(yi + p.gridmax, rgrid);
             int ix = (int)floor(wx), iy = (int)floor(wy);
             wx = 1 + floor(wx) - wx;
             wy = 1 + floor(wy) - wy;
@@ -1058,7 +1158,7 @@ __global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restri
         double k3gg, k3pp;
         o.k2gg = 0;
         o.k2pp = 0;
-        o.eval(gamma, theta);
+        o.eval(gamma, theta, s0, c0);
         double stpz = 0.5 * delz;
         gamma += stpz * o.k2gg;
         theta += stpz * o.k2pp;
@@ -1085,7 +1185,7 @@ __global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restri
         gamma += stpz * (k3gg + o.k2gg / 6.0);
         theta += stpz * (k3pp + o.k2pp / 6.0);
         if (f.chicane) theta += f.r56 * (gamma - f.gamma0);   // k_r56
-        transverse_one(f.t2, gamma, xi, yi, pxi, pyi);
+        transverse_one<GEN>(f.t2, gamma, xi, yi, pxi, pyi);
         g[i] = gamma;
         th[i] = theta;
         x[i] = xi;
@@ -1100,13 +1200,13 @@ __global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restri
         v[4] += yi;
         v[5] += yi * yi;
         double s1, c1;
-        sincos((0 + 1) * theta, &s1, &c1);
+        sincos64(theta, &s1, &c1);
         v[6] += c1;
         v[7] += s1;
         // deposit (k_deposit)
         if (dep && (xi > -d.gridmax) && (xi < d.gridmax) && (yi > -d.gridmax) && (yi < d.gridmax)) {
-            double wx = (xi + d.gridmax) / d.dgrid;
-            double wy = (yi + d.gridmax) / d.dgrid;
+            double wx = quot(xi + d.gridmax, rgrid);
+            double wy = quot(yi + d.gridmax, rgrid);
             const int ix = min((int)floor(wx), ng - 2), iy = min((int)floor(wy), ng - 2);
             bx0 = min(bx0, ix);
             bx1 = max(bx1, ix + 1);
@@ -1114,15 +1214,14 @@ __global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restri
             by1 = max(by1, iy + 1);
             const double ddx = xi - d.ax, ddy = yi - d.ay;
             const double faw2 = (1 + d.kx * ddx * ddx + d.ky * ddy * ddy + 2 * (d.gradx * ddx + d.grady * ddy));
-            const double part = sqrt(faw2) * scl / gamma;
+            const double part = quot(sqrt(faw2) * scl, recip(gamma));
             v[8] += fabs(part);
             if (fused) {
                 if (ix >= tx0 && ix + 1 < tx0 + tw && iy >= ty0 && iy + 1 < ty0 + tht) {
                     wx = 1 + floor(wx) - wx;
                     wy = 1 + floor(wy) - wy;
-                    double s, c;
-                    sincos(d.harm * theta, &s, &c);
-                    const double2 cp = make_double2(s * part, c * part);
+                    // the fused step has the fundamental only (harm = 1)
+                    const double2 cp = make_double2(s1 * part, c1 * part);
                     const int lk = (iy - ty0) * tw + (ix - tx0);
                     const double w00 = wx * wy, w10 = (1 - wx) * wy, w01 = wx * (1 - wy), w11 = (1 - wx) * (1 - wy);
                     fx_add(&tre[lk], fx(w00 * cp.x, fs1));
@@ -1179,8 +1278,8 @@ __global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restri
         for (long long i = a + t; i < b; i += kFuseNT) {
             const double xi = x[i], yi = y[i];
             if (!((xi > -d.gridmax) && (xi < d.gridmax) && (yi > -d.gridmax) && (yi < d.gridmax))) continue;
-            double wx = (xi + d.gridmax) / d.dgrid;
-            double wy = (yi + d.gridmax) / d.dgrid;
+            double wx = quot(xi + d.gridmax, rgrid);
+            double wy = quot(yi + d.gridmax, rgrid);
             const int ix = min((int)floor(wx), ng - 2), iy = min((int)floor(wy), ng - 2);
             if (iy + 1 < r0 || iy > r1) continue;
             wx = 1 + floor(wx) - wx;
@@ -1189,7 +1288,7 @@ __global__ void __launch_bounds__(kFuseNT) k_fp64_main(const long long *__restri
             const double faw2 = (1 + d.kx * ddx * ddx + d.ky * ddy * ddy + 2 * (d.gradx * ddx + d.grady * ddy));
             const double part = sqrt(faw2) * scl / g[i];
             double s, c;
-            sincos(d.harm * th[i], &s, &c);
+            sincos64(d.harm * th[i], &s, &c);
             const double2 cp = make_double2(s * part, c * part);
             const double wgt[4] = {wx * wy, (1 - wx) * wy, wx * (1 - wy), (1 - wx) * (1 - wy)};
             const int cx[4] = {ix, ix + 1, ix, ix + 1};
@@ -2063,7 +2162,7 @@ __global__ void __launch_bounds__(256) k_diag_beam(const long long *__restrict__
         v[4] += yi;
         v[5] += yi * yi;
         double s, c;
-        sincos((0 + 1) * th[i], &s, &c);
+        sincos64((0 + 1) * th[i], &s, &c);
         v[6] += c;
         v[7] += s;
     }
@@ -2090,7 +2189,7 @@ __global__ void __launch_bounds__(256) k_diag_bunch(const long long *__restrict_
         for (int k = 0; k < 8; k++)
             if (k < cnt) {
                 double sn, cs;
-                sincos((double)(h0 + k) * t, &sn, &cs);
+                sincos64((double)(h0 + k) * t, &sn, &cs);
                 v[2 * k] += cs;
                 v[2 * k + 1] += sn;
             }
@@ -2313,11 +2412,13 @@ void launch_fp64_main(hipStream_t s, int ns, const long long *off, double *g, do
                       const double *pmaxf, double2 *src, int4 *box, double *beamsum, const FuseParams &f) {
     static bool attr = false;
     if (!attr) {  // 64 KiB of dynamic LDS plus the static reduction scratch
-        (void)hipFuncSetAttribute((const void *)k_fp64_main, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  kFuseDyn * sizeof(double2));
+        for (const void *k : {(const void *)k_fp64_main<false>, (const void *)k_fp64_main<true>})
+            (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kFuseDyn * sizeof(double2));
         attr = true;
     }
-    hipLaunchKernelGGL(k_fp64_main, dim3(ns), dim3(kFuseNT), kFuseDyn * sizeof(double2), s, off, g, th, x, y, px,
+    const bool gen = f.t2.kindx < 0 || f.t2.kindy < 0 || (f.use_sc && f.nphi > 0);
+    auto k = gen ? k_fp64_main<true> : k_fp64_main<false>;
+    hipLaunchKernelGGL(k, dim3(ns), dim3(kFuseNT), kFuseDyn * sizeof(double2), s, off, g, th, x, y, px,
                        py, field, esc, cur, cen, dr, efield, pbox, pmaxf, src, box, beamsum, f);
 }
 
