@@ -7,6 +7,7 @@
 // restates; expressions keep the reference's association order.
 #include "g4mi_kernels.h"
 #include "g4mi_scan.h"
+#include "g4mi_tridiag.h"
 
 #include <algorithm>
 
@@ -368,15 +369,33 @@ __global__ void __launch_bounds__(kScanNT) k_sc_scan(int ns, const long long *__
 // per wavefront and accumulate in fixed point (fx_add), so the result is
 // bit-reproducible.
 constexpr int kScMaxNg = 256;
+// Row i of the radial operator of mode (m, l) (constructLaplaceOperator
+// :176-190, coefficients :240-245): cell volume and the three entries.
+struct ScRow {
+    double vol, low, mid, up;
+};
+__device__ __forceinline__ ScRow sc_row(int i, int ngr, int m, int l, double dr, double coef) {
+    const double pi = 2 * asin(1.0);
+    ScRow r;
+    r.vol = pi * dr * dr;
+    if (i > 0) r.vol = pi * dr * dr * (2 * i + 1);
+    const double ldig = 2 * pi * i, ldnext = i + 1 < ngr ? 2 * pi * (i + 1) : 0.0;
+    double lm = -ldig - ldnext;
+    if (m != 0) lm -= 2. * pi * m * m * (i == 0 ? 0.5 : log((double)(i + 1) / (double)i));
+    if (i == ngr - 1) lm -= 2 * pi * ngr;
+    r.mid = 1 + coef * lm / l / l / r.vol;
+    r.low = coef * ldig / l / l / r.vol;
+    r.up = coef * ldnext / l / l / r.vol;
+    return r;
+}
 __global__ void __launch_bounds__(256) k_sc_solve(
     const long long *__restrict__ off, const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ th, const double *__restrict__ cur, const double *__restrict__ cen,
     const double *__restrict__ dr_arr, int ngr, int nz, int nphi, double ks, double gz2,
     double *__restrict__ ez, double *__restrict__ efield) {
     __shared__ long long hist[4][kScMaxNg][2];
-    __shared__ double2 celm[kScMaxNg], gam[kScMaxNg], rhs[kScMaxNg];
-    __shared__ double vol[kScMaxNg], ldig[kScMaxNg + 1], rlog[kScMaxNg];
-    __shared__ double cupp[kScMaxNg], clow[kScMaxNg], cmid[kScMaxNg];
+    __shared__ double2 celm[kScMaxNg];
+    __shared__ double pcr[8 * kScMaxNg];
     const int is = blockIdx.x, t = threadIdx.x, w = t >> 6;
     const long long a = off[is], b = off[is + 1];
     const int npart = (int)(b - a);
@@ -384,21 +403,6 @@ __global__ void __launch_bounds__(256) k_sc_solve(
     if (t == 0) efield[is] = 0;
     if (npart < 1) return;
     const double dr = dr_arr[is], xc = cen[2 * is], yc = cen[2 * is + 1];
-    const double pi = 2 * asin(1.0);
-    // radial grid tables, one entry per lane (constructLaplaceOperator :176-190)
-    for (int j = t; j <= ngr; j += 256) {
-        if (j == ngr) {
-            ldig[ngr] = 0;
-        } else if (j == 0) {
-            vol[0] = pi * dr * dr;
-            rlog[0] = 0.5;
-            ldig[0] = 0;
-        } else {
-            vol[j] = pi * dr * dr * (2 * j + 1);
-            ldig[j] = 2 * pi * j;
-            rlog[j] = log((double)(j + 1) / (double)j);
-        }
-    }
     const double coef = -gz2 / ks / ks;
     const double econst = kVacimp / kEev * cur[is] / ks / (double)npart;
     const double hs = fx_scale((double)npart);  // |cos|, |sin| <= 1: a bin sums at most npart of them
@@ -421,38 +425,19 @@ __global__ void __launch_bounds__(256) k_sc_solve(
                 fx_add(&hist[w][bin][1], fx(v.y, hs));
             }
             __syncthreads();
-            // operator coefficients (:240-245) and source of every radial cell,
-            // one cell per lane; the sequential recurrence then only reads them
-            for (int i = t; i < ngr; i += 256) {
-                double lm = -ldig[i] - ldig[i + 1] - 2. * pi * m * m * rlog[i];
-                if (i == ngr - 1) lm -= 2 * pi * ngr;
-                cmid[i] = 1 + coef * lm / l / l / vol[i];
-                if (i > 0) {
-                    cupp[i] = coef * ldig[i] / l / l / vol[i - 1];
-                    clow[i] = coef * ldig[i] / l / l / vol[i];
-                }
+            // operator and source of every radial cell, one cell per lane
+            ScRow row = {1, 0, 1, 0};
+            double2 rhs = make_double2(0, 0);
+            if (t < ngr) {
+                row = sc_row(t, ngr, m, l, dr, coef);
                 const double2 cs = make_double2(
-                    (double)(hist[0][i][0] + hist[1][i][0] + hist[2][i][0] + hist[3][i][0]) / hs,
-                    (double)(hist[0][i][1] + hist[1][i][1] + hist[2][i][1] + hist[3][i][1]) / hs);
-                rhs[i] = cmul(cs, make_double2(0, econst / l / vol[i]));
+                    (double)(hist[0][t][0] + hist[1][t][0] + hist[2][t][0] + hist[3][t][0]) / hs,
+                    (double)(hist[0][t][1] + hist[1][t][1] + hist[2][t][1] + hist[3][t][1]) / hs);
+                rhs = cmul(cs, make_double2(0, econst / l / row.vol));
             }
-            __syncthreads();
-            if (t == 0) {  // tridiag (:260-272)
-                // the operator's entries are real (complex with zero
-                // imaginary parts in the reference), so bet and gam are real:
-                // one reciprocal per cell on the sequential chain
-                double bet = cmid[0], inv = 1.0 / bet;
-                celm[0] = cscale(rhs[0], inv);
-                for (int i = 1; i < ngr; i++) {
-                    const double g = cupp[i] * inv;
-                    gam[i].x = g;
-                    bet = cmid[i] - clow[i] * g;
-                    inv = 1.0 / bet;
-                    celm[i] = cscale(csub(rhs[i], cscale(celm[i - 1], clow[i])), inv);
-                }
-                for (int i = ngr - 2; i > -1; i--) celm[i] = csub(celm[i], cscale(celm[i + 1], gam[i + 1].x));
-                if (l == 1) efield[is] = hypot(celm[0].x, celm[0].y);
-            }
+            const double2 sol = tridiag_pcr(t, ngr, row.low, row.mid, row.up, rhs, pcr);
+            if (t < ngr) celm[t] = sol;
+            if (t == 0 && l == 1) efield[is] = hypot(sol.x, sol.y);
             __syncthreads();
             for (long long i = a + t; i < b; i += 256) {
                 double tx = x[i] - xc, ty = y[i] - yc;
@@ -831,7 +816,7 @@ constexpr int kFuseNW = kFuseNT / 64;
 constexpr int kFuseModes = 512;                        // mode-solution cells (double2)
 constexpr int kFuseDyn = kFuseModes + 3584;            // double2 cells of the dynamic region (64 KiB)
 constexpr int kFuseTile = kFuseDyn - kFuseModes;        // deposit tile cells
-static_assert(kFuseNW * kScMaxNg + 2 * kScMaxNg + (6 * kScMaxNg + 2) / 2 <= kFuseTile,
+static_assert(kFuseNW * kScMaxNg + 4 * kScMaxNg <= kFuseTile && kFuseNT >= kScMaxNg,
               "the short-range solver's scratch must fit in the tile region");
 
 __global__ void __launch_bounds__(kFrontNT) k_fp64_front(const long long *__restrict__ off,
@@ -984,27 +969,11 @@ __global__ void __launch_bounds__(kFuseNT, GEN ? 2 : 4) k_fp64_main(const long l
     // ---- short-range space charge (k_sc_solve): every mode's solution into celm
     if (sc) {
         long long(*hist)[kScMaxNg][2] = (long long(*)[kScMaxNg][2])work;   // [waves][ngr][2] fixed point
-        double2 *gam = work + kFuseNW * kScMaxNg, *rhs = gam + kScMaxNg;
-        double *vol = (double *)(rhs + kScMaxNg), *ldig = vol + kScMaxNg, *rlog = ldig + kScMaxNg + 1;
-        double *cupp = rlog + kScMaxNg, *clow = cupp + kScMaxNg, *cmid = clow + kScMaxNg;
+        double *pcr = (double *)(work + kFuseNW * kScMaxNg);
         const double dr = dr_arr[is];
         rdr = {dr, 1 / dr};
         xc = cen[2 * is];
         yc = cen[2 * is + 1];
-        const double pi = 2 * asin(1.0);
-        for (int j = t; j <= ngr; j += kFuseNT) {
-            if (j == ngr) {
-                ldig[ngr] = 0;
-            } else if (j == 0) {
-                vol[0] = pi * dr * dr;
-                rlog[0] = 0.5;
-                ldig[0] = 0;
-            } else {
-                vol[j] = pi * dr * dr * (2 * j + 1);
-                ldig[j] = 2 * pi * j;
-                rlog[j] = log((double)(j + 1) / (double)j);
-            }
-        }
         const double coef = -f.gz2 / f.ks / f.ks;
         const double econst = kVacimp / kEev * cur[is] / f.ks / (double)npart;
         const double hs = fx_scale((double)npart);
@@ -1028,37 +997,21 @@ __global__ void __launch_bounds__(kFuseNT, GEN ? 2 : 4) k_fp64_main(const long l
                     fx_add(&hist[w][bin][1], fx(v.y, hs));
                 }
                 __syncthreads();
-                for (int i = t; i < ngr; i += kFuseNT) {
-                    double lm = -ldig[i] - ldig[i + 1] - 2. * pi * m * m * rlog[i];
-                    if (i == ngr - 1) lm -= 2 * pi * ngr;
-                    cmid[i] = 1 + coef * lm / l / l / vol[i];
-                    if (i > 0) {
-                        cupp[i] = coef * ldig[i] / l / l / vol[i - 1];
-                        clow[i] = coef * ldig[i] / l / l / vol[i];
-                    }
-                    long long csx = hist[0][i][0], csy = hist[0][i][1];
+                ScRow row = {1, 0, 1, 0};
+                double2 rhs = make_double2(0, 0);
+                if (t < ngr) {
+                    row = sc_row(t, ngr, m, l, dr, coef);
+                    long long csx = hist[0][t][0], csy = hist[0][t][1];
                     for (int q = 1; q < kFuseNW; q++) {
-                        csx += hist[q][i][0];
-                        csy += hist[q][i][1];
+                        csx += hist[q][t][0];
+                        csy += hist[q][t][1];
                     }
                     const double2 cs = make_double2((double)csx / hs, (double)csy / hs);
-                    rhs[i] = cmul(cs, make_double2(0, econst / l / vol[i]));
+                    rhs = cmul(cs, make_double2(0, econst / l / row.vol));
                 }
-                __syncthreads();
-                if (t == 0) {
-                    double2 *ce = celm + mode * ngr;
-                    double bet = cmid[0], inv = 1.0 / bet;
-                    ce[0] = cscale(rhs[0], inv);
-                    for (int i = 1; i < ngr; i++) {
-                        const double gg = cupp[i] * inv;
-                        gam[i].x = gg;
-                        bet = cmid[i] - clow[i] * gg;
-                        inv = 1.0 / bet;
-                        ce[i] = cscale(csub(rhs[i], cscale(ce[i - 1], clow[i])), inv);
-                    }
-                    for (int i = ngr - 2; i > -1; i--) ce[i] = csub(ce[i], cscale(ce[i + 1], gam[i + 1].x));
-                    if (l == 1) efield[is] = hypot(ce[0].x, ce[0].y);
-                }
+                const double2 sol = tridiag_pcr(t, ngr, row.low, row.mid, row.up, rhs, pcr);
+                if (t < ngr) celm[mode * ngr + t] = sol;
+                if (t == 0 && l == 1) efield[is] = hypot(sol.x, sol.y);
             }
         }
     }

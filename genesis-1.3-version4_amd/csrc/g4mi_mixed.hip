@@ -24,6 +24,7 @@
 
 #include "g4mi_mixed.h"
 #include "g4mi_scan.h"
+#include "g4mi_tridiag.h"
 
 namespace g4mi {
 
@@ -465,14 +466,13 @@ __device__ bool main_step(const MixArrays &a, const int is, int sc_on, float2 *d
     // rounded up to a double2 boundary), then the histograms and later the
     // deposit tile in the rest
     static_assert((NT / 64) * kScMax <= (DYN - kCelmCells) / 2, "the histograms must fit in the tile region");
+    static_assert(NT >= kScMax, "the radial solver takes one row per thread, in place of the histograms");
     const int ncelm = sc_on ? (((2 * a.sc_nphi + 1) * a.sc_nz * a.sc_ng + 1) & ~1) : 0;
     const int tile_cells = (DYN - ncelm) / 2;             // double2 cells
     // deposit tile cells: two planes of TileT
     const int dep_cells = (DYN - ncelm) * (int)sizeof(float2) / (2 * (int)sizeof(TileT));
     __shared__ int bred[5 * (NT / 64)];
     __shared__ double wred[9 * (NT / 64)];
-    __shared__ float gsol[kScMax], scupp[kScMax], sclow[kScMax], scmid[kScMax];
-    __shared__ float2 scrhs[kScMax];
     const MixStep &S = a.steps[a.st->istep];
     const int t = threadIdx.x, w = t >> 6;
     const long long b0 = a.off[is], b1 = a.off[is + 1];
@@ -572,42 +572,34 @@ __device__ bool main_step(const MixArrays &a, const int is, int sc_on, float2 *d
                 }
                 __syncthreads();
                 // constructLaplaceOperator (:176-190): coefficients and source of
-                // every radial cell, one cell per lane; tridiag (:260-272) on
-                // lane 0.  The operator is real, the right-hand side complex.
-                for (int i = t; i < ngr; i += NT) {
-                    const double voli = kPi * drd * drd * (i == 0 ? 1.0 : (double)(2 * i + 1));
-                    const double ldi = i > 0 ? 2 * kPi * i : 0.0;
-                    const double ldn = (i + 1 < ngr) ? 2 * kPi * (i + 1) : 0.0;
-                    const double rl = i == 0 ? 0.5 : log((double)(i + 1) / (double)i);
-                    double lm = -ldi - ldn - 2. * kPi * m * m * rl;
-                    if (i == ngr - 1) lm -= 2 * kPi * ngr;
-                    scmid[i] = (float)(1 + coef * lm / l / l / voli);
-                    if (i > 0) {
-                        const double volm = kPi * drd * drd * (i == 1 ? 1.0 : (double)(2 * i - 1));
-                        scupp[i] = (float)(coef * ldi / l / l / volm);
-                        sclow[i] = (float)(coef * ldi / l / l / voli);
-                    }
+                // every radial cell, one cell per lane.  The operator is real,
+                // the right-hand side complex; both in FP64, the solution
+                // stored in FP32.
+                double low = 0, mid = 1, up = 0;
+                double2 rhs = make_double2(0, 0);
+                if (t < ngr) {
+                    const double voli = kPi * drd * drd * (t == 0 ? 1.0 : (double)(2 * t + 1));
+                    const double ldi = 2 * kPi * t;
+                    const double ldn = (t + 1 < ngr) ? 2 * kPi * (t + 1) : 0.0;
+                    double lm = -ldi - ldn;
+                    if (m != 0) lm -= 2. * kPi * m * m * (t == 0 ? 0.5 : log((double)(t + 1) / (double)t));
+                    if (t == ngr - 1) lm -= 2 * kPi * ngr;
+                    const double cv = coef / l / l / voli;
+                    mid = 1 + cv * lm;
+                    low = cv * ldi;
+                    up = cv * ldn;
                     double csx = 0, csy = 0;
                     for (int q = 0; q < (NT / 64) * nsub; q++) {
-                        csx += hs[q * ngr + i].x;
-                        csy += hs[q * ngr + i].y;
+                        csx += hs[q * ngr + t].x;
+                        csy += hs[q * ngr + t].y;
                     }
                     const double e = econst / l / voli;
-                    scrhs[i] = f2((float)(-csy * e), (float)(csx * e));
+                    rhs = make_double2(-csy * e, csx * e);
                 }
-                __syncthreads();
-                if (t == 0) {
-                    float2 *ce = celm + mode * ngr;
-                    float bet = scmid[0];
-                    ce[0] = fscale(scrhs[0], 1.f / bet);
-                    for (int i = 1; i < ngr; i++) {
-                        gsol[i] = scupp[i] / bet;
-                        bet = scmid[i] - sclow[i] * gsol[i];
-                        ce[i] = fscale(fsub(scrhs[i], fscale(ce[i - 1], sclow[i])), 1.f / bet);
-                    }
-                    for (int i = ngr - 2; i > -1; i--) ce[i] = fsub(ce[i], fscale(ce[i + 1], gsol[i + 1]));
-                    if (l == 1) a.efield[is] = hypot((double)ce[0].x, (double)ce[0].y);
-                }
+                __syncthreads();  // the histograms are read: the solver's rows take their place
+                const double2 sol = tridiag_pcr(t, ngr, low, mid, up, rhs, (double *)work);
+                if (t < ngr) celm[mode * ngr + t] = f2((float)sol.x, (float)sol.y);
+                if (t == 0 && l == 1) a.efield[is] = hypot(sol.x, sol.y);
             }
         }
     }
