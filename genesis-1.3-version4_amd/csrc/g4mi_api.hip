@@ -57,6 +57,14 @@ struct PlanCache {
     }
 };
 
+// The split deposit's accumulators of one field (small windows): the slices'
+// fixed-point planes, zero between steps, and the footprint corners of this
+// step and the next (alternating by step parity).
+struct SplitPlane {
+    long long *acc = nullptr;
+    int *corner[2] = {nullptr, nullptr};
+};
+
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -77,6 +85,14 @@ struct Ctx {
     int4 *d_box = nullptr;
     int nblk = 0, blk_cap = 0;
     int *d_blk_slice = nullptr;
+    long long *d_blk_first = nullptr;  // [ns+1] first block of each slice
+    // small windows (split_step): block sums, deposit scale per slice and its
+    // parity, the fundamental's planes; split_off: they did not fit
+    double *d_part = nullptr;
+    unsigned long long *d_pmax[2] = {nullptr, nullptr};
+    int split_par = 0;
+    SplitPlane split;
+    bool split_off = false;
     long long *d_blk_begin = nullptr;
     double *d_diag_b = nullptr, *d_diag_f = nullptr;
     double *d_bunch = nullptr;  // harmonic bunching sums, [ns][8][2]
@@ -97,6 +113,7 @@ struct Ctx {
     // field diagnostics sums written by the fused ADI of the last field
     // step, and the storage slices slippage has zeroed since then
     bool field_diag_fresh = false;
+    bool tiles_fresh = false;          // they are still per tile, in d_tilediag
     std::vector<int> zeroed_since_adi;
     // ADI kernel chosen by the autotuner (-1: not tuned yet) and its timings:
     // 0 two-kernel Thomas, 1 fused recurrence, 2 fused recurrence with
@@ -142,6 +159,7 @@ struct Ctx {
         int4 *d_box = nullptr;
         PlanCache<AdiPlan> plans;
         std::map<double, int> choice;  // the tuner's kernel per step size
+        SplitPlane split;
     };
     std::vector<HField> hf;
     // records of g4mi_run waiting for the host: their per-slice sums sit in
@@ -168,6 +186,7 @@ struct Ctx {
     int4 *d_pbox = nullptr;                // in-grid footprint per slice after the first half step
     double *d_pmaxf = nullptr;             // per slice: largest sqrt(faw2) / gamma in the grid (deposit scale)
     bool beamsum_fresh = false;            // d_beamsum describes the current particles
+    bool beampart_fresh = false;           // d_part does, per block of 256
     SortWork sw{};
     long long *d_off_new = nullptr;
     double wake_dz = 0;
@@ -304,14 +323,17 @@ static TransParams transverse_params(const Ctx *c, const g4mi_step_params &st, d
 }
 
 static void build_block_table(const std::vector<long long> &off, std::vector<int> &bs,
-                              std::vector<long long> &bb) {
+                              std::vector<long long> &bb, std::vector<long long> &bf) {
     bs.clear();
     bb.clear();
-    for (size_t is = 0; is + 1 < off.size(); is++)
+    bf.assign(off.size(), 0);
+    for (size_t is = 0; is + 1 < off.size(); is++) {
         for (long long a = off[is]; a < off[is + 1]; a += 256) {
             bs.push_back((int)is);
             bb.push_back(a);
         }
+        bf[is + 1] = (long long)bs.size();
+    }
 }
 
 constexpr size_t kPlanBytes = 64u << 20;  // of one cache of plans
@@ -462,17 +484,9 @@ static int energy_kicks(Ctx *c, const g4mi_step_params &st, double gamma0, doubl
     return G4MI_OK;
 }
 
-static int beam_track(Ctx *c, const g4mi_step_params &st, double gamma0, double delz) {
-    if (!c->has_beam) {
-        set_error("beam not uploaded");
-        return G4MI_E_STATE;
-    }
-    TransParams t1 = transverse_params(c, st, gamma0, delz * 0.5, false);
-    if (c->ev) G4_HIP(hipEventRecord(c->ev[0], c->stream));
-    launch_transverse(c->stream, c->ntot, c->d_g, c->d_x, c->d_y, c->d_px, c->d_py, t1);
-
-    // BeamSolver::advance
-    if (c->ev) G4_HIP(hipEventRecord(c->ev[1], c->stream));
+// Space charge of the positions after the first transverse half step
+// (BeamSolver::advance, src/Core/BeamSolver.cpp:36-51), in separate kernels.
+static void space_charge(Ctx *c, const g4mi_step_params &st, double gamma0) {
     const double aw = st.aw;
     const bool sc = (c->sc_nz > 0) && (c->sc_ng > 2);
     if (c->longrange || sc) {
@@ -493,14 +507,16 @@ static int beam_track(Ctx *c, const g4mi_step_params &st, double gamma0, double 
         launch_sc_solve(c->stream, c->ns, c->d_off, c->d_x, c->d_y, c->d_th, c->d_cur, c->d_cen,
                         c->d_dr, c->sc_ng, c->sc_nz, c->sc_nphi, ks, gz2, c->d_ez, c->d_efield);
     }
-    if (c->ev) G4_HIP(hipEventRecord(c->ev[2], c->stream));
+}
+
+static PushParams push_params(const Ctx *c, const g4mi_step_params &st, double gamma0, double delz) {
     PushParams p{};
     p.delz = delz;
     p.xks = c->xks;
     p.rtmp = coupling(st, 1) / c->xks;
     p.xku = st.ku;
     if (p.xku == 0) p.xku = c->xks * 0.5 / gamma0 / gamma0;
-    p.aw = aw;
+    p.aw = st.aw;
     p.autophase = st.phaseshift;
     p.ax = st.ax;
     p.ay = st.ay;
@@ -513,7 +529,7 @@ static int beam_track(Ctx *c, const g4mi_step_params &st, double gamma0, double 
     p.ngrid = c->ng;
     p.first = c->first;
     p.nslice = c->ns;
-    p.use_sc = sc ? 1 : 0;
+    p.use_sc = (c->sc_nz > 0 && c->sc_ng > 2) ? 1 : 0;
     p.nh = (int)c->hf.size();
     for (int k = 0; k < p.nh; k++) {
         const Ctx::HField &h = c->hf[k];
@@ -524,6 +540,23 @@ static int beam_track(Ctx *c, const g4mi_step_params &st, double gamma0, double 
         p.hg[k].harm = (double)h.harm;
         p.hg[k].rtmp = coupling(st, h.harm) / h.xks;  // BeamSolver.cpp:28
     }
+    return p;
+}
+
+static int beam_track(Ctx *c, const g4mi_step_params &st, double gamma0, double delz) {
+    if (!c->has_beam) {
+        set_error("beam not uploaded");
+        return G4MI_E_STATE;
+    }
+    TransParams t1 = transverse_params(c, st, gamma0, delz * 0.5, false);
+    if (c->ev) G4_HIP(hipEventRecord(c->ev[0], c->stream));
+    launch_transverse(c->stream, c->ntot, c->d_g, c->d_x, c->d_y, c->d_px, c->d_py, t1);
+
+    // BeamSolver::advance
+    if (c->ev) G4_HIP(hipEventRecord(c->ev[1], c->stream));
+    space_charge(c, st, gamma0);
+    if (c->ev) G4_HIP(hipEventRecord(c->ev[2], c->stream));
+    const PushParams p = push_params(c, st, gamma0, delz);
     launch_push(c->stream, c->nblk, c->d_blk_slice, c->d_blk_begin, c->d_off, c->d_g, c->d_th,
                 c->d_x, c->d_y, c->d_px, c->d_py, c->d_field, c->d_esc, c->d_ez, p);
     if (c->ev) G4_HIP(hipEventRecord(c->ev[3], c->stream));
@@ -546,7 +579,7 @@ struct AdiField {
     const AdiPlan *p;
     const double2 *src;
     const int4 *box;
-    double *tilediag, *diag;
+    double *tilediag, *diag;  // the tiles' sums stay per tile: launch_record or launch_tile_sums folds them
 };
 
 static bool adi_eligible(const AdiField &a, int kind) {
@@ -566,7 +599,7 @@ static void adi_launch(Ctx *c, int kind, const AdiField &a, double2 *fin, double
                                 p.band_m, p.klo, p.khi, a.diag);
     else if (kind == 3)
         launch_adi_band(c->stream, c->ns, fin, fout, a.src, a.box, p.band, p.cstep, a.ng, c->first, p.band_m,
-                        p.klo, p.khi, a.tilediag, a.diag);
+                        p.klo, p.khi, a.tilediag, nullptr);
     else if (kind == 1 || kind == 2)
         launch_adi_fused(c->stream, c->ns, fin, fout, a.src, a.box, f, c->first, a.diag, p.tile, kind == 2);
     else
@@ -833,7 +866,21 @@ static int fft_field_step(Ctx *c, double delz) {
 // and the ADI with the field's own tables, in the fastest of its kernels
 // (97 slices at 151^2: 48 us a step in the banded tiles, 317 us in the
 // two Thomas sweeps that every harmonic field ran before).
-static int harmonics_track(Ctx *c, const g4mi_step_params &st, double delz) {
+// The source of one field: split over blocks of particles (small windows,
+// split_step) or one workgroup per slice.
+static void deposit_field(Ctx *c, bool split, const DepositParams &d, double2 *src, int4 *box, const SplitPlane &sp,
+                          bool fundamental) {
+    if (!split || !d.enabled) {
+        launch_deposit(c->stream, c->ns, c->d_off, c->d_g, c->d_th, c->d_x, c->d_y, c->d_cur, src, box, d);
+        return;
+    }
+    const int q = c->split_par;
+    launch_deposit_split(c->stream, c->ns, c->ntot, c->maxn, c->d_off, c->d_g, c->d_th, c->d_x, c->d_y, c->d_cur,
+                         c->d_pmax[q], fundamental ? c->d_pmax[q ^ 1] : nullptr, sp.acc, sp.corner[q],
+                         sp.corner[q ^ 1], src, box, d);
+}
+
+static int harmonics_track(Ctx *c, const g4mi_step_params &st, double delz, bool split) {
     for (Ctx::HField &h : c->hf) {
         AdiPlan p;
         G4_TRY(adi_plan(c, h.plans, h.ng, h.dgrid, h.xks, delz, &p));
@@ -852,7 +899,7 @@ static int harmonics_track(Ctx *c, const g4mi_step_params &st, double delz) {
         d.gradx = st.gradx;
         d.grady = st.grady;
         d.ngrid = h.ng;
-        launch_deposit(c->stream, c->ns, c->d_off, c->d_g, c->d_th, c->d_x, c->d_y, c->d_cur, h.d_src, h.d_box, d);
+        deposit_field(c, split, d, h.d_src, h.d_box, h.split, false);
         const AdiField a{h.ng, &p, h.d_src, h.d_box, nullptr, nullptr};
         // the fundamental's rules: a fixed kernel where it is eligible, the
         // tuner's choice for the step size otherwise
@@ -874,12 +921,12 @@ static int harmonics_track(Ctx *c, const g4mi_step_params &st, double delz) {
     return G4MI_OK;
 }
 
-static int field_track(Ctx *c, const g4mi_step_params &st, double delz, bool deposit = true) {
+static int field_track(Ctx *c, const g4mi_step_params &st, double delz, bool deposit = true, bool split = false) {
     if (!c->has_field) {
         set_error("field not uploaded");
         return G4MI_E_STATE;
     }
-    if (!c->hf.empty()) G4_TRY(harmonics_track(c, st, delz));
+    if (!c->hf.empty()) G4_TRY(harmonics_track(c, st, delz, split));
     if (!c->fft) G4_TRY(ensure_factors(c, delz));
     if (c->ev) G4_HIP(hipEventRecord(c->ev[5], c->stream));
     DepositParams d{};
@@ -897,9 +944,8 @@ static int field_track(Ctx *c, const g4mi_step_params &st, double delz, bool dep
     d.gradx = st.gradx;
     d.grady = st.grady;
     d.ngrid = c->ng;
-    if (deposit)
-        launch_deposit(c->stream, c->ns, c->d_off, c->d_g, c->d_th, c->d_x, c->d_y, c->d_cur,
-                       c->d_src, c->d_box, d);
+    if (deposit) deposit_field(c, split, d, c->d_src, c->d_box, c->split, true);
+    if (split && d.enabled) c->split_par ^= 1;
     if (c->ev) G4_HIP(hipEventRecord(c->ev[6], c->stream));
     if (c->fft) {
         G4_TRY(fft_field_step(c, delz));
@@ -914,6 +960,7 @@ static int field_track(Ctx *c, const g4mi_step_params &st, double delz, bool dep
         c->adi_choice[c->adi_delz] = c->adi_kernel;
     }
     adi_launch(c, c->adi_kernel, a, c->d_field, c->d_work);
+    c->tiles_fresh = c->adi_kernel == 3;
     if (c->adi_kernel >= 3) std::swap(c->d_field, c->d_work);  // result is in the other buffer
     c->field_diag_fresh = c->adi_kernel != 0;
     c->zeroed_since_adi.clear();
@@ -1258,7 +1305,12 @@ static int diag(Ctx *c, g4mi_diag_out *o) {
     const int ns = c->ns, ng = c->ng;
     launch_diag_beam(c->stream, ns, c->d_off, c->d_g, c->d_th, c->d_x, c->d_y, c->d_diag_b);
     // the fused ADI already summed the field of this step; otherwise sum now
-    if (!c->field_diag_fresh) launch_diag_field(c->stream, ns, c->d_field, ng, c->d_diag_f);
+    if (!c->field_diag_fresh) {
+        launch_diag_field(c->stream, ns, c->d_field, ng, c->d_diag_f);
+    } else if (c->tiles_fresh) {
+        launch_tile_sums(c->stream, ns, c->d_tilediag, ng, c->d_diag_f);
+        c->tiles_fresh = false;
+    }
     std::vector<double> hb(8 * (size_t)ns), hf(8 * (size_t)ns);
     G4_HIP(hipMemcpyAsync(hb.data(), c->d_diag_b, hb.size() * 8, hipMemcpyDeviceToHost, c->stream));
     G4_HIP(hipMemcpyAsync(hf.data(), c->d_diag_f, hf.size() * 8, hipMemcpyDeviceToHost, c->stream));
@@ -1348,13 +1400,18 @@ static int sort_beam(Ctx *c) {
     for (int s = 0; s < c->ns; s++) c->h_cur[s] = (double)(c->off[s + 1] - c->off[s]) * kCe / c->slicelength;
     std::vector<int> bs;
     std::vector<long long> bb;
-    build_block_table(c->off, bs, bb);
+    std::vector<long long> bf;
+    build_block_table(c->off, bs, bb, bf);
+    c->maxn = 0;
+    for (int q = 0; q < c->ns; q++) c->maxn = std::max(c->maxn, c->off[q + 1] - c->off[q]);
     if ((int)bs.size() > c->blk_cap) {
         set_error("sort: block table capacity exceeded");
         return G4MI_E_STATE;
     }
     c->nblk = (int)bs.size();
     G4_HIP(hipMemcpyAsync(c->d_cur, c->h_cur.data(), c->ns * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    G4_HIP(hipMemcpyAsync(c->d_blk_first, bf.data(), bf.size() * sizeof(long long), hipMemcpyHostToDevice,
+                          c->stream));
     if (c->nblk) {
         G4_HIP(hipMemcpyAsync(c->d_blk_slice, bs.data(), bs.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
         G4_HIP(hipMemcpyAsync(c->d_blk_begin, bb.data(), bb.size() * sizeof(long long), hipMemcpyHostToDevice,
@@ -1472,15 +1529,125 @@ static int fused_step(Ctx *c, const g4mi_step_params &st, double gamma0, double 
     return G4MI_OK;
 }
 
+// The split path's device state, allocated on its first step.  Where it does
+// not fit, the context keeps to the other kernels.
+static int split_alloc(Ctx *c) {
+    bool ok = true;
+    auto get = [&](auto **p, size_t n, int fill) {
+        if (!ok || *p) return;
+        void *q = nullptr;
+        if (hipMalloc(&q, n * sizeof(**p)) != hipSuccess) {
+            (void)hipGetLastError();
+            ok = false;
+            return;
+        }
+        c->allocs.push_back(q);
+        *p = (std::remove_reference_t<decltype(*p)>)q;
+        if (fill) {  // empty corners
+            const std::vector<int> none(n, 1 << 30);
+            ok = hipMemcpy(q, none.data(), n * sizeof(int), hipMemcpyHostToDevice) == hipSuccess;
+        } else {
+            ok = hipMemsetAsync(q, 0, n * sizeof(**p), c->stream) == hipSuccess;
+        }
+    };
+    const size_t ns = (size_t)c->ns;
+    get(&c->d_part, 8 * (size_t)c->blk_cap, 0);
+    for (int q = 0; q < 2; q++) get(&c->d_pmax[q], ns, 0);
+    auto plane = [&](SplitPlane &sp, int ng) {
+        get(&sp.acc, 2 * ns * ng * ng, 0);
+        for (int q = 0; q < 2; q++) get(&sp.corner[q], 4 * ns, 1);
+    };
+    plane(c->split, c->ng);
+    for (Ctx::HField &h : c->hf) plane(h.split, h.ng);
+    c->split_off = !ok;
+    return G4MI_OK;
+}
+
+// Whether a step takes the split path: a window too small to fill the chip
+// with a workgroup per slice (the fused kernels' rule), no energy kicks
+// between the push and R56, no sort between the beam and the field track.
+static bool splittable(const Ctx *c, const g4mi_step_params &st) {
+    if (c->split_off || c->ns >= kFuseMinSlices || !c->has_beam || !c->has_field) return false;
+    if (c->incoh && st.aw > 0 && (c->incoh_loss || c->incoh_spread)) return false;
+    return !c->d_wake && !((st.marker & 4) && c->one4one);
+}
+
+static int split_step(Ctx *c, const g4mi_step_params &st, double gamma0, double delz) {
+    TrackParams f{};
+    f.t1 = transverse_params(c, st, gamma0, delz * 0.5, false);
+    f.t2 = transverse_params(c, st, gamma0, delz * 0.5, true);
+    f.p = push_params(c, st, gamma0, delz);
+    f.first = !(c->longrange || f.p.use_sc);
+    f.chicane = st.chic_angle != 0 ? 1 : 0;
+    if (f.chicane) f.r56 = chicane_r56(st.chic_angle, st.chic_lb, st.chic_ld, c->lambda0, gamma0);
+    f.gamma0 = gamma0;
+    f.d.enabled = st.aw > 0 ? 1 : 0;
+    f.d.ax = st.ax;
+    f.d.ay = st.ay;
+    f.d.kx = st.kx;
+    f.d.ky = st.ky;
+    f.d.gradx = st.gradx;
+    f.d.grady = st.grady;
+    if (c->ev) G4_HIP(hipEventRecord(c->ev[0], c->stream));
+    if (!f.first) launch_transverse(c->stream, c->ntot, c->d_g, c->d_x, c->d_y, c->d_px, c->d_py, f.t1);
+    if (c->ev) G4_HIP(hipEventRecord(c->ev[1], c->stream));
+    if (!f.first) space_charge(c, st, gamma0);
+    if (c->ev) G4_HIP(hipEventRecord(c->ev[2], c->stream));
+    launch_track(c->stream, c->nblk, c->d_blk_slice, c->d_blk_begin, c->d_off, c->d_g, c->d_th, c->d_x, c->d_y,
+                 c->d_px, c->d_py, c->d_field, c->d_esc, c->d_ez, f, c->d_part, c->d_pmax[c->split_par]);
+    if (c->ev) {
+        G4_HIP(hipEventRecord(c->ev[3], c->stream));
+        G4_HIP(hipEventRecord(c->ev[4], c->stream));
+    }
+    G4_HIP(hipGetLastError());
+    G4_TRY(field_track(c, st, delz, true, true));
+    c->beampart_fresh = true;
+    return G4MI_OK;
+}
+
+// Deferred records of the FP64 run loop: each record's beam and field sums
+// (and, when asked for, the auxiliary sums with the space-charge fields and
+// the spectral moments) are written into a pinned slot by copy kernels on
+// the step's stream, and the host finishes them when the slots are full or
+// the run ends, so a record after every step does not stall the device
+// between steps (one4one runs finish theirs before a sort changes the slices).
+static int flush_records(Ctx *c) {
+    if (c->pend.empty()) return G4MI_OK;
+    G4_HIP(hipStreamSynchronize(c->stream));
+    const size_t ns = (size_t)c->ns, row = kRecRow * ns;
+    std::vector<double> hb(8 * ns), hf(8 * ns);
+    for (size_t k = 0; k < c->pend.size(); k++) {
+        Ctx::PendingRecord &r = c->pend[k];
+        const double *slot = c->h_recs + k * row;
+        std::copy(slot, slot + 8 * ns, hb.begin());
+        std::copy(slot + 8 * ns, slot + 16 * ns, hf.begin());
+        if (r.fresh)  // slices zeroed by slippage after the ADI's sums
+            for (int z : r.zeroed)
+                for (int q = 0; q < 8; q++) hf[8 * (size_t)z + q] = 0;
+        finish_diag(c, hb, hf, r.first, &r.out);
+        if (wants_aux(&r.out)) finish_aux(c, slot + 16 * ns, slot + 32 * ns, slot + 33 * ns, r.wake, &r.out);
+        if (wants_spectral(&r.out)) finish_spectral(c, slot + 34 * ns, r.first, &r.out);
+    }
+    c->pend.clear();
+    return G4MI_OK;
+}
+
 static int step(Ctx *c, const g4mi_step_params &st, double gamma0) {
     const double delz = st.dz;
-    c->beamsum_fresh = false;
+    c->beamsum_fresh = c->beampart_fresh = false;
     G4_TRY(step_begin_timing(c));
     if (fp64_fusable(c, st)) {
         G4_TRY(fused_step(c, st, gamma0, delz));
+    } else if (splittable(c, st)) {
+        G4_TRY(split_alloc(c));
+        if (c->split_off) return step(c, st, gamma0);
+        G4_TRY(split_step(c, st, gamma0, delz));
     } else {
         G4_TRY(beam_track(c, st, gamma0, delz));
-        if ((st.marker & 4) && c->one4one) G4_TRY(sort_beam(c));  // Gencore.cpp:124-134
+        if ((st.marker & 4) && c->one4one) {  // Gencore.cpp:124-134
+            G4_TRY(flush_records(c));         // with the slices that they were taken of
+            G4_TRY(sort_beam(c));
+        }
         G4_TRY(field_track(c, st, delz));
     }
     G4_TRY(slippage(c, st.slip));
@@ -2407,13 +2574,16 @@ int g4mi_create(g4mi_ctx **out, int device, int nslice, const long long *off, in
     if (fp64 && (rc = alloc_records(c))) return fail(rc);
     std::vector<int> bs;
     std::vector<long long> bb;
-    build_block_table(c->off, bs, bb);
+    std::vector<long long> bf;
+    build_block_table(c->off, bs, bb, bf);
     c->nblk = (int)bs.size();
     // capacity for any redistribution of the particles over the slices
     c->blk_cap = (int)(ns + (size_t)c->ntot / 256 + 1);
-    if ((rc = dalloc(c, &c->d_blk_slice, (size_t)c->blk_cap)) || (rc = dalloc(c, &c->d_blk_begin, (size_t)c->blk_cap)))
+    if ((rc = dalloc(c, &c->d_blk_slice, (size_t)c->blk_cap)) ||
+        (rc = dalloc(c, &c->d_blk_begin, (size_t)c->blk_cap)) || (rc = dalloc(c, &c->d_blk_first, ns + 1)))
         return fail(rc);
-    if (hipMemcpy(c->d_off, off, (ns + 1) * sizeof(long long), hipMemcpyHostToDevice) != hipSuccess ||
+    if (hipMemcpy(c->d_blk_first, bf.data(), (ns + 1) * sizeof(long long), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(c->d_off, off, (ns + 1) * sizeof(long long), hipMemcpyHostToDevice) != hipSuccess ||
         (c->nblk && hipMemcpy(c->d_blk_slice, bs.data(), bs.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess) ||
         (c->nblk && hipMemcpy(c->d_blk_begin, bb.data(), bb.size() * sizeof(long long), hipMemcpyHostToDevice) != hipSuccess) ||
         hipMemset(c->d_esc, 0, ns * sizeof(double)) != hipSuccess ||
@@ -2952,64 +3122,40 @@ int g4mi_step(g4mi_ctx *h, const g4mi_step_params *st, double gammaref) {
     return step_end_timing(&h->c);
 }
 
-// Deferred records of the FP64 run loop: each record's beam and field sums
-// (and, when asked for, the auxiliary sums with the space-charge fields and
-// the spectral moments) are written into a pinned slot by copy kernels on
-// the step's stream, and the host finishes them when the slots are full or
-// the run ends, so a record after every step does not stall the device
-// between steps.  one4one runs (whose slices change at sorts) take the
-// synchronous path.
-static bool record_deferrable(const Ctx *c, const g4mi_diag_out *o) {
-    (void)o;
-    return !c->one4one;
-}
-
-static int flush_records(Ctx *c) {
-    if (c->pend.empty()) return G4MI_OK;
-    G4_HIP(hipStreamSynchronize(c->stream));
-    const size_t ns = (size_t)c->ns, row = kRecRow * ns;
-    std::vector<double> hb(8 * ns), hf(8 * ns);
-    for (size_t k = 0; k < c->pend.size(); k++) {
-        Ctx::PendingRecord &r = c->pend[k];
-        const double *slot = c->h_recs + k * row;
-        std::copy(slot, slot + 8 * ns, hb.begin());
-        std::copy(slot + 8 * ns, slot + 16 * ns, hf.begin());
-        if (r.fresh)  // slices zeroed by slippage after the ADI's sums
-            for (int z : r.zeroed)
-                for (int q = 0; q < 8; q++) hf[8 * (size_t)z + q] = 0;
-        finish_diag(c, hb, hf, r.first, &r.out);
-        if (wants_aux(&r.out)) finish_aux(c, slot + 16 * ns, slot + 32 * ns, slot + 33 * ns, r.wake, &r.out);
-        if (wants_spectral(&r.out)) finish_spectral(c, slot + 34 * ns, r.first, &r.out);
-    }
-    c->pend.clear();
-    return G4MI_OK;
-}
-
 static int enqueue_record(Ctx *c, const g4mi_diag_out *o) {
     const size_t ns = (size_t)c->ns, row = kRecRow * ns;
     if (!c->h_recs) G4_TRY(alloc_records(c));
     if ((int)c->pend.size() == c->rec_cap) G4_TRY(flush_records(c));
-    // the beam sums go straight into the slot; the field sums of the ADI
-    // (or of k_diag_field) are copied after them
     double *slot = c->d_recs + c->pend.size() * row;
-    if (c->beamsum_fresh)  // the fused main kernel summed the step's particles
-        launch_copy_out(c->stream, c->d_beamsum, slot, (long long)(8 * ns));
-    else
+    RecordSources r{};
+    if (c->beampart_fresh) {  // the step summed its particles per block
+        r.part = c->d_part;
+        r.blk_first = c->d_blk_first;
+    } else if (c->beamsum_fresh) {  // per slice (fused main kernel)
+        r.beam = c->d_beamsum;
+    } else {
         launch_diag_beam(c->stream, c->ns, c->d_off, c->d_g, c->d_th, c->d_x, c->d_y, slot);
-    if (!c->field_diag_fresh) launch_diag_field(c->stream, c->ns, c->d_field, c->ng, c->d_diag_f);
-    launch_copy_out(c->stream, c->d_diag_f, slot + 8 * ns, (long long)(8 * ns));
+    }
+    r.field = c->d_diag_f;
+    if (!c->field_diag_fresh) {
+        launch_diag_field(c->stream, c->ns, c->d_field, c->ng, c->d_diag_f);
+    } else if (c->tiles_fresh) {
+        r.tiles = c->d_tilediag;
+        r.ntiles = adi_band_tiles(c->ng);
+    }
     std::vector<double> wake;
     if (wants_aux(o)) {
         G4_TRY(launch_aux(c));
-        launch_copy_out(c->stream, c->d_aux, slot + 16 * ns, (long long)(16 * ns));
-        launch_copy_out(c->stream, c->d_esc, slot + 32 * ns, (long long)ns);
-        launch_copy_out(c->stream, c->d_efield, slot + 33 * ns, (long long)ns);
+        r.aux = c->d_aux;
+        r.esc = c->d_esc;
+        r.ssc = c->d_efield;
         wake = c->wake_applied;
     }
     if (wants_spectral(o)) {
         G4_TRY(spectral_moments(c, c->d_field));
-        launch_copy_out(c->stream, c->d_fft_mom, slot + 34 * ns, (long long)(5 * ns));
+        r.mom = c->d_fft_mom;
     }
+    launch_record(c->stream, c->ns, r, slot);
     G4_HIP(hipGetLastError());
     c->pend.push_back({*o, c->first, c->field_diag_fresh, c->zeroed_since_adi, std::move(wake)});
     return G4MI_OK;
@@ -3028,14 +3174,7 @@ int g4mi_run(g4mi_ctx *h, const g4mi_step_params *steps, int nsteps, double gamm
     for (int i = 0; i < nsteps && rc == G4MI_OK; i++) {
         if (steps[i].marker & 8) break;
         rc = step(c, steps[i], gammaref);
-        if (rc == G4MI_OK && records) {
-            if (record_deferrable(c, &records[i])) {
-                rc = enqueue_record(c, &records[i]);
-            } else {
-                rc = flush_records(c);
-                if (rc == G4MI_OK) rc = diag(c, &records[i]);
-            }
-        }
+        if (rc == G4MI_OK && records) rc = enqueue_record(c, &records[i]);
         if (rc == G4MI_OK) rc = step_end_timing(c);
         if (rc == G4MI_OK) done++;
     }

@@ -69,6 +69,27 @@ void launch_fp64_main(hipStream_t s, int ns, const long long *off, double *g, do
                       double *px, double *py, const double2 *field, const double *esc, const double *cur,
                       const double *cen, const double *dr, double *efield, const int4 *pbox,
                       const double *pmaxf, double2 *src, int4 *box, double *beamsum, const FuseParams &f);
+// The particle half of a step over blocks of particles (small windows).
+// track: the push, R56 and second half step, the first half step before them
+// when `first`; per-block sums part[8 nblocks], per-slice pmax.
+struct TrackParams {
+    PushParams p;
+    TransParams t1, t2;
+    DepositParams d;               // the fundamental's (its enabled and faw2 terms)
+    double r56, gamma0;            // R56 (chicane != 0)
+    int chicane, first;
+};
+void launch_track(hipStream_t s, int nblocks, const int *blk_slice, const long long *blk_begin,
+                  const long long *off, double *g, double *th, double *x, double *y, double *px, double *py,
+                  const double2 *field, const double *esc, const double *ezsc, const TrackParams &f, double *part,
+                  unsigned long long *pmax);
+// The deposit split over the slices' particles: acc (ns ngrid^2 fixed-point
+// cells, all zero before and after) and corner (4 ns) of this step; leaves
+// corner_next and, unless null, pmax_next empty for the next one.
+void launch_deposit_split(hipStream_t s, int ns, long long ntot, long long maxn, const long long *off,
+                          const double *g, const double *th, const double *x, const double *y, const double *cur,
+                          const unsigned long long *pmax, unsigned long long *pmax_next, long long *acc,
+                          int *corner, int *corner_next, double2 *src, int4 *box, const DepositParams &p);
 void launch_deposit(hipStream_t s, int ns, const long long *off, const double *g,
                     const double *th, const double *x, const double *y, const double *cur,
                     double2 *src, int4 *box, const DepositParams &p);
@@ -86,8 +107,9 @@ int launch_adi_fused(hipStream_t s, int ns, double2 *field, double2 *work, const
 // [ngrid][2M+1] complex rows of A^-1 around the diagonal, a = Im(cstep).
 // m: 7, 8 or 12.  Rows [klo, khi] of the band equal row (klo+khi)/2 to
 // 2^-60.  tilediag: scratch [ns][adi_band_tiles(ngrid)][8], or null: no
-// field sums.
+// field sums; diag null: the tiles' sums are left for launch_tile_sums.
 int adi_band_tiles(int ng);
+void launch_tile_sums(hipStream_t s, int ns, const double *tilediag, int ng, double *diag);
 int launch_adi_band(hipStream_t s, int ns, const double2 *fin, double2 *fout, const double2 *src,
                     const int4 *box, const double2 *band, double a, int ng, int first, int m,
                     int klo, int khi, double *tilediag, double *diag);
@@ -101,8 +123,17 @@ int launch_adi_wide64(hipStream_t s, int ns, const double2 *fin, double2 *fout, 
                       const int4 *box, const double2 *band, double a, int ng, int first, int m, int klo, int khi,
                       double *diag);
 void launch_zero(hipStream_t s, double2 *p, long long n);
-// n doubles from device memory to pinned host memory (dst: its device address)
-void launch_copy_out(hipStream_t s, const double *src, double *dst, long long n);
+// A record's slot (device address of pinned memory): beam sums [8 ns] from
+// part (per block of the slices' blk_first ranges) or beam, or left alone;
+// field sums [8 ns] from tiles (ntiles per slice) or field; with aux the
+// auxiliary sums [16 ns] and the space-charge fields esc, ssc [ns each]; with
+// mom the spectral moments [5 ns].
+struct RecordSources {
+    const double *part, *beam, *tiles, *field, *aux, *esc, *ssc, *mom;
+    const long long *blk_first;
+    int ntiles;
+};
+void launch_record(hipStream_t s, int ns, const RecordSources &r, double *slot);
 // harmonic bunching sums for h0 .. h0 + cnt - 1 (cnt <= 8), out[ns][cnt][2]
 void launch_diag_bunch(hipStream_t s, int ns, const long long *off, const double *th, int h0, int cnt,
                        double *out);

@@ -489,24 +489,12 @@ struct Ode {
     }
 };
 
+// The push of one particle (theta with the autophase added; ez: its
+// short-range field).
 template <int NH>
-__global__ void __launch_bounds__(256) k_push(const int *__restrict__ blk_slice,
-                                              const long long *__restrict__ blk_begin,
-                                              const long long *__restrict__ off,
-                                              double *__restrict__ g, double *__restrict__ th,
-                                              const double *__restrict__ x,
-                                              const double *__restrict__ y,
-                                              const double *__restrict__ px,
-                                              const double *__restrict__ py,
-                                              const double2 *__restrict__ field,
-                                              const double *__restrict__ esc,
-                                              const double *__restrict__ ezsc, PushParams p) {
-    const int is = blk_slice[blockIdx.x];
-    const long long i = blk_begin[blockIdx.x] + threadIdx.x;
-    if (i >= off[is + 1]) return;
-    double gamma = g[i];
-    double theta = th[i] + p.autophase;
-    const double xi = x[i], yi = y[i], pxi = px[i], pyi = py[i];
+__device__ __forceinline__ void push_one(const PushParams &p, int is, const double2 *__restrict__ field,
+                                         const double *__restrict__ esc, double ez, double xi, double yi,
+                                         double pxi, double pyi, double &gamma, double &theta) {
     double dx = xi - p.ax, dy = yi - p.ay;
     double awloc = (1 + 0.5 * (p.kx * dx * dx + p.ky * dy * dy) + p.gradx * dx + p.grady * dy);
     Ode<NH> o;
@@ -514,7 +502,7 @@ __global__ void __launch_bounds__(256) k_push(const int *__restrict__ blk_slice,
     o.xku = p.xku;
     o.btpar = 1 + pxi * pxi + pyi * pyi + p.aw * p.aw * awloc * awloc;
     double eloss = -esc[is] / kEev;
-    o.ez = (p.use_sc ? ezsc[i] : 0.0) + eloss;
+    o.ez = ez + eloss;
     if ((xi > -p.gridmax) && (xi < p.gridmax) && (yi > -p.gridmax) && (yi < p.gridmax)) {
         double wx = (xi + p.gridmax) / p.dgrid;
         double wy = (yi + p.gridmax) / p.dgrid;
@@ -590,6 +578,26 @@ __global__ void __launch_bounds__(256) k_push(const int *__restrict__ blk_slice,
     o.eval(gamma, theta);
     gamma += stpz * (k3gg + o.k2gg / 6.0);
     theta += stpz * (k3pp + o.k2pp / 6.0);
+}
+
+template <int NH>
+__global__ void __launch_bounds__(256) k_push(const int *__restrict__ blk_slice,
+                                              const long long *__restrict__ blk_begin,
+                                              const long long *__restrict__ off,
+                                              double *__restrict__ g, double *__restrict__ th,
+                                              const double *__restrict__ x,
+                                              const double *__restrict__ y,
+                                              const double *__restrict__ px,
+                                              const double *__restrict__ py,
+                                              const double2 *__restrict__ field,
+                                              const double *__restrict__ esc,
+                                              const double *__restrict__ ezsc, PushParams p) {
+    const int is = blk_slice[blockIdx.x];
+    const long long i = blk_begin[blockIdx.x] + threadIdx.x;
+    if (i >= off[is + 1]) return;
+    double gamma = g[i];
+    double theta = th[i] + p.autophase;
+    push_one<NH>(p, is, field, esc, p.use_sc ? ezsc[i] : 0.0, x[i], y[i], px[i], py[i], gamma, theta);
     g[i] = gamma;
     th[i] = theta;
 }
@@ -1260,6 +1268,228 @@ __global__ void __launch_bounds__(kFuseNT, GEN ? 2 : 4) k_fp64_main(const long l
             plane[ry * ng + rx] = make_double2((double)pre[k] / fs2, (double)pim[k] / fs2);
         }
         __syncthreads();
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The particle half of a step for windows too small to fill the chip with one
+// workgroup per slice: every pass runs over blocks of the particles, not over
+// slices, and a slice's sums are put together from its blocks' in a fixed
+// order.
+//
+// k_track: push (k_push), R56 (k_r56) and second transverse half step, before
+// them the first one where no space-charge pass needs its positions first;
+// the sums of DiagBeam per block (part[8 block]) and the slice's largest
+// sqrt(faw2) / gamma (pmax, the deposit's fixed-point scale: a maximum, so
+// the order of the atomics does not matter).
+// k_deposit_part: the source of `chunk` particles in an LDS tile over their
+// own footprint, its cells then added to the slice's fixed-point plane with
+// integer atomics (any order, the same bits); particles spread over more cells
+// than the tile holds go to the plane directly.  k_deposit_out turns the
+// plane's cells inside the footprint of the whole slice into the source and
+// clears them for the next step.
+//
+// One slice of 8192 particles at 151^2: the two transverse kernels, the push,
+// k_diag_beam and k_deposit took 3 + 5 + 3 + 13 + 33 us, most of it one
+// workgroup's latency.
+// ---------------------------------------------------------------------------
+template <int NH>
+__global__ void __launch_bounds__(256) k_track(const int *__restrict__ blk_slice,
+                                               const long long *__restrict__ blk_begin,
+                                               const long long *__restrict__ off, double *__restrict__ g,
+                                               double *__restrict__ th, double *__restrict__ x,
+                                               double *__restrict__ y, double *__restrict__ px,
+                                               double *__restrict__ py, const double2 *__restrict__ field,
+                                               const double *__restrict__ esc, const double *__restrict__ ezsc,
+                                               TrackParams f, double *__restrict__ part,
+                                               unsigned long long *__restrict__ pmax) {
+    __shared__ double red[8 * 4];
+    const int is = blk_slice[blockIdx.x], t = threadIdx.x;
+    const long long i = blk_begin[blockIdx.x] + t;
+    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0}, m = 0;
+    if (i < off[is + 1]) {
+        double gamma = g[i], theta = th[i];
+        double xi = x[i], yi = y[i], pxi = px[i], pyi = py[i];
+        if (f.first) transverse_one(f.t1, gamma, xi, yi, pxi, pyi);
+        theta += f.p.autophase;
+        push_one<NH>(f.p, is, field, esc, f.p.use_sc ? ezsc[i] : 0.0, xi, yi, pxi, pyi, gamma, theta);
+        if (f.chicane) theta += f.r56 * (gamma - f.gamma0);
+        transverse_one(f.t2, gamma, xi, yi, pxi, pyi);
+        g[i] = gamma;
+        th[i] = theta;
+        x[i] = xi;
+        y[i] = yi;
+        px[i] = pxi;
+        py[i] = pyi;
+        double s, c;
+        sincos64(theta, &s, &c);
+        v[0] = gamma;
+        v[1] = gamma * gamma;
+        v[2] = xi;
+        v[3] = xi * xi;
+        v[4] = yi;
+        v[5] = yi * yi;
+        v[6] = c;
+        v[7] = s;
+        if (f.d.enabled) {
+            const double dx = xi - f.d.ax, dy = yi - f.d.ay;
+            const double faw2 = (1 + f.d.kx * dx * dx + f.d.ky * dy * dy + 2 * (f.d.gradx * dx + f.d.grady * dy));
+            m = fmax(0.0, sqrt(faw2) / fabs(gamma));
+        }
+    }
+    block_sum_waves<256, 8>(v, red);
+    if (t == 0)
+        for (int k = 0; k < 8; k++) part[8 * (long long)blockIdx.x + k] = v[k];
+    if (!f.d.enabled) return;  // uniform
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+    if ((t & 63) == 0) red[t >> 6] = m;
+    __syncthreads();
+    if (t == 0) {
+        m = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+        atomicMax(&pmax[is], (unsigned long long)__double_as_longlong(m));  // m >= 0: ordered as its bits
+    }
+}
+
+constexpr int kPartTile = 3072;       // cells of k_deposit_part's tile (48 KiB: three workgroups per CU)
+constexpr int kDepNone = 1 << 30;     // footprint corner of no particle
+
+// fixed-point scale of slice is: no cell sums to more than n max|part|
+__device__ __forceinline__ double dep_scale(const DepositParams &p, double cur, long long n, double pmax,
+                                            double *scl) {
+    const double scl0 = p.fcoup * kVacimp * cur * p.xks * p.delz;
+    *scl = scl0 / (4 * kEev * (double)n * p.dgrid * p.dgrid);
+    return fx_scale((double)n * pmax * fabs(*scl));
+}
+
+__global__ void __launch_bounds__(256) k_deposit_part(const long long *__restrict__ off,
+                                                      const double *__restrict__ g, const double *__restrict__ th,
+                                                      const double *__restrict__ x, const double *__restrict__ y,
+                                                      const double *__restrict__ cur,
+                                                      const unsigned long long *__restrict__ pmax,
+                                                      long long *__restrict__ acc, int *__restrict__ corner,
+                                                      DepositParams p, int chunk) {
+    __shared__ long long tile[2 * kPartTile];
+    __shared__ int ired[4 * 4];
+    const int is = blockIdx.y, t = threadIdx.x, ng = p.ngrid;
+    const long long a = off[is] + (long long)blockIdx.x * chunk;
+    const long long b = min(off[is + 1], a + chunk);
+    if (a >= b) return;  // uniform
+    double scl;
+    const double fs = dep_scale(p, cur[is], off[is + 1] - off[is], __longlong_as_double((long long)pmax[is]), &scl);
+    const Recip rgrid = {p.dgrid, 1 / p.dgrid};
+    auto inside = [&](double xi, double yi) {
+        return (xi > -p.gridmax) && (xi < p.gridmax) && (yi > -p.gridmax) && (yi < p.gridmax);
+    };
+    int bv[4] = {kDepNone, kDepNone, kDepNone, kDepNone};
+    for (long long i = a + t; i < b; i += 256) {
+        const double xi = x[i], yi = y[i];
+        if (!inside(xi, yi)) continue;
+        const int ix = min((int)floor(quot(xi + p.gridmax, rgrid)), ng - 2);
+        const int iy = min((int)floor(quot(yi + p.gridmax, rgrid)), ng - 2);
+        bv[0] = min(bv[0], ix);
+        bv[1] = min(bv[1], iy);
+        bv[2] = min(bv[2], -(ix + 1));
+        bv[3] = min(bv[3], -(iy + 1));
+    }
+    block_min_waves<256, 4>(bv, ired);
+    if (bv[0] == kDepNone) return;  // uniform
+    if (t < 4) atomicMin(&corner[4 * is + t], t == 0 ? bv[0] : t == 1 ? bv[1] : t == 2 ? bv[2] : bv[3]);
+    const int bx0 = bv[0], by0 = bv[1], ww = -bv[2] - bx0 + 1, ncell = ww * (-bv[3] - by0 + 1);
+    const bool local = ncell <= kPartTile;
+    long long *plane = acc + 2LL * is * ng * ng;
+    if (local)
+        for (int k = t; k < 2 * ncell; k += 256) tile[k] = 0;
+    __syncthreads();
+    // the same trip count for every lane, so that the lanes of a group of
+    // four (a beamlet's particles at one position) combine their values first
+    for (long long base = a; base < b; base += 256) {
+        const long long i = base + t;
+        bool act = i < b;
+        double xi = 0, yi = 0;
+        if (act) {
+            xi = x[i];
+            yi = y[i];
+            act = inside(xi, yi);
+        }
+        int ix = 0, iy = 0;
+        double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // (re, im) for cells (ix,iy) (ix+1,iy) (ix,iy+1) (ix+1,iy+1)
+        if (act) {
+            double wx = quot(xi + p.gridmax, rgrid), wy = quot(yi + p.gridmax, rgrid);
+            ix = min((int)floor(wx), ng - 2);
+            iy = min((int)floor(wy), ng - 2);
+            wx = 1 + floor(wx) - wx;
+            wy = 1 + floor(wy) - wy;
+            const double dx = xi - p.ax, dy = yi - p.ay;
+            const double faw2 = (1 + p.kx * dx * dx + p.ky * dy * dy + 2 * (p.gradx * dx + p.grady * dy));
+            const double part = sqrt(faw2) * scl / g[i];
+            double s, c;
+            sincos64(p.harm * th[i], &s, &c);
+            const double wgt[4] = {wx * wy, (1 - wx) * wy, wx * (1 - wy), (1 - wx) * (1 - wy)};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                v[2 * k] = wgt[k] * (s * part);
+                v[2 * k + 1] = wgt[k] * (c * part);
+            }
+        }
+        // every lane takes all shuffles before any compare
+        const int key = act ? iy * ng + ix : -1 - (t & 3);
+        const int k1 = __shfl_xor(key, 1), k2 = __shfl_xor(key, 2), k3 = __shfl_xor(key, 3);
+        const bool grp = (key == k1) & (key == k2) & (key == k3);
+        long long iv[8], ivs[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            iv[q] = fx(v[q], fs);
+            ivs[q] = iv[q] + __shfl_xor(iv[q], 1);
+            ivs[q] += __shfl_xor(ivs[q], 2);
+        }
+        if (!act || (grp && (t & 3) != 0)) continue;
+        const long long *val = grp ? ivs : iv;
+        long long *dst = local ? tile + 2 * ((iy - by0) * ww + (ix - bx0)) : plane + 2 * (iy * ng + ix);
+        const int row = 2 * (local ? ww : ng);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            fx_add(dst + (k >> 1) * row + 2 * (k & 1), val[2 * k]);
+            fx_add(dst + (k >> 1) * row + 2 * (k & 1) + 1, val[2 * k + 1]);
+        }
+    }
+    if (!local) return;  // uniform
+    __syncthreads();
+    for (int k = t; k < ncell; k += 256) {
+        const long long re = tile[2 * k], im = tile[2 * k + 1];
+        long long *cell = plane + 2 * ((by0 + k / ww) * ng + bx0 + k % ww);
+        if (re) fx_add(cell, re);
+        if (im) fx_add(cell + 1, im);
+    }
+}
+
+__global__ void __launch_bounds__(256) k_deposit_out(const long long *__restrict__ off,
+                                                     const double *__restrict__ cur,
+                                                     const unsigned long long *__restrict__ pmax,
+                                                     long long *__restrict__ acc, const int *__restrict__ corner,
+                                                     int *__restrict__ corner_next,
+                                                     unsigned long long *__restrict__ pmax_next,
+                                                     double2 *__restrict__ src, int4 *__restrict__ box,
+                                                     DepositParams p) {
+    const int is = blockIdx.y, ng = p.ngrid;
+    const int x0 = corner[4 * is], y0 = corner[4 * is + 1], x1 = -corner[4 * is + 2], y1 = -corner[4 * is + 3];
+    const bool none = x0 == kDepNone;
+    if (blockIdx.x == 0 && threadIdx.x < 4) {
+        corner_next[4 * is + threadIdx.x] = kDepNone;  // the next step's state: nothing reads it now
+        if (threadIdx.x == 0) {
+            if (pmax_next) pmax_next[is] = 0;
+            box[is] = none ? make_int4(1, 1, 0, 0) : make_int4(x0, y0, x1, y1);
+        }
+    }
+    if (none) return;
+    double scl;
+    const double fs = dep_scale(p, cur[is], off[is + 1] - off[is], __longlong_as_double((long long)pmax[is]), &scl);
+    const double ifs = 1 / fs;  // a power of two: exact
+    const int ww = x1 - x0 + 1, ncell = ww * (y1 - y0 + 1);
+    for (int k = blockIdx.x * 256 + threadIdx.x; k < ncell; k += gridDim.x * 256) {
+        const long long idx = (long long)(y0 + k / ww) * ng + x0 + k % ww;
+        long long *cell = acc + 2 * ((long long)is * ng * ng + idx);
+        src[(long long)is * ng * ng + idx] = make_double2((double)cell[0] * ifs, (double)cell[1] * ifs);
+        cell[0] = cell[1] = 0;
     }
 }
 
@@ -2375,6 +2605,42 @@ void launch_fp64_main(hipStream_t s, int ns, const long long *off, double *g, do
                        py, field, esc, cur, cen, dr, efield, pbox, pmaxf, src, box, beamsum, f);
 }
 
+void launch_track(hipStream_t s, int nblocks, const int *blk_slice, const long long *blk_begin,
+                  const long long *off, double *g, double *th, double *x, double *y, double *px, double *py,
+                  const double2 *field, const double *esc, const double *ezsc, const TrackParams &f, double *part,
+                  unsigned long long *pmax) {
+    if (nblocks <= 0) return;
+#define G4_TRACK(NH)                                                                                             \
+    hipLaunchKernelGGL(k_track<NH>, dim3((unsigned)nblocks), dim3(256), 0, s, blk_slice, blk_begin, off, g, th, \
+                       x, y, px, py, field, esc, ezsc, f, part, pmax)
+    switch (f.p.nh) {
+    case 0: G4_TRACK(0); break;
+    case 1: G4_TRACK(1); break;
+    case 2: G4_TRACK(2); break;
+    case 3: G4_TRACK(3); break;
+    default: G4_TRACK(4); break;
+    }
+#undef G4_TRACK
+}
+// Particles per workgroup of the split deposit: 512 (two per lane) until that
+// makes more than twice the chip's workgroups, so that few particles still
+// spread over the chip and many share their tile's write-out.
+static int deposit_chunk(long long ntot) {
+    const long long c = ((ntot + 511) / 512 + 511) / 512 * 512;
+    return (int)std::min<long long>(8192, std::max<long long>(512, c));
+}
+void launch_deposit_split(hipStream_t s, int ns, long long ntot, long long maxn, const long long *off,
+                          const double *g, const double *th, const double *x, const double *y, const double *cur,
+                          const unsigned long long *pmax, unsigned long long *pmax_next, long long *acc,
+                          int *corner, int *corner_next, double2 *src, int4 *box, const DepositParams &p) {
+    const int chunk = deposit_chunk(ntot);
+    const unsigned nc = (unsigned)std::max<long long>(1, (maxn + chunk - 1) / chunk);
+    hipLaunchKernelGGL(k_deposit_part, dim3(nc, ns), dim3(256), 0, s, off, g, th, x, y, cur, pmax, acc, corner, p,
+                       chunk);
+    const unsigned nb = (unsigned)std::max(1, std::min(16, 512 / ns));
+    hipLaunchKernelGGL(k_deposit_out, dim3(nb, ns), dim3(256), 0, s, off, cur, pmax, acc, corner, corner_next,
+                       pmax_next, src, box, p);
+}
 void launch_deposit(hipStream_t s, int ns, const long long *off, const double *g,
                     const double *th, const double *x, const double *y, const double *cur,
                     double2 *src, int4 *box, const DepositParams &p) {
@@ -2426,6 +2692,9 @@ int launch_adi_fused(hipStream_t s, int ns, double2 *field, double2 *work, const
 #undef G4_ADI
     return 0;
 }
+void launch_tile_sums(hipStream_t s, int ns, const double *tilediag, int ng, double *diag) {
+    hipLaunchKernelGGL(k_adi_tile_diag, dim3((ns + 63) / 64), dim3(64), 0, s, tilediag, adi_band_tiles(ng), ns, diag);
+}
 template <int M>
 static void launch_adi_band_t(hipStream_t s, int ns, const double2 *fin, double2 *fout,
                               const double2 *src, const int4 *box, const double2 *band, double a,
@@ -2443,9 +2712,7 @@ static void launch_adi_band_t(hipStream_t s, int ns, const double2 *fin, double2
     const unsigned nblocks = (unsigned)(((ns + 7) / 8) * 8) * (unsigned)(ntx * ntx);
     hipLaunchKernelGGL(k_adi_band<M>, dim3(nblocks), dim3(256), lds, s, fin, fout, src, box,
                        band, a, ng, first, ns, ntx, klo, khi, tilediag);
-    if (tilediag)
-        hipLaunchKernelGGL(k_adi_tile_diag, dim3((ns + 63) / 64), dim3(64), 0, s, tilediag,
-                           ntx * ntx, ns, diag);
+    if (tilediag && diag) launch_tile_sums(s, ns, tilediag, ng, diag);
 }
 
 int adi_band_tiles(int ng) {
@@ -2494,16 +2761,44 @@ int launch_adi_band(hipStream_t s, int ns, const double2 *fin, double2 *fout, co
     return 0;
 }
 
-// Copy n doubles into pinned host memory (its device address) with plain
-// stores on the compute queue: a record then costs no copy-engine transfer
-// and no hand-off between the copy and compute queues.
-__global__ void __launch_bounds__(256) k_copy_out(const double *__restrict__ src, double *__restrict__ dst,
-                                                  long long n) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = src[i];
+// One record's slot in pinned host memory (its device address), written with
+// plain stores on the compute queue: a record then costs no copy-engine
+// transfer and no hand-off between the copy and compute queues, and one
+// launch.  One wavefront per slice: its beam sums (from the blocks' partial
+// sums, or copied), the field sums of the storage slice of the same number
+// (from the tiles', or copied) and the copies of the optional blocks.
+__global__ void __launch_bounds__(64) k_record(RecordSources r, int ns, double *__restrict__ slot) {
+    const int is = blockIdx.x, lane = threadIdx.x;
+    if (r.part) {
+        double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        for (long long b = r.blk_first[is] + lane; b < r.blk_first[is + 1]; b += 64)
+            for (int k = 0; k < 8; k++) v[k] += r.part[8 * b + k];
+        for (int k = 0; k < 8; k++) {
+            const double w = wave_sum(v[k]);
+            if (lane == 0) slot[8 * (long long)is + k] = w;
+        }
+    } else if (r.beam && lane < 8) {
+        slot[8 * (long long)is + lane] = r.beam[8 * (long long)is + lane];
+    }
+    double *field = slot + 8 * (long long)ns;
+    if (r.tiles) {
+        double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        for (int q = lane; q < r.ntiles; q += 64)
+            for (int k = 0; k < 8; k++) v[k] += r.tiles[((long long)is * r.ntiles + q) * 8 + k];
+        for (int k = 0; k < 8; k++) {
+            const double w = wave_sum(v[k]);
+            if (lane == 0) field[8 * (long long)is + k] = w;
+        }
+    } else if (lane < 8) {
+        field[8 * (long long)is + lane] = r.field[8 * (long long)is + lane];
+    }
+    if (r.aux && lane < 16) slot[16 * (long long)ns + 16 * (long long)is + lane] = r.aux[16 * (long long)is + lane];
+    if (r.aux && lane == 16) slot[32 * (long long)ns + is] = r.esc[is];
+    if (r.aux && lane == 17) slot[33 * (long long)ns + is] = r.ssc[is];
+    if (r.mom && lane < 5) slot[34 * (long long)ns + 5 * (long long)is + lane] = r.mom[5 * (long long)is + lane];
 }
-void launch_copy_out(hipStream_t s, const double *src, double *dst, long long n) {
-    if (n > 0) hipLaunchKernelGGL(k_copy_out, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, src, dst, n);
+void launch_record(hipStream_t s, int ns, const RecordSources &r, double *slot) {
+    hipLaunchKernelGGL(k_record, dim3(ns), dim3(64), 0, s, r, ns, slot);
 }
 void launch_zero(hipStream_t s, double2 *p, long long n) {
     if (n > 0) hipLaunchKernelGGL(k_zero, dim3(nblk(n, 256)), dim3(256), 0, s, p, n);
