@@ -28,4 +28,9 @@ void launch_to_offsets(hipStream_t s, int ns, const long long *off, long long n,
                        const double *py, float *fg, float *ft, float *fx, float *fy, float *fpx, float *fpy,
                        int maxpart);
 
+// Particles [lo, lo + n) of one coordinate back in FP64: in[i], add + in[i]
+// (plus_add) or base[slice of i] + in[i] (base set), into out[0, n)
+void launch_from_offsets(hipStream_t s, const float *in, long long lo, long long n, bool plus_add, double add,
+                         const double *base, const long long *off, int ns, double *out);
+
 }  // namespace g4mi

@@ -326,6 +326,28 @@ __global__ void __launch_bounds__(256) k_to_offsets(const long long *__restrict_
     }
 }
 
+// Particles [lo, lo + n) of one coordinate back from the mixed form: the FP32
+// value alone, plus `add` (plus_add), or plus its slice's base (base set).
+__global__ void __launch_bounds__(256) k_from_offsets(const float *__restrict__ in, long long lo, long long n,
+                                                      int plus_add, double add, const double *__restrict__ base,
+                                                      const long long *__restrict__ off, int ns,
+                                                      double *__restrict__ out) {
+    for (long long k = blockIdx.x * 256LL + threadIdx.x; k < n; k += gridDim.x * 256LL) {
+        const double v = (double)in[lo + k];
+        if (!base) {
+            out[k] = plus_add ? add + v : v;
+            continue;
+        }
+        int a = 0, b = ns;  // the slice: off[a] <= lo + k < off[b]
+        while (b - a > 1) {
+            const int m = (a + b) / 2;
+            if (off[m] <= lo + k) a = m;
+            else b = m;
+        }
+        out[k] = base[a] + v;
+    }
+}
+
 }  // namespace
 
 void launch_quiet_load(hipStream_t s, int ns, const long long *off, const unsigned int *starts,
@@ -356,6 +378,14 @@ void launch_to_offsets(hipStream_t s, int ns, const long long *off, long long n,
     const unsigned gx = (unsigned)std::max(1, std::min(64, (maxpart + 255) / 256));
     hipLaunchKernelGGL(k_to_offsets, dim3(gx, (unsigned)ns), dim3(256), 0, s, off, ns, n, base, gref, g, th, x, y,
                        px, py, fg, ft, fx, fy, fpx, fpy);
+}
+
+void launch_from_offsets(hipStream_t s, const float *in, long long lo, long long n, bool plus_add, double add,
+                         const double *base, const long long *off, int ns, double *out) {
+    if (n <= 0) return;
+    const unsigned gx = (unsigned)std::min<long long>((n + 255) / 256, 16384);
+    hipLaunchKernelGGL(k_from_offsets, dim3(gx), dim3(256), 0, s, in, lo, n, plus_add ? 1 : 0, add, base, off, ns,
+                       out);
 }
 
 }  // namespace g4mi
