@@ -37,7 +37,9 @@ struct AdiPlan {
     int tile = 0;     // 8 or 16: window of the fused recurrence kernel; 0: not eligible
     int band_m = 0;   // 7, 8, 12 or 16: half width of the banded-inverse kernel; 0: not eligible
     int klo = 0, khi = -1;  // rows sharing the central band row
-    double2 *fac = nullptr, *band = nullptr;  // one allocation: c | cbet | cwet, then the band
+    double2 *fac = nullptr, *band = nullptr;  // one allocation: c | cbet | cwet, the band, strip_k's tables
+    int strip = -1;                           // the strip kernel's form; -1: none holds the step size
+    StripCoef strip_k{};
 };
 // The spectral solver's tables for one step size: the convolution's kernel
 // transform and, once a GEMM needs it, the propagator matrix.
@@ -113,11 +115,11 @@ struct Ctx {
     // field diagnostics sums written by the fused ADI of the last field
     // step, and the storage slices slippage has zeroed since then
     bool field_diag_fresh = false;
-    bool tiles_fresh = false;          // they are still per tile, in d_tilediag
+    int ntiles = 0;                    // they are still per tile or strip in d_tilediag, this many a slice
     std::vector<int> zeroed_since_adi;
     // ADI kernel chosen by the autotuner (-1: not tuned yet) and its timings:
     // 0 two-kernel Thomas, 1 fused recurrence, 2 fused recurrence with
-    // prefetch, 3 banded inverse
+    // prefetch, 3 banded inverse, 4 column strips
     int adi_kernel = -1;
     bool adi_fixed = false;               // set by g4mi_set_schedule("adi_kernel", k >= 0)
     std::map<double, int> adi_choice;     // the tuner's kernel per step size
@@ -362,6 +364,33 @@ static int plans_room(Ctx *c, PlanCache<Plan> &pc, size_t bytes) {
     return G4MI_OK;
 }
 
+// The strip kernel's form and x factors for Im(cstep) = a: the first form
+// whose convolution and back substitution leave out less than `bar` of the
+// diagonal; -1 if none does.
+static int strip_coef(double a, double bar, StripCoef *k) {
+    const AdiRoot r = adi_root(a);
+    int form = 0;
+    while (form < kStripForms && !((double)std::pow(std::abs(r.w), strip_dims(form).reach()) < bar)) form++;
+    if (form == kStripForms) return -1;
+    typedef std::complex<long double> cld;
+    auto d2 = [](cld v) { return make_double2((double)v.real(), (double)v.imag()); };
+    const StripDims d = strip_dims(form);
+    k->a = a;
+    // sum_{n < B} w^n S^n and its mirror image together: distance m gets w^m sum_{n < B - m} w^2n
+    for (int m = 0; m < d.B; m++) {
+        cld t = 0;
+        for (int n = d.B - m; n-- > 0;) t = 1.0L + r.w * r.w * t;
+        k->e[m] = d2(r.g * (1.0L - r.w * r.w) * std::pow(r.w, m) * t);
+    }
+    cld wj = std::pow(r.w, d.B);
+    for (int l = 0; l < d.L; l++, wj *= wj) {
+        k->c[l] = d2(1.0L + wj * wj);
+        k->s[l] = d2(wj);
+    }
+    k->x = d2(r.g * wj);  // at B 2^L
+    return form;
+}
+
 // FieldSolverADI::init for one grid and step size, kept in `pc`.
 static int adi_plan(Ctx *c, PlanCache<AdiPlan> &pc, int ng, double dgrid, double xks, double delz, AdiPlan *out) {
     if (const AdiPlan *have = pc.find(delz)) {
@@ -409,6 +438,13 @@ static int adi_plan(Ctx *c, PlanCache<AdiPlan> &pc, int ng, double dgrid, double
         h.insert(h.end(), band.begin(), band.end());
         break;
     }
+    const size_t tables = h.size();
+    p.strip = strip_coef(p.cstep, tiny, &p.strip_k);
+    if (p.strip >= 0) {  // cbet, then -cwet with the zeros that end the back substitution
+        for (int i = 0; i < 2 * ng; i++) h.push_back(h[2 * ng + i]);
+        for (int i = 0; i < 2 * ng; i++) h.push_back(-h[4 * ng + i]);
+        h.insert(h.end(), 2 * kStripPad, 0.0);
+    }
     G4_TRY(plans_room(c, pc, h.size() * sizeof(double)));
     G4_HIP(hipMalloc(&p.fac, h.size() * sizeof(double)));
     if (hipMemcpy(p.fac, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
@@ -417,9 +453,18 @@ static int adi_plan(Ctx *c, PlanCache<AdiPlan> &pc, int ng, double dgrid, double
         return G4MI_E_HIP;
     }
     p.band = p.band_m ? p.fac + 3 * (size_t)ng : nullptr;
+    p.strip_k.cbet = p.fac + tables / 2;
+    p.strip_k.ncwet = p.strip_k.cbet + ng;
     pc.plans.emplace_back(delz, p);
     *out = p;
     return G4MI_OK;
+}
+
+// The most blocks of field sums that any ADI kernel writes per slice.
+static int adi_sum_blocks(int ng) {
+    int n = adi_band_tiles(ng);
+    for (int f = 0; f < kStripForms; f++) n = std::max(n, strip_dims(f).count(ng));
+    return n;
 }
 
 static int ensure_factors(Ctx *c, double delz) {
@@ -427,8 +472,8 @@ static int ensure_factors(Ctx *c, double delz) {
     c->adi_delz = std::nan("");  // until the new plan is there
     G4_TRY(adi_plan(c, c->adi_plans, c->ng, c->dgrid, c->xks, delz, &c->adi));
     c->adi_delz = delz;
-    if (c->adi.band_m && !c->d_tilediag)
-        G4_HIP(hipMalloc(&c->d_tilediag, (size_t)c->ns * adi_band_tiles(c->ng) * 8 * sizeof(double)));
+    if ((c->adi.band_m || c->adi.strip >= 0) && !c->d_tilediag)
+        G4_HIP(hipMalloc(&c->d_tilediag, (size_t)c->ns * adi_sum_blocks(c->ng) * 8 * sizeof(double)));
     if (!c->adi_fixed) {
         // the tuner's choice for this step size, or tune it at the next field step
         auto it = c->adi_choice.find(delz);
@@ -437,7 +482,7 @@ static int ensure_factors(Ctx *c, double delz) {
         if (!c->adi.tile) c->adi_kernel = -1;      // re-tune if no longer eligible
     } else if (c->adi_kernel == 3 && !c->adi.band_m) {
         c->adi_kernel = -1;
-    } else if (c->adi_kernel == 4 && !adi_wide64_ok(c->ng, c->adi.band_m, c->adi.klo, c->adi.khi)) {
+    } else if (c->adi_kernel == 4 && c->adi.strip < 0) {
         c->adi_kernel = -1;
     }
     return G4MI_OK;
@@ -585,7 +630,7 @@ struct AdiField {
 static bool adi_eligible(const AdiField &a, int kind) {
     if (kind == 1 || kind == 2) return a.p->tile != 0 && a.diag;
     if (kind == 3) return a.p->band_m != 0;
-    if (kind == 4) return adi_wide64_ok(a.ng, a.p->band_m, a.p->klo, a.p->khi);
+    if (kind == 4) return a.p->strip >= 0;
     return kind == 0;
 }
 
@@ -595,8 +640,7 @@ static void adi_launch(Ctx *c, int kind, const AdiField &a, double2 *fin, double
     const AdiPlan &p = *a.p;
     const AdiFactors f{p.fac, p.fac + a.ng, p.fac + 2 * a.ng, p.cstep, a.ng};
     if (kind == 4)
-        (void)launch_adi_wide64(c->stream, c->ns, fin, fout, a.src, a.box, p.band, p.cstep, a.ng, c->first,
-                                p.band_m, p.klo, p.khi, a.diag);
+        launch_adi_strip(c->stream, c->ns, fin, fout, a.src, a.box, p.strip_k, p.strip, a.ng, c->first, a.tilediag);
     else if (kind == 3)
         launch_adi_band(c->stream, c->ns, fin, fout, a.src, a.box, p.band, p.cstep, a.ng, c->first, p.band_m,
                         p.klo, p.khi, a.tilediag, nullptr);
@@ -960,7 +1004,7 @@ static int field_track(Ctx *c, const g4mi_step_params &st, double delz, bool dep
         c->adi_choice[c->adi_delz] = c->adi_kernel;
     }
     adi_launch(c, c->adi_kernel, a, c->d_field, c->d_work);
-    c->tiles_fresh = c->adi_kernel == 3;
+    c->ntiles = c->adi_kernel == 3 ? adi_band_tiles(c->ng) : c->adi_kernel == 4 ? strip_dims(c->adi.strip).count(c->ng) : 0;
     if (c->adi_kernel >= 3) std::swap(c->d_field, c->d_work);  // result is in the other buffer
     c->field_diag_fresh = c->adi_kernel != 0;
     c->zeroed_since_adi.clear();
@@ -1307,9 +1351,9 @@ static int diag(Ctx *c, g4mi_diag_out *o) {
     // the fused ADI already summed the field of this step; otherwise sum now
     if (!c->field_diag_fresh) {
         launch_diag_field(c->stream, ns, c->d_field, ng, c->d_diag_f);
-    } else if (c->tiles_fresh) {
-        launch_tile_sums(c->stream, ns, c->d_tilediag, ng, c->d_diag_f);
-        c->tiles_fresh = false;
+    } else if (c->ntiles) {
+        launch_tile_sums(c->stream, ns, c->d_tilediag, c->ntiles, c->d_diag_f);
+        c->ntiles = 0;
     }
     std::vector<double> hb(8 * (size_t)ns), hf(8 * (size_t)ns);
     G4_HIP(hipMemcpyAsync(hb.data(), c->d_diag_b, hb.size() * 8, hipMemcpyDeviceToHost, c->stream));
@@ -3163,9 +3207,9 @@ static int enqueue_record(Ctx *c, const g4mi_diag_out *o) {
     r.field = c->d_diag_f;
     if (!c->field_diag_fresh) {
         launch_diag_field(c->stream, c->ns, c->d_field, c->ng, c->d_diag_f);
-    } else if (c->tiles_fresh) {
+    } else if (c->ntiles) {
         r.tiles = c->d_tilediag;
-        r.ntiles = adi_band_tiles(c->ng);
+        r.ntiles = c->ntiles;
     }
     std::vector<double> wake;
     if (wants_aux(o)) {

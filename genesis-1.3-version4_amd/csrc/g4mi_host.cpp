@@ -152,6 +152,15 @@ double adi_factors(int ngrid, double delz, double dgrid, double xks, double *c, 
     return rtmp;
 }
 
+AdiRoot adi_root(double a) {
+    // -i a (w^2 + 1) + (1 + 2 i a) w = 0 has roots w and 1/w; with q = 1 + 2 i a,
+    // p = 2 i a the one inside is p / (q + sqrt(q^2 - p^2)) (no cancellation)
+    typedef std::complex<long double> cld;
+    const cld p(0, 2 * (long double)a), q = 1.0L + p;
+    const cld r = std::sqrt(q * q - p * p);
+    return {p / (q + r), 1.0L / r};
+}
+
 AdiInverse::AdiInverse(int ngrid, const double *c, const double *cbet, const double *cwet)
     : n_(ngrid), inv_((size_t)ngrid * ngrid), rel_(ngrid, 0.0) {
     typedef std::complex<double> cd;

@@ -45,6 +45,13 @@ class AdiInverse {
     std::vector<double> rel_;                // largest relative entry q columns off the diagonal
 };
 
+// The same inverse's Toeplitz interior: (A^-1)[k][k+m] = g w^|m| for a system
+// without edges; a = Im(cstep).
+struct AdiRoot {
+    std::complex<long double> w, g;
+};
+AdiRoot adi_root(double a);
+
 // Spectral solver matrices (FieldSolverFFT, src/Core/FieldSolverFFT.cpp),
 // interleaved complex, row-major n x n.
 // The step's propagator: M[j][l] = m[(j - l) mod n] with

@@ -1,6 +1,7 @@
 // Launchers of the FP64 device kernels (defined in g4mi_kernels.hip).
 #pragma once
 
+#include "g4mi_adi_strip.h"
 #include "g4mi_common.h"
 
 namespace g4mi {
@@ -109,19 +110,14 @@ int launch_adi_fused(hipStream_t s, int ns, double2 *field, double2 *work, const
 // 2^-60.  tilediag: scratch [ns][adi_band_tiles(ngrid)][8], or null: no
 // field sums; diag null: the tiles' sums are left for launch_tile_sums.
 int adi_band_tiles(int ng);
-void launch_tile_sums(hipStream_t s, int ns, const double *tilediag, int ng, double *diag);
+void launch_tile_sums(hipStream_t s, int ns, const double *tilediag, int ntiles, double *diag);
 int launch_adi_band(hipStream_t s, int ns, const double2 *fin, double2 *fout, const double2 *src,
                     const int4 *box, const double2 *band, double a, int ng, int first, int m,
                     int klo, int khi, double *tilediag, double *diag);
-// The banded operator as a whole-width stream (one workgroup per slice, one
-// lane per column; the products of launch_adi_band as four partial sums,
-// diagnostics straight into diag[8 ns], none where it is null).  Eligible for band half widths 7 and 8, grids up to 512
-// columns whose rows [klo, khi] share the central band except in the first
-// and last 32 columns; returns -1 otherwise.
-bool adi_wide64_ok(int ng, int m, int klo, int khi);
-int launch_adi_wide64(hipStream_t s, int ns, const double2 *fin, double2 *fout, const double2 *src,
-                      const int4 *box, const double2 *band, double a, int ng, int first, int m, int klo, int khi,
-                      double *diag);
+// Both half steps in strips of columns, one wavefront each (any grid):
+// tilediag [ns][strip_dims(form).count(ng)][8] or null.
+void launch_adi_strip(hipStream_t s, int ns, const double2 *fin, double2 *fout, const double2 *src, const int4 *box,
+                      const StripCoef &k, int form, int ng, int first, double *tilediag);
 void launch_zero(hipStream_t s, double2 *p, long long n);
 // A record's slot (device address of pinned memory): beam sums [8 ns] from
 // part (per block of the slices' blk_first ranges) or beam, or left alone;

@@ -59,3 +59,36 @@ def test_harmonic_field_in_each_adi_kernel(kernel, ngrid):
     print(f"  harmonic {ngrid}^2, kernel {kernel}: {e:.2e}", flush=True)
     assert e < 4e-13  # four steps of the single step's 1e-13 bar
     ctx.close()
+
+
+@pytest.mark.parametrize("delz", [0.004, 0.03, 0.1, 0.24, 0.4])
+@pytest.mark.parametrize("ngrid", [3, 5, 16, 17, 18, 26, 33, 34, 35, 42, 49, 50, 51, 63, 64, 100, 101, 130, 255, 300])
+def test_column_strips(ngrid, delz):
+    """The strip kernel (adi_kernel 4) at grids narrower than its halo, at the
+    edges of its strips (50 to 26 columns) and blocks of 8 rows, with the
+    source's footprint anywhere in the grid (and none), for one step size per
+    form (8, 9, 12, 16 and 20 terms), against the oracle: two steps of the
+    single step's 1e-13 bar."""
+    gridmax = 0.5e-3 * (ngrid - 1) / 150  # the cell of 151 columns on 1 mm
+    sim = H.make_state([256, 512, 0, 1024, 256], ngrid=ngrid, gridmax=gridmax, timerun=False)
+    rng = np.random.default_rng(ngrid)
+    sim.x += gridmax * 0.9 * np.repeat([0, -1, 0, 1, 0], [256, 512, 0, 1024, 256])
+    sim.y += gridmax * 0.9 * np.repeat([0, 1, 0, -1, -1], [256, 512, 0, 1024, 256])
+    sim.theta += 0.3 * np.sin(sim.theta)
+    sim.field[:] = rng.normal(size=sim.field.shape) * 1e9
+    ctx = H.to_gpu(sim)
+    ctx.set_schedule("adi_kernel", 4)
+    st = H.steps(1, 2)
+    one = H.gsteps(st)[0]
+    for _ in range(2):
+        ctx.field_track(one, delz)
+        H.oracle_call("orc_field_advance", sim, C.byref(st[0]), C.c_double(delz))
+    assert ctx.schedule()["adi"] == "band-wide"
+    f, _ = ctx.download_field()
+    err = np.max(np.abs(f - sim.field)) / np.max(np.abs(sim.field))
+    d = ctx.diag()
+    w = (sim.field ** 2).sum(axis=2).sum(axis=1)
+    print(f"  {ngrid}^2, delz {delz}: {err:.2e}", flush=True)
+    assert err < 2e-13
+    assert np.max(np.abs(d["power"] / d["power"].sum() - w / w.sum())) < 1e-12
+    ctx.close()
