@@ -650,27 +650,42 @@ static void adi_launch(Ctx *c, int kind, const AdiField &a, double2 *fin, double
         launch_adi(c->stream, c->ns, fin, fout, a.src, a.box, f, c->first);
 }
 
-// Autotuner of the ADI: run each eligible kernel on a scratch copy of the
-// current field (same sources and boxes) and return the fastest.  Runs
-// before a field's first step of each step size; ms[5] receives the timings.
-static int tune_adi(Ctx *c, const AdiField &a, const double2 *field, double2 *work, int *choice, float *ms) {
+// Autotuner of the ADI, before a field's first step of each step size; ms[5]
+// receives the timings, -1 for kernels not run.  Where the banded inverse or
+// the strips hold the step size, only these two are run: they always beat the
+// others (ms a launch, strips | band | recurrence | recurrence with prefetch |
+// Thomas, - not eligible: 509 slices of 255^2, 0.08 m 0.36 | 1.45 | 1.30 |
+// 0.79 | 2.7; 97 of 151^2 0.095 | 0.066 | 0.240 | 0.185 | 0.31; one of 255^2
+// 0.17 | 0.032 | - | - | 0.40), and they leave their input alone, so they run
+// on the field itself.  Few slices want the band's many tiles, many the strips'
+// fewer operations, and where they cross depends on the step size, so both are
+// timed.  A single candidate is taken as it is.
+static int tune_adi(Ctx *c, const AdiField &a, double2 *field, double2 *work, int *choice, float *ms) {
+    const bool out = adi_eligible(a, 3) || adi_eligible(a, 4);
+    std::vector<int> kinds;
+    for (int kind = 0; kind < 5; kind++) {
+        ms[kind] = -1.f;
+        if (adi_eligible(a, kind) && (kind >= 3) == out) kinds.push_back(kind);
+    }
+    *choice = kinds[0];
+    if (kinds.size() == 1) return G4MI_OK;
     const size_t bytes = (size_t)c->ns * a.ng * a.ng * sizeof(double2);
     double2 *scratch = nullptr;
-    G4_HIP(hipMalloc(&scratch, bytes));
+    if (!out) {
+        G4_HIP(hipMalloc(&scratch, bytes));
+        G4_HIP(hipMemcpyAsync(scratch, field, bytes, hipMemcpyDeviceToDevice, c->stream));
+    }
+    double2 *const fin = out ? field : scratch;
     hipEvent_t e0, e1;
     G4_HIP(hipEventCreate(&e0));
     G4_HIP(hipEventCreate(&e1));
-    G4_HIP(hipMemcpyAsync(scratch, field, bytes, hipMemcpyDeviceToDevice, c->stream));
-    int best_kind = 0;
     float best_ms = 1e30f;
-    for (int kind = 0; kind < 5; kind++) {
-        ms[kind] = -1.f;
-        if (!adi_eligible(a, kind)) continue;
-        adi_launch(c, kind, a, scratch, work);  // warm-up
+    for (int kind : kinds) {
+        adi_launch(c, kind, a, fin, work);  // warm-up
         float best = 1e30f;
         for (int rep = 0; rep < 3; rep++) {
             G4_HIP(hipEventRecord(e0, c->stream));
-            adi_launch(c, kind, a, scratch, work);
+            adi_launch(c, kind, a, fin, work);
             G4_HIP(hipEventRecord(e1, c->stream));
             G4_HIP(hipEventSynchronize(e1));
             float t = 0;
@@ -680,14 +695,13 @@ static int tune_adi(Ctx *c, const AdiField &a, const double2 *field, double2 *wo
         ms[kind] = best;
         if (best < best_ms) {
             best_ms = best;
-            best_kind = kind;
+            *choice = kind;
         }
     }
     G4_HIP(hipGetLastError());
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    G4_HIP(hipFree(scratch));
-    *choice = best_kind;
+    if (scratch) G4_HIP(hipFree(scratch));
     return G4MI_OK;
 }
 

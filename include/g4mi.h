@@ -237,10 +237,11 @@ int g4mi_sort_index(g4mi_ctx *ctx, double slen, int *atar, long long *moved);
  * share that scratch and race. */
 int g4mi_sort_index_noalloc(g4mi_ctx *ctx, double slen, int *atar, long long *moved);
 
-/* Kernel schedule.  The first field step of each step size times every
- * ADI kernel eligible for its grid and step (two-kernel Thomas, fused
- * recurrence with and without prefetch, banded inverse in 32x32 tiles and
- * in strips of whole columns) on a scratch copy of its field and keeps the
+/* Kernel schedule.  The first field step of each step size times the ADI
+ * kernels that can be the fastest for its grid and step (banded inverse in
+ * 32x32 tiles and in strips of whole columns where they hold the step size;
+ * fused recurrence with and without prefetch and two-kernel Thomas
+ * otherwise) on its field or a scratch copy of it and keeps the
  * fastest for that step size (the library's autotuner).  g4mi_set_schedule
  * fixes an entry instead ("adi_kernel": 0..4, -1 re-enables tuning; a
  * kernel not eligible for a step size falls back to the tuner's choice);
