@@ -172,7 +172,7 @@ def roofline(cfg, kt, ntot, precision=g4mi.FP64, schedule=None):
     gbs = per[name] / (ms * 1e-3) / 1e9
     dev = KERNEL_OF["fp64_fused" if fused else precision].get(name)
     if name == "adi" and precision == g4mi.FP32 and schedule:
-        dev = {"band32-wide": "k_mix_adi_wide", "band32-stream": "k_mix_adi_stream",
+        dev = {"band32-wide": "k_mix_adi_strip", "band32-stream": "k_mix_adi_stream",
                "band32-tile": "k_mix_adi<"}.get(schedule.get("adi"), dev)
     if name == "adi" and precision == g4mi.FP64 and schedule:
         # the ADI kernel the tuner chose for the undulator step (the timed steps)

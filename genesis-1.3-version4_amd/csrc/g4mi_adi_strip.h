@@ -8,10 +8,10 @@
 // those, cut off at m < B 2^L, into (1 + .. + w^(B-1) S^(B-1)) (1 + w^B S^B)
 // (1 + w^2B S^2B)...; the two sides of one binary factor together are
 // (1 + w^2j) + w^j (S^j + S^-j), one complex product for the cell and one for
-// the sum of its two neighbours j away.  B = 2, L = 2 reaches m = 7 with 30
-// operations a cell (36 with a single term at 8, X) where the band of the
-// inverse takes 8 to 9 products of the neighbours' sums (46 to 52), and 6 to 8
-// LDS accesses for 17; B = 5, L = 2 reaches m = 19 with 48.  At the edges the
+// the sum of its two neighbours j away.  B = 3, L = 1 reaches m = 5 with 26
+// operations a cell (32 with a single term at 6, X), B = 2, L = 2 m = 7 with
+// 30, where the band of the inverse takes 7 to 9 products of the neighbours'
+// sums (42 to 52); B = 5, L = 2 reaches m = 19 with 48.  At the edges the
 // system is the same convolution of the right-hand side continued oddly about
 // the cells -1 and ng (where the solution is zero), so every lane runs the same
 // code: its column is a mirror image with a sign outside the grid.
@@ -22,14 +22,24 @@
 // w^(8 NB + 1).  14 operations a cell (NB = 1) for the band's 46.
 //
 // A wavefront owns U columns and H on each side that its neighbours own too;
-// it shares nothing with other wavefronts, so there is no barrier.
-// Neighbours 1 away come by a wavefront shift, the others through LDS, which
-// serves a wavefront's accesses in order.  Up to 9 terms it is bound by HBM:
-// 1024 slices of 151^2 in FP64 202 us, 3.7 TB/s of one read and one write of
-// the field (the whole-width band product it replaces: 438 us); 509 of 255^2
-// 331 us (458).  Beyond, by the halo's share of the columns (26 of 64 are its
-// own with 20 terms): 363 us with 16 terms (the window recurrence 785), 554
-// with 20 (band product of 33 terms 1446, Thomas' two sweeps 2713).
+// it shares nothing with other wavefronts, so there is no barrier.  Neighbours
+// come through LDS, which serves a wavefront's accesses in order (those 1 away
+// by a wavefront shift where the right-hand side is not in LDS anyway).  The
+// number of terms also sets the number of strips: 255 columns are 5 strips of
+// 52 with 7 terms, 6 of 50 with 8.
+//
+// us a launch (floor: one read and one write of the field), and what it replaces:
+//   FP64  1024 slices of 151^2,  7 terms  164 (159)   whole-width band product 438
+//          509 slices of 255^2,  9 terms  263 (225)   the same 458
+//                               16 terms  354         window recurrence 785
+//                               20 terms  476         band of 33 terms 1446, Thomas 2713
+//   FP32  1024 slices of 151^2,  6 terms  114  (79)   FP32 band product with correction 198
+//         4096 slices of 255^2,  7 terms 1171 (903)   the same 1697
+//                               12 terms 1853         the same 2243
+//                               16 terms 1968         the same 3243
+// Up to 9 terms FP64 is bound by HBM; FP32 and the rest by FP64 arithmetic
+// (86 to 100 vector instructions a cell, 3 wavefronts per SIMD) and the halo's
+// share of the columns.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -54,16 +64,20 @@ struct StripGeom {
 };
 
 // The forms of the kernel, from the cheapest to the farthest reaching.
-constexpr int kStripForms = 5;
+constexpr int kStripForms = 8;  // 6, 7, 8, 9, 12, 16, 20, 24 terms
+template <int N>
+using StripInt = std::integral_constant<int, N>;
 template <class F>
 inline void strip_form(int form, F f) {
-    using std::integral_constant;
     switch (form) {
-    case 0: f(integral_constant<int, 2>{}, integral_constant<int, 2>{}, integral_constant<int, 0>{}, integral_constant<int, 1>{}); break;
-    case 1: f(integral_constant<int, 2>{}, integral_constant<int, 2>{}, integral_constant<int, 1>{}, integral_constant<int, 1>{}); break;
-    case 2: f(integral_constant<int, 3>{}, integral_constant<int, 2>{}, integral_constant<int, 0>{}, integral_constant<int, 2>{}); break;
-    case 3: f(integral_constant<int, 2>{}, integral_constant<int, 3>{}, integral_constant<int, 0>{}, integral_constant<int, 2>{}); break;
-    default: f(integral_constant<int, 5>{}, integral_constant<int, 2>{}, integral_constant<int, 0>{}, integral_constant<int, 3>{}); break;
+    case 0: f(StripInt<3>{}, StripInt<1>{}, StripInt<0>{}, StripInt<1>{}); break;
+    case 1: f(StripInt<3>{}, StripInt<1>{}, StripInt<1>{}, StripInt<1>{}); break;
+    case 2: f(StripInt<2>{}, StripInt<2>{}, StripInt<0>{}, StripInt<1>{}); break;
+    case 3: f(StripInt<2>{}, StripInt<2>{}, StripInt<1>{}, StripInt<1>{}); break;
+    case 4: f(StripInt<3>{}, StripInt<2>{}, StripInt<0>{}, StripInt<2>{}); break;
+    case 5: f(StripInt<2>{}, StripInt<3>{}, StripInt<0>{}, StripInt<2>{}); break;
+    case 6: f(StripInt<5>{}, StripInt<2>{}, StripInt<0>{}, StripInt<3>{}); break;
+    default: f(StripInt<3>{}, StripInt<3>{}, StripInt<0>{}, StripInt<3>{}); break;
     }
 }
 struct StripDims {
@@ -79,6 +93,16 @@ inline StripDims strip_dims(int form) {
     return d;
 }
 
+// Blocks of four wavefronts, one per SIMD: the strips of a slice in one block
+// (6 wavefronts at 255^2) leave room for only one block on a CU, 1.5
+// wavefronts per SIMD of the registers' 3.  Workgroups go to the 8 XCDs in
+// turn, so each XCD takes a run of strips: neighbours share their halo in its L2.
+constexpr int kStripWaves = 4;
+inline unsigned strip_blocks(int ns, int nstrip) {
+    const long long nb = ((long long)ns * nstrip + kStripWaves - 1) / kStripWaves;
+    return (unsigned)((nb + 7) / 8 * 8);
+}
+
 // Coefficients of a step size: the x convolution's first factor at distances
 // 0 .. 4, its binary factors (cell and neighbours), the single term, and the y
 // elimination's tables (device): cbet[ng] and -cwet[ng + kStripPad] (zero from
@@ -92,10 +116,15 @@ struct StripCoef {
 
 namespace strip {
 
+// this wavefront's strip of all slices' (may lie past the last)
+__device__ __forceinline__ long long item() {
+    const long long b = (long long)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    return b * kStripWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+}
 template <int CTRL>
 __device__ __forceinline__ double shift1(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
     return __hiloint2double(hi, lo);
 }
 // the sum of both neighbours one lane away (0 beyond the wavefront)
@@ -121,6 +150,20 @@ __device__ __forceinline__ double2 entry(const double2 *t, int i) {
     typedef const __attribute__((address_space(4))) double *Const;
     Const p = (Const)(unsigned long long)t;
     return make_double2(p[2 * i], p[2 * i + 1]);
+}
+// coefficients kept in device memory, read the same way
+__device__ __forceinline__ StripCoef coef(const StripCoef *d) {
+    static_assert(sizeof(StripCoef) % 8 == 0, "");
+    typedef const __attribute__((address_space(4))) unsigned long long *Const;
+    Const p = (Const)(unsigned long long)d;
+    union U {
+        StripCoef k;
+        unsigned long long w[sizeof(StripCoef) / 8];
+        __device__ U() {}
+    } u;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(StripCoef) / 8); i++) u.w[i] = p[i];
+    return u.k;
 }
 __device__ __forceinline__ double2 wide(double2 v) { return v; }
 __device__ __forceinline__ double2 wide(float2 v) { return make_double2(v.x, v.y); }
@@ -150,12 +193,15 @@ __device__ __forceinline__ void adi_strip(const T2 *__restrict__ u, T2 *__restri
     const bool fixed = t == 0 || t == ng + 1, image = t > ng + 1;
     const int col = fixed ? 0 : image ? per - t - 1 : t - 1;
     const double sign = fixed ? 0.0 : image ? -1.0 : 1.0;
+    const bool edge = __any(sign != 1.0);
     // rows are uniform, so a load is a scalar row address and the lane's column;
     // source rows outside the box load the nearest row inside and drop it
     const bool sin = col >= bx.x && col <= bx.z;
-    const unsigned ucol = (unsigned)col, scol = sin ? (unsigned)col : 0u;
-    auto uload = [&](int r) -> T2 { return (u + (long long)min(r, ng - 1) * ng)[ucol]; };
-    auto sload = [&](int r) -> T2 { return (S + (long long)max(0, min(max(r, bx.y), bx.w)) * ng)[scol]; };
+    const unsigned ucol = (unsigned)(col * sizeof(T2)), scol = sin ? ucol : 0u, ocol = (unsigned)(x * (int)sizeof(T2));
+    auto uload = [&](int r) -> T2 { return *(const T2 *)((const char *)(u + (long long)min(r, ng - 1) * ng) + ucol); };
+    auto sload = [&](int r) -> T2 {
+        return *(const T2 *)((const char *)(S + (long long)max(0, min(max(r, bx.y), bx.w)) * ng) + scol);
+    };
     auto inbox = [&](int r) -> bool { return sin && r >= bx.y && r <= bx.w; };
     double2 *const erow = lds + H + lane;  // the right-hand side, then each factor's input
     double2 *row[L];
@@ -171,6 +217,7 @@ __device__ __forceinline__ void adi_strip(const T2 *__restrict__ u, T2 *__restri
     for (int j = 0; j < RING; j++) Y[j] = z2;
     double s_w = 0, s_yw = 0, s_yyw = 0, s_re = 0, s_im = 0, s_cen = 0;
     const double shift = -0.5 * (double)(ng - 1);
+    double dy = shift;  // of the next row completed
     // eight rows of the elimination, then the back substitution that completes
     // the eight rows above them.  FULL: the rows and
     // the two below them exist.
@@ -182,18 +229,23 @@ __device__ __forceinline__ void adi_strip(const T2 *__restrict__ u, T2 *__restri
             double2 y = z2;
             if (FULL || r < ng) {  // uniform
                 // E = S + u + i a (u(r+1) - 2 u(r) + u(r-1)), zero rows outside
-                double2 s = wide(sv);
-                if (!inbox(r)) s = z2;
+                T2 sb = sv;
+                if (!inbox(r)) sb.x = sb.y = 0;
+                const double2 s = wide(sb);
                 const double dx = __builtin_fma(-2.0, uc.x, un.x) + um.x, dy = __builtin_fma(-2.0, uc.y, un.y) + um.y;
                 double2 E = make_double2(__builtin_fma(-k.a, dy, s.x + uc.x), __builtin_fma(k.a, dx, s.y + uc.y));
-                E.x *= sign;
-                E.y *= sign;
-                double2 v = fma2(k.e[1], beside(E), mul(k.e[0], E)), far = z2;
-                if (G::taps) {
+                if (edge) {  // uniform
+                    E.x *= sign;
+                    E.y *= sign;
+                }
+                double2 v = mul(k.e[0], E), far = z2;
+                if (!G::taps) {
+                    v = fma2(k.e[1], beside(E), v);
+                } else {
                     *erow = E;
                     lds_order();
 #pragma unroll
-                    for (int d = 2; d < B; d++) v = fma2(k.e[d], sum(erow[-d], erow[d]), v);
+                    for (int d = 1; d < B; d++) v = fma2(k.e[d], sum(erow[-d], erow[d]), v);
                     if (X) far = sum(erow[-(B << L)], erow[B << L]);
                 }
 #pragma unroll
@@ -236,11 +288,12 @@ __device__ __forceinline__ void adi_strip(const T2 *__restrict__ u, T2 *__restri
                 for (int j = 0; j < R; j++) {
                     if (FULL || k0 + j < ng) {
                         const double2 o = Y[j];
-                        narrow(o, &(uo + (long long)(k0 + j) * ng)[(unsigned)x]);
-                        const double wei = __builtin_fma(o.x, o.x, o.y * o.y), dy = (double)(k0 + j) + shift;
+                        narrow(o, (T2 *)((char *)(uo + (long long)(k0 + j) * ng) + ocol));
+                        const double wei = __builtin_fma(o.x, o.x, o.y * o.y), yw = dy * wei;
                         s_w += wei;
-                        s_yw = __builtin_fma(dy, wei, s_yw);
-                        s_yyw = __builtin_fma(dy * dy, wei, s_yyw);
+                        s_yw += yw;
+                        s_yyw = __builtin_fma(dy, yw, s_yyw);
+                        dy += 1.0;
                         s_re += o.x;
                         s_im += o.y;
                         if (k0 + j == ng / 2) s_cen = wei;

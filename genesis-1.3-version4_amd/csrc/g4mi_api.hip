@@ -223,6 +223,8 @@ struct Ctx {
     std::vector<MixBand> h_binfo;
     std::map<double, int> band_of_dz;      // step size -> band index
     std::vector<int> band_tmpl;            // template half width of each band
+    std::vector<int> band_form;            // and the strip kernel's form
+    double2 *m_strip = nullptr;            // the strip kernel's tables, kMixMaxBands of 2 ng + kStripPad
     bool m_refine = true;                  // FP64 residual correction in the ADI (schedule "adi_refine")
     bool m_graphs = true;                  // replay captured step graphs
     int m_adi_mode = kAdiWide;             // mixed ADI kernel (schedule "mixed_adi"): tile 0, strips 1, wide 2
@@ -237,7 +239,7 @@ struct Ctx {
     double m_tune_main[8] = {0, 0, 0, 0, 0, 0, 0, 0}, m_tune_adi[3] = {0, 0, 0}, m_tune_graph = -1;
     int m_tune_nmain[8] = {0, 0, 0, 0, 0, 0, 0, 0}, m_tune_nadi[3] = {0, 0, 0};
     hipEvent_t m_tune_ev[9] = {};
-    std::map<std::tuple<int, int, int, int, int, int, int, int, int>, hipGraphExec_t> m_graph;
+    std::map<std::tuple<int, int, int, int, int, int, int, int, int, int>, hipGraphExec_t> m_graph;
     double *m_rec_pin = nullptr;           // pinned host mirror of the record ring
     hipEvent_t m_rec_ev[2] = {nullptr, nullptr};  // copy of each half of the ring done
     std::vector<double> h_cur;             // currents [ns] (host copy)
@@ -439,7 +441,7 @@ static int adi_plan(Ctx *c, PlanCache<AdiPlan> &pc, int ng, double dgrid, double
         break;
     }
     const size_t tables = h.size();
-    p.strip = strip_coef(p.cstep, tiny, &p.strip_k);
+    p.strip = strip_coef(p.cstep, std::ldexp(1.0, -58), &p.strip_k);  // 1/32 of FP64's rounding
     if (p.strip >= 0) {  // cbet, then -cwet with the zeros that end the back substitution
         for (int i = 0; i < 2 * ng; i++) h.push_back(h[2 * ng + i]);
         for (int i = 0; i < 2 * ng; i++) h.push_back(-h[4 * ng + i]);
@@ -654,13 +656,20 @@ static void adi_launch(Ctx *c, int kind, const AdiField &a, double2 *fin, double
 // receives the timings, -1 for kernels not run.  Where the banded inverse or
 // the strips hold the step size, only these two are run: they always beat the
 // others (ms a launch, strips | band | recurrence | recurrence with prefetch |
-// Thomas, - not eligible: 509 slices of 255^2, 0.08 m 0.36 | 1.45 | 1.30 |
+// Thomas, - not eligible: 509 slices of 255^2, 0.08 m 0.35 | 1.45 | 1.30 |
 // 0.79 | 2.7; 97 of 151^2 0.095 | 0.066 | 0.240 | 0.185 | 0.31; one of 255^2
 // 0.17 | 0.032 | - | - | 0.40), and they leave their input alone, so they run
 // on the field itself.  Few slices want the band's many tiles, many the strips'
 // fewer operations, and where they cross depends on the step size, so both are
-// timed.  A single candidate is taken as it is.
+// timed, up to one strip for each of the 1024 SIMDs: from there the strips are
+// taken (0.26 | 0.54 for 509 slices of 255^2, 0.16 | 0.44 for 1024 of 151^2).
+// A single candidate is taken as it is.
 static int tune_adi(Ctx *c, const AdiField &a, double2 *field, double2 *work, int *choice, float *ms) {
+    if (adi_eligible(a, 4) && (long long)c->ns * strip_dims(a.p->strip).count(a.ng) >= 1024) {
+        *choice = 4;
+        std::fill(ms, ms + 5, -1.f);
+        return G4MI_OK;
+    }
     const bool out = adi_eligible(a, 3) || adi_eligible(a, 4);
     std::vector<int> kinds;
     for (int kind = 0; kind < 5; kind++) {
@@ -1822,11 +1831,21 @@ static int mix_band(Ctx *c, double delz, int *band) {
     bi.klo = kc - half;
     bi.khi = kc + half;
     bi.m = need;
+    // the strips leave out less than 2^-47 of the diagonal, as far below FP32's
+    // rounding as that is below 1 (the corrected band product's error too)
+    const int form = strip_coef(rtmp, std::ldexp(1.0, -47), &bi.strip);
+    std::vector<double> st(h.begin() + 2 * (size_t)ng, h.begin() + 4 * (size_t)ng);  // cbet, then -cwet
+    for (int i = 0; i < 2 * ng; i++) st.push_back(-h[4 * (size_t)ng + i]);
+    st.resize(st.size() + 2 * kStripPad, 0.0);
+    bi.strip.cbet = c->m_strip + c->h_binfo.size() * (2 * (size_t)ng + kStripPad);
+    bi.strip.ncwet = bi.strip.cbet + ng;
     for (size_t k = 0; k < bd.size() / 2; k++)
         c->h_bands.push_back(make_float2((float)bd[2 * k], (float)bd[2 * k + 1]));
     const int idx = (int)c->h_binfo.size();
     c->h_binfo.push_back(bi);
     c->band_tmpl.push_back(tm);
+    c->band_form.push_back(form);
+    G4_HIP(hipMemcpyAsync((void *)bi.strip.cbet, st.data(), st.size() * 8, hipMemcpyHostToDevice, c->stream));
     G4_HIP(hipMemcpyAsync(c->m_bands + bi.off, c->h_bands.data() + bi.off, bd.size() / 2 * sizeof(float2),
                           hipMemcpyHostToDevice, c->stream));
     G4_HIP(hipMemcpyAsync(c->m_binfo + idx, &c->h_binfo[idx], sizeof(MixBand), hipMemcpyHostToDevice,
@@ -1896,13 +1915,13 @@ static int mix_fill_step(Ctx *c, const g4mi_step_params &st, double gamma0, MixS
 }
 
 // band, refine, sc, moments, maxzero, ADI kernel (kAdi*), main threads per slice, main LDS region,
-// front kernel launched (0 when the previous step's main kernel ran the front)
-typedef std::tuple<int, int, int, int, int, int, int, int, int> MixKey;
+// front kernel launched (0 when the previous step's main kernel ran the front), the strip kernel's form
+typedef std::tuple<int, int, int, int, int, int, int, int, int, int> MixKey;
 
 static int mix_launch(Ctx *c, const MixKey &k, hipEvent_t *ev) {
     const MixArrays a = mix_arrays(c);
     if (launch_mix_step(c->stream, a, std::get<0>(k), std::get<1>(k) != 0, std::get<2>(k) != 0,
-                        std::get<3>(k) != 0, std::get<4>(k), ev, std::get<5>(k), std::get<6>(k),
+                        std::get<3>(k) != 0, std::get<4>(k), ev, std::get<5>(k), std::get<9>(k), std::get<6>(k),
                         std::get<7>(k), std::get<8>(k) != 0) != 0) {
         set_error("mixed form: no ADI instantiation for this band width");
         return G4MI_E_ARG;
@@ -1964,7 +1983,7 @@ static int mix_step_fno(Ctx *c, const MixKey &k) {
     if (c->fno_mode == 1) {
         launch_mix_beam(c->stream, a, sc, moments, nullptr, false, std::get<6>(k), std::get<7>(k),
                         std::get<8>(k) != 0);
-        if (launch_mix_adi(c->stream, a, tm, refine, adi_mode, &ntiles)) {
+        if (launch_mix_adi(c->stream, a, tm, refine, adi_mode, std::get<9>(k), &ntiles)) {
             set_error("mixed form: no ADI instantiation for this band width");
             return G4MI_E_ARG;
         }
@@ -1994,7 +2013,7 @@ static int mix_step_fno(Ctx *c, const MixKey &k) {
             c->fno_adi_steps++;
             launch_mix_beam(c->stream, a, sc, moments, nullptr, false, std::get<6>(k), std::get<7>(k),
                         std::get<8>(k) != 0);
-            if (launch_mix_adi(c->stream, a, tm, refine, adi_mode, &ntiles)) {
+            if (launch_mix_adi(c->stream, a, tm, refine, adi_mode, std::get<9>(k), &ntiles)) {
                 set_error("mixed form: no ADI instantiation for this band width");
                 return G4MI_E_ARG;
             }
@@ -2058,7 +2077,7 @@ static int mix_step_fno(Ctx *c, const MixKey &k) {
             G4_HIP(hipMemcpyAsync(c->m_judge, c->m_field[hs.cur ^ 1], (size_t)ns * P * sizeof(float2),
                                   hipMemcpyDeviceToDevice, c->stream));
         }
-        if (launch_mix_adi(c->stream, a, tm, refine, adi_mode, &ntiles)) {
+        if (launch_mix_adi(c->stream, a, tm, refine, adi_mode, std::get<9>(k), &ntiles)) {
             set_error("mixed form: no ADI instantiation for this band width");
             return G4MI_E_ARG;
         }
@@ -2102,7 +2121,7 @@ static int mix_step_fno(Ctx *c, const MixKey &k) {
 
 // One step of the mixed-form schedule tuner (see mix_run): tuning step k
 // runs main candidate k % 8 with ADI candidate (k / 8 + k) % 3 (k < 16: the
-// whole-width streaming kernel, the strips, the tiles), the graph of the
+// column strips, the FP32 band's strips, the tiles), the graph of the
 // chosen kernels (k = 16) or the persistent launch (k = 17).  The main
 // candidates: 6, 4 or 8 wavefronts per slice with 68 or 44 KiB of LDS, and
 // 4 or 6 wavefronts with 32 KiB (more workgroups per CU, a smaller
@@ -2111,6 +2130,11 @@ constexpr int kMixTuneSteps = 18;
 constexpr int kMainCands = 8;
 static const int kMainCand[kMainCands][2] = {{384, 0}, {256, 0}, {512, 0}, {384, 1},
                                               {256, 1}, {512, 1}, {256, 2}, {384, 2}};
+
+// A wavefront per strip on each of the 1024 SIMDs: the column strips are then
+// the fastest ADI by far (ms a launch, column strips | FP32 band strips |
+// tiles: 4096 slices of 255^2 1.2 | 2.27 | 9.9) and the others are not tried.
+static bool mix_strips_only(const Ctx *c) { return (long long)c->ns * ((c->ng + 63) / 64) >= 1024; }
 
 static int mix_tune_step(Ctx *c, const MixKey &key) {
     hipEvent_t *tev = c->m_tune_ev;
@@ -2121,7 +2145,7 @@ static int mix_tune_step(Ctx *c, const MixKey &key) {
     float ms = 0;
     if (k < 2 * kMainCands) {
         // every main candidate twice, each ADI kernel four to six times
-        const int mc = k % kMainCands, ac = (k / kMainCands + k) % 3;
+        const int mc = k % kMainCands, ac = mix_strips_only(c) ? 0 : (k / kMainCands + k) % 3;
         const int tm = std::get<0>(kk);
         const bool tile_ok = !c->m_refine || tm <= 9;
         const int mode = ac == 0 ? kAdiWide : ac == 1 ? kAdiStrips : (tile_ok ? kAdiTile : kAdiWide);
@@ -2239,7 +2263,7 @@ static int mix_run(Ctx *c, const g4mi_step_params *steps, int nsteps, double gam
         // the tile kernel's correction needs more LDS than a CU has beyond a half width of 9
         const int refine = (c->m_refine && (c->m_adi_mode != kAdiTile || tm <= 9)) ? 1 : 0;
         keys[i] = MixKey(tm, refine, sc ? 1 : 0, moments ? 1 : 0, maxzero, c->m_adi_mode, c->m_main_nt,
-                         c->m_main_lds, 1);
+                         c->m_main_lds, 1, c->band_form[tab[i].band]);
     }
     // the main kernel of every step but the run's last also runs the next
     // step's front, while its slice's particles are fresh in the caches; the
@@ -2519,6 +2543,7 @@ static int mix_alloc(Ctx *c) {
         (rc = dalloc(c, &c->m_rec, (size_t)kMixRecRows * ns * kMixRecord)) ||
         (rc = dalloc(c, &c->m_st, 1)) ||
         (rc = dalloc(c, &c->m_bands, (size_t)kMixMaxBands * c->ng * kMixBandRowMax)) ||
+        (rc = dalloc(c, &c->m_strip, (size_t)kMixMaxBands * (2 * (size_t)c->ng + kStripPad))) ||
         (rc = dalloc(c, &c->m_binfo, (size_t)kMixMaxBands)))
         return rc;
     c->m_nrec = kMixRecRows;

@@ -2123,11 +2123,11 @@ __global__ void __launch_bounds__(64) k_adi_tile_diag(const double *__restrict__
 
 // ---------------------------------------------------------------------------
 // K5+K6 in strips (g4mi_adi_strip.h): one wavefront per strip, the field sums
-// of each strip to tilediag[slice][strip][8].  Three wavefronts per SIMD for
-// one block of look-ahead (151 to 163 registers; held to the 128 of four it
-// spills: 416 us for the 284 of 509 slices of 255^2), two for more.
+// of each strip to tilediag[slice][strip][8].  Three wavefronts per SIMD up to
+// 16 terms (151 to 168 registers and 36 bytes of spills; held to the 128 of
+// four 8 terms spill: 416 us for the 264 of 509 slices of 255^2), two beyond.
 template <int B, int L, int X, int NB>
-__global__ void __launch_bounds__(512, NB == 1 ? 3 : 2)
+__global__ void __launch_bounds__(64 * kStripWaves, NB <= 2 ? 3 : 2)
     k_adi_strip(const double2 *__restrict__ fin, double2 *__restrict__ fout, const double2 *__restrict__ src,
                 const int4 *__restrict__ box, StripCoef k, int ng, int first, int ns, int nstrip,
                 double *__restrict__ tilediag) {
@@ -2136,7 +2136,7 @@ __global__ void __launch_bounds__(512, NB == 1 ? 3 : 2)
     double2 *mine = strip_lds + (threadIdx.x >> 6) * G::lds;
     for (int i = threadIdx.x & 63; i < G::lds; i += 64) mine[i] = make_double2(0, 0);
     strip::lds_order();
-    const long long id = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const long long id = strip::item();
     if (id >= (long long)ns * nstrip) return;  // uniform per wavefront; no barrier follows
     const int ii = (int)(id / nstrip), q = (int)(id % nstrip);
     const long long fs = (long long)((ii + first) % ns), cells = (long long)ng * ng;
@@ -2533,11 +2533,9 @@ void launch_tile_sums(hipStream_t s, int ns, const double *tilediag, int ntiles,
 void launch_adi_strip(hipStream_t s, int ns, const double2 *fin, double2 *fout, const double2 *src, const int4 *box,
                       const StripCoef &k, int form, int ng, int first, double *tilediag) {
     const int nstrip = strip_dims(form).count(ng);
-    const int nw = std::min(nstrip, 8);  // a slice's strips on one CU: they share their halos in its cache
-    const unsigned nb = (unsigned)(((long long)ns * nstrip + nw - 1) / nw);
     strip_form(form, [&](auto b, auto l, auto x, auto n) {
-        const size_t lds = (size_t)nw * StripGeom<b(), l(), x(), n()>::lds * sizeof(double2);
-        hipLaunchKernelGGL((k_adi_strip<b(), l(), x(), n()>), dim3(nb), dim3(64 * nw), lds, s, fin, fout, src, box, k,
+        const size_t lds = (size_t)kStripWaves * StripGeom<b(), l(), x(), n()>::lds * sizeof(double2);
+        hipLaunchKernelGGL((k_adi_strip<b(), l(), x(), n()>), dim3(strip_blocks(ns, nstrip)), dim3(64 * kStripWaves), lds, s, fin, fout, src, box, k,
                            ng, first, ns, nstrip, tilediag);
     });
 }

@@ -15,6 +15,7 @@
 // replays any step of a run with no host work in between.
 #pragma once
 
+#include "g4mi_adi_strip.h"
 #include "g4mi_common.h"
 
 namespace g4mi {
@@ -48,6 +49,7 @@ struct MixBand {
     int klo, khi;                   // rows sharing the band of (klo+khi)/2
     int m;                          // half width the step size needs (<= template M)
     int pad;
+    StripCoef strip;
 };
 
 // Device-resident run state.
@@ -109,19 +111,20 @@ size_t mix_band_lds(int tmpl_m, bool refine);
 
 // One step: front (transverse + moments + radius), radial scan, main
 // (space charge + push + R56 + transverse + deposit + beam sums), ADI
-// (template band width tmpl_m, FP64 residual correction when refine),
+// (template band width tmpl_m, FP64 residual correction when refine, or the
+// strip kernel's `form`),
 // slippage, zeroing and the step record.  ev (optional, 9 events) brackets
 // the kernel groups: front [0,1], main [3 - 2], ADI [6,7], slippage + record
 // [7,8]; the other intervals are empty.
-// adi_mode: kAdiTile (32x32 tiles, correction up to a half width of 9),
-// kAdiStrips (streaming, one wavefront per column strip) or kAdiWide
-// (streaming, one workgroup per slice covering all columns; grids up to 512
-// columns, wider ones run the strips).
+// adi_mode: kAdiTile (FP32 band in 32x32 tiles, correction up to a half width
+// of 9), kAdiStrips (FP32 band streaming, one wavefront per column strip) or
+// kAdiWide (FP64 arithmetic in strips of whole columns, g4mi_adi_strip.h;
+// kAdiStrips for step sizes beyond its forms, form -1).
 // main_nt: threads per slice of the main kernel (256, 384, 512); main_lds: its
 // dynamic LDS region, 0 = 68 KiB, 1 = 44 KiB.
 constexpr int kAdiTile = 0, kAdiStrips = 1, kAdiWide = 2;
 int launch_mix_step(hipStream_t s, const MixArrays &a, int tmpl_m, bool refine, bool sc,
-                    bool moments, int maxzero, hipEvent_t *ev, int adi_mode, int main_nt, int main_lds,
+                    bool moments, int maxzero, hipEvent_t *ev, int adi_mode, int form, int main_nt, int main_lds,
                     bool front = true);
 // The same step as one cooperative launch of co-resident workgroups with
 // grid barriers between the phases (the streaming ADI); ev (optional, 9
@@ -135,7 +138,7 @@ int launch_mix_step_persistent(hipStream_t s, const MixArrays &a, int tmpl_m, bo
 // front: launch the front kernel (false when the previous step's main kernel ran it)
 void launch_mix_beam(hipStream_t s, const MixArrays &a, bool sc, bool moments, hipEvent_t *ev, bool egsum,
                      int main_nt = 384, int main_lds = 0, bool front = true);
-int launch_mix_adi(hipStream_t s, const MixArrays &a, int tmpl_m, bool refine, int adi_mode, int *ntiles);
+int launch_mix_adi(hipStream_t s, const MixArrays &a, int tmpl_m, bool refine, int adi_mode, int form, int *ntiles);
 void launch_mix_tail(hipStream_t s, const MixArrays &a, int maxzero, int ntiles, hipEvent_t *ev);
 // Field sums per storage slice ([ns][8], as the ADI's diagnostics with one
 // block per slice) of the live buffer (next = 0) or the other one (1).

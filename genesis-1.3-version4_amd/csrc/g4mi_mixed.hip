@@ -1555,298 +1555,30 @@ __global__ void __launch_bounds__(64) k_mix_adi_stream(MixArrays a) {
 }
 
 // ---------------------------------------------------------------------------
-// Whole-width streaming ADI: the row recurrence of adi_stream_body with one
-// workgroup of NW = blockDim / 64 wavefronts covering every column of a
-// slice (one lane per column), so no column is computed twice; the strips
-// above recompute a 2H-column halo (320 lanes for 255 columns at M = 4 with
-// the correction).  The E and u1 rows pass between the wavefronts through
-// LDS with one workgroup barrier per exchange whose fences cover LDS only,
-// so the field rows prefetched from HBM stay in flight across it.  Cells off
-// the grid hold zeros in the LDS rows: the Dirichlet boundary of A.
-//
-// Column map: wavefront 0 takes the first and the last 32 columns, whose
-// band rows differ from the central one; wavefronts 1.. take the columns in
-// between and use the symmetric central row when all of theirs lie in
-// [klo, khi].  Lanes left over sit on column ng (off the grid, zero).
-//
-// Buffers: the E row is double-buffered by row parity.  Without the
-// correction a wavefront may write row r+1 while another still reads row r
-// (one barrier per row).  With it, a second barrier between the E reads and
-// the u1 reads separates every write of a row from the reads of the row
-// before, so u1 needs one buffer.
-//
-// Dynamic LDS: E rows [2][NC + 2M] float2, u1 row [NC + 2] float2 (with the
-// correction), per-column band rows [W][NC] float2, wavefront sums [NW][8].
+// The ADI in column strips (g4mi_adi_strip.h): FP64 arithmetic from the stored
+// FP32 field to the stored FP32 result, so no residual correction follows.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-template <int M, bool REF>
-size_t wide_lds_bytes(int nw) {
-    const int nc = 64 * nw;
-    return (size_t)2 * (nc + 2 * M) * sizeof(float2) + (REF ? (size_t)(nc + 2) * sizeof(double2) : 0) +
-           (size_t)(2 * M + 1) * nc * sizeof(float2) + (size_t)nw * 8 * sizeof(double);
-}
-
-// three wavefronts per SIMD where the registers allow it without spilling
-template <int M, bool REF>
-__global__ void __launch_bounds__(512, (REF && M == 9) ? 2 : 3) k_mix_adi_wide(MixArrays a) {
-    using G = StreamGeom<M, REF>;
-    constexpr int W = G::W, QN = G::QN, PF = G::PF, UN = G::UN;
-    constexpr bool FIX = G::FIX;
-    extern __shared__ double2 wide_lds[];
-    const int nt = blockDim.x, nw = nt >> 6, nc = nt;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    float2 *lrow0 = (float2 *)wide_lds;                    // [2][nc + 2M]
-    const int lp = nc + 2 * M;
-    double2 *lu = (double2 *)(lrow0 + 2 * lp);              // [nc + 2] u1 row (FP32 values, widened)
-    float2 *lband = (float2 *)(lu + (REF ? nc + 2 : 0));    // [W][nc]
-    double *wsum = (double *)(lband + W * nc);              // [nw][8]
-    const int ii = blockIdx.x;
-    if (ii >= a.ns) return;
-    const MixStep &S = a.steps[a.st->istep];
-    const MixBand bi = a.binfo[S.band];
-    const float2 *band = a.bands + bi.off;
-    const double ad = bi.a;
-    const float af = (float)bi.a;
-    const double dn = 1.0 / (1.0 + 4.0 * ad * ad);
-    const int ng = a.ng, ns = a.ns;
-    // this lane's column
-    int x;
-    if (ng <= 64) x = lane < ng ? lane : ng;
-    else if (w == 0) x = lane < 32 ? lane : ng - 64 + lane;
-    else {
-        x = 32 + 64 * (w - 1) + lane;
-        if (x >= ng - 32) x = ng;
-    }
-    const bool xin = x < ng;
-    // every grid column of this wavefront shares the central band row (uniform)
-    bool wsym;
-    if (ng <= 64 || w == 0) wsym = bi.klo <= 0 && bi.khi >= ng - 1;
-    else {
-        const int xlo = 32 + 64 * (w - 1), xhi = min(xlo + 63, ng - 33);
-        wsym = xlo > xhi || (xlo >= bi.klo && xhi <= bi.khi);
-    }
-    // zero rows (the pads stay zero: only lanes on the grid write non-zero values)
-    for (int k = t; k < 2 * lp; k += nt) lrow0[k] = f2(0, 0);
-    if constexpr (REF)
-        for (int k = t; k < nc + 2; k += nt) lu[k] = d2(0, 0);
-    if (!wsym)
-        for (int m = 0; m < W; m++) lband[m * nc + t] = xin ? band[(long long)x * W + m] : f2(0, 0);
-    const float2 *bc = band + (long long)((bi.klo + bi.khi) / 2) * W;
-    float2 bcr[M + 1];  // the central row's right half b_M .. b_2M (symmetric)
-#pragma unroll
-    for (int m = 0; m <= M; m++) bcr[m] = bc[M + m];
-    const long long fs = (long long)((ii + a.st->first) % ns);
+template <int B, int L, int X, int NB>
+__global__ void __launch_bounds__(64 * kStripWaves, NB <= 2 ? 3 : 2) k_mix_adi_strip(MixArrays a, int nstrip) {
+    using G = StripGeom<B, L, X, NB>;
+    extern __shared__ double2 strip_lds[];
+    double2 *mine = strip_lds + (threadIdx.x >> 6) * G::lds;
+    for (int i = threadIdx.x & 63; i < G::lds; i += 64) mine[i] = d2(0, 0);
+    strip::lds_order();
+    const long long id = strip::item();
+    if (id >= (long long)a.ns * nstrip) return;  // uniform per wavefront; no barrier follows
+    const int ii = (int)(id / nstrip), q = (int)(id % nstrip);
+    const long long fs = (long long)((ii + a.st->first) % a.ns), cells = (long long)a.ng * a.ng;
+    const StripCoef k = strip::coef(&a.binfo[a.steps[a.st->istep].band].strip);
     const int cur = a.st->cur;
-    const float2 *u = a.field[cur] + fs * ng * ng;
-    float2 *uo = a.field[cur ^ 1] + fs * ng * ng;
-    const float2 *Sp = a.src + (long long)ii * ng * ng;
-    const int4 bx = a.box[ii];
-    const bool sxin = xin && x >= bx.x && x <= bx.z;
-    const int xcl = min(x, ng - 1);
-    const float2 *ucol = u + xcl, *scol = Sp + xcl;
-    auto uload = [&](int rr) -> float2 { return ucol[(long long)min(rr, ng - 1) * ng]; };
-    auto sload = [&](int rr) -> float2 {
-        const bool in = sxin && rr >= bx.y && rr <= bx.w;
-        return *(in ? scol + (long long)rr * ng : g_zero_row + xcl);
-    };
-    float2 q[QN], sq[QN];
-    q[0] = f2(0, 0);
-    sq[0] = f2(0, 0);
+    double dg[8];
+    adi_strip<float2, B, L, X, NB>(a.field[cur] + fs * cells, a.field[cur ^ 1] + fs * cells, a.src + ii * cells,
+                                   a.box[ii], a.ng, q, k, mine, dg);
 #pragma unroll
-    for (int k = 1; k < QN; k++) {
-        q[k] = uload(k - 1);
-        sq[k] = sload(k - 1);
-    }
-    float2 ring[W];
-#pragma unroll
-    for (int m = 0; m < W; m++) ring[m] = f2(0, 0);
-    constexpr int NL = REF ? (FIX ? W : M + 2) : 1;
-    float2 lo[NL];
-#pragma unroll
-    for (int m = 0; m < NL; m++) lo[m] = f2(0, 0);
-    float2 p1 = f2(0, 0), p2 = f2(0, 0);
-    // REF: the field rows r-1, r (and r+1 while row r is formed) widened to
-    // FP64 once each, as they enter the three-row window
-    double2 d_l = d2(0, 0), d_c = tod(q[1]);
-    // field sums of this column: x is fixed, so the x moments are dx, dx^2
-    // times the column's power, applied at the end
-    double s_w = 0, s_yw = 0, s_yyw = 0, s_re = 0, s_im = 0, s_cen = 0;
-    const bool xcen = x == ng / 2;
-    const double shift = -0.5 * (double)(ng - 1);
-    // output row y: the stored FP32 value o, the sums from o64 (the value
-    // before rounding with the correction)
-    auto emit = [&](int y, float2 o, double2 o64) {
-        if (xin) {
-            uo[(long long)y * ng + x] = o;
-            const double ox = o64.x, oy = o64.y;
-            const double wei = ox * ox + oy * oy;
-            const double dy = (double)y + shift;
-            s_w += wei;
-            s_yw += dy * wei;
-            s_yyw += dy * dy * wei;
-            s_re += ox;
-            s_im += oy;
-            if (xcen && y == ng / 2) s_cen = wei;
-        }
-    };
-    lds_barrier();
-    float2 *lx = lrow0 + x + M;  // this column in E row 0; row 1 is lp further
-    const int nrow = ng + M + (REF ? 1 : 0);
-    for (int r0 = 0; r0 < nrow; r0 += UN) {
-        // j = jj QN + jq: the queue slot of row r0 + j is a function of jq
-        // alone (a remainder of the flat index here keeps the loop from
-        // unrolling)
-#pragma unroll
-        for (int jj = 0; jj < UN / QN; jj++)
-#pragma unroll
-        for (int jq = 0; jq < QN; jq++) {
-            const int j = jj * QN + jq;
-            const int r = r0 + j;
-            if (r >= nrow) break;
-            float2 Fr = f2(0, 0), Flo = f2(0, 0);
-            if (r < ng) {
-                const float2 sv = sq[(jq + 1) % QN];
-                const float2 uc = q[(jq + 1) % QN];
-                const float2 un = (r + 1 < ng) ? q[(jq + 2) % QN] : f2(0, 0);
-                const float2 ul = (r > 0) ? q[jq] : f2(0, 0);
-                double2 E64 = d2(0, 0);
-                float2 E = f2(0, 0);
-                double2 sv64 = d2(0, 0);
-                if constexpr (REF) {
-                    const double2 d_n = (r + 1 < ng) ? tod(un) : d2(0, 0);
-                    if (xin) {
-                        sv64 = tod(sv);
-                        const double sx = fma(-2.0, d_c.x, d_n.x) + d_l.x;
-                        const double sy = fma(-2.0, d_c.y, d_n.y) + d_l.y;
-                        E64 = d2(fma(-ad, sy, sv64.x + d_c.x), fma(ad, sx, sv64.y + d_c.y));
-                    }
-                    d_l = d_c;
-                    d_c = d_n;
-                    E = tof(E64);
-                } else {
-                    const float sx = un.x - 2.f * uc.x + ul.x, sy = un.y - 2.f * uc.y + ul.y;
-                    E = xin ? f2(sv.x + uc.x - af * sy, sv.y + uc.y + af * sx) : f2(0, 0);
-                }
-                float2 *lr = lx + (r & 1) * lp;
-                lr[0] = E;
-                lds_barrier();
-                float2 up = f2(0, 0), up1 = f2(0, 0);  // two partial sums (even, odd terms)
-                if (xin) {
-                    if (wsym) {
-                        up = fmul(bcr[0], lr[0]);
-#pragma unroll
-                        for (int k = 1; k <= M; k++) {
-                            if (k & 1) up1 = ffma(bcr[k], fadd(lr[-k], lr[k]), up1);
-                            else up = ffma(bcr[k], fadd(lr[-k], lr[k]), up);
-                        }
-                    } else {
-#pragma unroll
-                        for (int m = 0; m < W; m++) {
-                            if (m & 1) up1 = ffma(lband[m * nc + t], lr[m - M], up1);
-                            else up = ffma(lband[m * nc + t], lr[m - M], up);
-                        }
-                    }
-                    up = fadd(up, up1);
-                }
-                if constexpr (REF) {
-                    // u1 goes to the row widened once, not by each neighbour
-                    const double2 u1 = tod(up);
-                    lu[x + 1] = u1;  // zero off the grid
-                    lds_barrier();
-                    const double2 nl = lu[x], nr = lu[x + 2];
-                    const double2 au = adi_apply(u1, d2(nl.x + nr.x, nl.y + nr.y), ad);
-                    const double2 upd = jacobi_update(u1, d2(E64.x - au.x, E64.y - au.y), ad, dn);
-                    if (xin) {
-                        const double2 F64 = d2(fma(2.0, upd.x, sv64.x) - E64.x, fma(2.0, upd.y, sv64.y) - E64.y);
-                        Fr = tof(F64);
-                        Flo = f2((float)(F64.x - (double)Fr.x), (float)(F64.y - (double)Fr.y));
-                    }
-                } else {
-                    Fr = xin ? f2(sv.x + 2.f * up.x - E.x, sv.y + 2.f * up.y - E.y) : f2(0, 0);
-                }
-                q[jq] = uload(r + PF + 1);
-                sq[jq] = sload(r + PF + 1);
-            }
-            if constexpr (FIX) {
-                ring[j % W] = Fr;
-                if constexpr (REF) lo[j % W] = Flo;
-            } else {
-#pragma unroll
-                for (int m = 0; m < W - 1; m++) ring[m] = ring[m + 1];
-                ring[W - 1] = Fr;
-                if constexpr (REF) {
-#pragma unroll
-                    for (int m = 0; m < NL - 1; m++) lo[m] = lo[m + 1];
-                    lo[NL - 1] = Flo;
-                }
-            }
-            float2 rw[W];
-#pragma unroll
-            for (int k = 0; k < W; k++) {
-                if constexpr (FIX) rw[k] = ring[(j + 1 + k) % W];
-                else rw[k] = ring[k];
-            }
-            const int y = r - M;
-            float2 o = f2(0, 0), o1 = f2(0, 0);
-            if (y >= 0 && y < ng) {
-                if (y >= bi.klo && y <= bi.khi) {
-                    o = fmul(bcr[0], rw[M]);
-#pragma unroll
-                    for (int k = 1; k <= M; k++) {
-                        if (k & 1) o1 = ffma(bcr[k], fadd(rw[M - k], rw[M + k]), o1);
-                        else o = ffma(bcr[k], fadd(rw[M - k], rw[M + k]), o);
-                    }
-                } else {
-                    const float2 *by = band + (long long)y * W;
-#pragma unroll
-                    for (int m = 0; m < W; m++) {
-                        if (m & 1) o1 = ffma(by[m], rw[m], o1);
-                        else o = ffma(by[m], rw[m], o);
-                    }
-                }
-                o = fadd(o, o1);
-            }
-            if constexpr (REF) {
-                const int yf = y - 1;
-                if (yf >= 0 && yf < ng) {
-                    const float2 fh = rw[M - 1];
-                    float2 fl;
-                    if constexpr (FIX) fl = lo[(j + W - M - 1) % W];
-                    else fl = lo[0];
-                    const double2 F64 = d2((double)fh.x + (double)fl.x, (double)fh.y + (double)fl.y);
-                    const double2 u2 = tod(p1);
-                    const double2 nb = d2((double)p2.x + (double)o.x, (double)p2.y + (double)o.y);
-                    const double2 au = adi_apply(u2, nb, ad);
-                    const double2 res = jacobi_update(u2, d2(F64.x - au.x, F64.y - au.y), ad, dn);
-                    emit(yf, tof(res), res);
-                }
-                p2 = p1;
-                p1 = o;
-            } else {
-                if (y >= 0) emit(y, o, tod(o));
-            }
-        }
-    }
-    const double dx = (double)x + shift;
-    double dg[8] = {s_w, dx * s_w, dx * dx * s_w, s_yw, s_yyw, s_re, s_im, s_cen};
-    if (!xin)
-        for (int k = 0; k < 8; k++) dg[k] = 0;
-#pragma unroll
-    for (int k = 0; k < 8; k++)
-        for (int o = 32; o > 0; o >>= 1) dg[k] += __shfl_xor(dg[k], o);
-    if (lane == 0)
-        for (int k = 0; k < 8; k++) wsum[w * 8 + k] = dg[k];
-    __syncthreads();
-    if (t < 8) {
-        double v = wsum[t];
-        for (int q2 = 1; q2 < nw; q2++) v += wsum[q2 * 8 + t];
-        a.tilediag[fs * 8 + t] = v;
-    }
+    for (int c = 0; c < 8; c++)
+        for (int o = 32; o > 0; o >>= 1) dg[c] += __shfl_xor(dg[c], o);
+    if ((threadIdx.x & 63) == 0)
+        for (int c = 0; c < 8; c++) a.tilediag[(fs * nstrip + q) * 8 + c] = dg[c];
 }
 
 // ---------------------------------------------------------------------------
@@ -2088,7 +1820,9 @@ bool mix_band_supported(int m, int *tmpl_m) {
 int mix_band_tiles(int ng) {
     const int ntx = (ng + 31) / 32;
     // the tile-diagnostic scratch also holds the strip sums of the streaming kernel
-    return std::max(ntx * ntx, stream_strips(ng, 12, true));
+    int n = std::max(ntx * ntx, stream_strips(ng, 12, true));
+    for (int f = 0; f < kStripForms; f++) n = std::max(n, strip_dims(f).count(ng));
+    return n;
 }
 
 size_t mix_band_lds(int tmpl_m, bool refine) {
@@ -2124,24 +1858,6 @@ void launch_main(hipStream_t s, const MixArrays &a, int sc, int nt, int lds) {
         else if (nt == 512) launch_main_t<EG, 512, kMixDyn>(s, a, sc);
         else launch_main_t<EG, 384, kMixDyn>(s, a, sc);
     }
-}
-
-constexpr size_t kLdsMax = 160 * 1024;
-
-// the whole-width kernel's LDS limit: what eight wavefronts need, at most
-// the CU's 160 KiB (wider grids with wide bands then run the strips)
-template <int M, bool REF>
-int set_wide_attr() {
-    return hipFuncSetAttribute((const void *)k_mix_adi_wide<M, REF>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)std::min(wide_lds_bytes<M, REF>(8), kLdsMax)) == hipSuccess;
-}
-
-size_t wide_lds_need(int tmpl_m, bool refine, int nw) {
-#define G4_L(MM) \
-    if (tmpl_m == MM) return refine ? wide_lds_bytes<MM, true>(nw) : wide_lds_bytes<MM, false>(nw);
-    G4_L(3) G4_L(4) G4_L(6) G4_L(9) G4_L(12)
-#undef G4_L
-    return ~(size_t)0;
 }
 
 template <int M, bool REF>
@@ -2191,8 +1907,7 @@ int mix_prepare() {
           set_main_attr<false, 256, kMixDynT>() && set_main_attr<false, 384, kMixDynT>();
 #undef G4_M
 #define G4_P(MM) ok &= set_adi_attr<MM, false>(); if (MixGeom<MM, true>::lds_bytes <= 160 * 1024) ok &= set_adi_attr<MM, true>(); \
-    ok &= set_persistent_attr<MM, false>(); ok &= set_persistent_attr<MM, true>(); \
-    ok &= set_wide_attr<MM, false>(); ok &= set_wide_attr<MM, true>();
+    ok &= set_persistent_attr<MM, false>(); ok &= set_persistent_attr<MM, true>();
     G4_P(3) G4_P(4) G4_P(6) G4_P(9) G4_P(12)
 #undef G4_P
     return ok ? 0 : -1;
@@ -2218,34 +1933,19 @@ void launch_mix_beam(hipStream_t s, const MixArrays &a, bool sc, bool moments, h
     mark(6);
 }
 
-int launch_mix_adi(hipStream_t s, const MixArrays &a, int tmpl_m, bool refine, int mode, int *ntiles) {
-    // eight wavefronts cover 512 columns; the LDS of one workgroup at most 160 KiB
-    if (mode == kAdiWide &&
-        (a.ng > 512 || wide_lds_need(tmpl_m, refine, std::max(1, (a.ng + 63) / 64)) > kLdsMax))
-        mode = kAdiStrips;
-    const bool stream = mode != kAdiTile;
-    if (refine && !stream && mix_band_lds(tmpl_m, true) > 160 * 1024) return -1;
+int launch_mix_adi(hipStream_t s, const MixArrays &a, int tmpl_m, bool refine, int mode, int form, int *ntiles) {
+    if (mode == kAdiWide && form < 0) mode = kAdiStrips;  // grids within the band's reach, any step size
     if (mode == kAdiWide) {
-        // whole-width kernel: one workgroup of ceil(ng / 64) wavefronts per slice
-        *ntiles = 1;
-        const int nw = std::max(1, (a.ng + 63) / 64);
-#define G4_W(MM)                                                                                          \
-    else if (tmpl_m == MM) {                                                                              \
-        if (refine) {                                                                                     \
-            const size_t lds = wide_lds_bytes<MM, true>(nw);                                              \
-            hipLaunchKernelGGL((k_mix_adi_wide<MM, true>), dim3(a.ns), dim3(64 * nw), lds, s, a);         \
-        } else {                                                                                          \
-            const size_t lds = wide_lds_bytes<MM, false>(nw);                                             \
-            hipLaunchKernelGGL((k_mix_adi_wide<MM, false>), dim3(a.ns), dim3(64 * nw), lds, s, a);        \
-        }                                                                                                 \
-    }
-        if (false) {
-        }
-        G4_W(3) G4_W(4) G4_W(6) G4_W(9) G4_W(12)
-        else return -1;
-#undef G4_W
+        const int nstrip = *ntiles = strip_dims(form).count(a.ng);
+        strip_form(form, [&](auto b, auto l, auto x, auto n) {
+            const size_t lds = (size_t)kStripWaves * StripGeom<b(), l(), x(), n()>::lds * sizeof(double2);
+            hipLaunchKernelGGL((k_mix_adi_strip<b(), l(), x(), n()>), dim3(strip_blocks(a.ns, nstrip)),
+                               dim3(64 * kStripWaves), lds, s, a, nstrip);
+        });
         return 0;
     }
+    const bool stream = mode != kAdiTile;
+    if (refine && !stream && mix_band_lds(tmpl_m, true) > 160 * 1024) return -1;
 #define G4_A(MM)                                         \
     else if (tmpl_m == MM) {                             \
         if (refine) launch_adi_t<MM, true>(s, a);        \
@@ -2287,11 +1987,11 @@ void launch_mix_tail(hipStream_t s, const MixArrays &a, int maxzero, int ntiles,
 }
 
 int launch_mix_step(hipStream_t s, const MixArrays &a, int tmpl_m, bool refine, bool sc,
-                    bool moments, int maxzero, hipEvent_t *ev, int adi_mode, int main_nt, int main_lds,
+                    bool moments, int maxzero, hipEvent_t *ev, int adi_mode, int form, int main_nt, int main_lds,
                     bool front) {
     launch_mix_beam(s, a, sc, moments, ev, false, main_nt, main_lds, front);
     int ntiles = 0;
-    if (launch_mix_adi(s, a, tmpl_m, refine, adi_mode, &ntiles) != 0) return -1;
+    if (launch_mix_adi(s, a, tmpl_m, refine, adi_mode, form, &ntiles) != 0) return -1;
     launch_mix_tail(s, a, maxzero, ntiles, ev);
     return 0;
 }

@@ -264,8 +264,8 @@ int g4mi_sort_index_noalloc(g4mi_ctx *ctx, double slen, int *atar, long long *mo
  * wavefronts per slice x 68 or 44 KiB of LDS, 4 or 6 x 32 KiB), the three ADI kernels,
  * and the step as a graph of kernels against one persistent
  * cooperative launch, and keep the fastest.  Entries: "adi_refine" (FP64
- * residual correction, default 1), "mixed_adi" (2 whole-width streaming,
- * 1 streaming strips, 0 tiles),
+ * residual correction of its FP32 band products, default 1), "mixed_adi" (2
+ * FP64 arithmetic in column strips, 1 FP32 band in streaming strips, 0 in tiles),
  * "main_nt" (256, 384, 512), "main_lds" (0: 68 KiB, 1: 44 KiB, 2: 32 KiB;
  * 512 threads take 44 KiB for 2),
  * "persistent", "graphs" (0/1); setting any of the kernel entries turns the

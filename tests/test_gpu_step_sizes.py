@@ -6,8 +6,10 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import cases
 import g4mi
 import harness as H
+import oracle_py as O
 
 pytestmark = pytest.mark.gpu
 
@@ -61,13 +63,16 @@ def test_harmonic_field_in_each_adi_kernel(kernel, ngrid):
     ctx.close()
 
 
-@pytest.mark.parametrize("delz", [0.004, 0.03, 0.1, 0.24, 0.4])
-@pytest.mark.parametrize("ngrid", [3, 5, 16, 17, 18, 26, 33, 34, 35, 42, 49, 50, 51, 63, 64, 100, 101, 130, 255, 300])
+STRIP_GRIDS = [3, 5, 16, 17, 18, 26, 33, 34, 35, 42, 48, 49, 50, 51, 54, 55, 64, 100, 105, 130, 255, 300]
+
+
+@pytest.mark.parametrize("delz", [0.004, 0.015, 0.03, 0.045, 0.1, 0.24, 0.55, 0.75])
+@pytest.mark.parametrize("ngrid", STRIP_GRIDS)
 def test_column_strips(ngrid, delz):
     """The strip kernel (adi_kernel 4) at grids narrower than its halo, at the
-    edges of its strips (50 to 26 columns) and blocks of 8 rows, with the
+    edges of its strips (54 to 18 columns) and blocks of 8 rows, with the
     source's footprint anywhere in the grid (and none), for one step size per
-    form (8, 9, 12, 16 and 20 terms), against the oracle: two steps of the
+    form (6 to 24 terms), against the oracle: two steps of the
     single step's 1e-13 bar."""
     gridmax = 0.5e-3 * (ngrid - 1) / 150  # the cell of 151 columns on 1 mm
     sim = H.make_state([256, 512, 0, 1024, 256], ngrid=ngrid, gridmax=gridmax, timerun=False)
@@ -91,4 +96,34 @@ def test_column_strips(ngrid, delz):
     print(f"  {ngrid}^2, delz {delz}: {err:.2e}", flush=True)
     assert err < 2e-13
     assert np.max(np.abs(d["power"] / d["power"].sum() - w / w.sum())) < 1e-12
+    ctx.close()
+
+
+@pytest.mark.parametrize("ngrid,delz", [(n, d) for n in STRIP_GRIDS for d in (0.004, 0.03, 0.06, 0.1, 0.24, 0.4, 0.75, 1.1)] +
+                         [(5, 4.0), (9, 4.0)])
+def test_column_strips_mixed(ngrid, delz):
+    """The mixed form's strip kernel (mixed_adi 2) at the same edges, one step
+    size per form (6 to 24 terms) and beyond them, against the oracle: without current, two
+    steps of one FP32 rounding each (2^-24 of a component, so of the largest
+    value) on a seed that FP32 holds exactly."""
+    gridmax = 0.5e-3 * (ngrid - 1) / 150
+    sim = H.make_state([256] * 3, ngrid=ngrid, gridmax=gridmax, timerun=False)
+    sim.current[:] = 0.0
+    rng = np.random.default_rng(ngrid)
+    sim.field[:] = rng.normal(size=sim.field.shape).astype(np.float32) * 2.0 ** 30
+    ctx = H.to_gpu(sim, precision=g4mi.FP32)
+    ctx.set_schedule("mixed_adi", 2)
+    st = H.steps(1, 2)
+    st[0].dz = delz
+    for _ in range(2):
+        O.lib().orc_step_all(C.byref(sim.s), C.byref(st[0]), cases.GAMMA0)
+        ctx.step(H.gsteps(st)[0], cases.GAMMA0)
+    assert ctx.schedule()["adi"] == "band32-wide"
+    f, _ = ctx.download_field()
+    err = np.max(np.abs(f - sim.field)) / np.max(np.abs(sim.field))
+    d = ctx.diag()
+    w = (sim.field ** 2).sum(axis=2).sum(axis=1)
+    print(f"  {ngrid}^2, delz {delz}: {err:.2e}", flush=True)
+    assert err < 2.5 * 2.0 ** -24
+    assert np.max(np.abs(d["power"] / d["power"].sum() - w / w.sum())) < 1e-6
     ctx.close()
