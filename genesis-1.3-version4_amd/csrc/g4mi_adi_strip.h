@@ -106,7 +106,10 @@ inline unsigned strip_blocks(int ns, int nstrip) {
 // Coefficients of a step size: the x convolution's first factor at distances
 // 0 .. 4, its binary factors (cell and neighbours), the single term, and the y
 // elimination's tables (device): cbet[ng] and -cwet[ng + kStripPad] (zero from
-// ng on: the back substitution reads up to 8 NB rows past the last).
+// ng on: the back substitution reads up to 8 NB rows past the last).  The
+// cell's coefficients are kept as their difference from 1: they lie close to
+// it, and their rounding would be the same for every cell and step (2e-16 to
+// 4e-16 of the power a step, several times Thomas').
 constexpr int kStripPad = 32;
 struct StripCoef {
     double a;  // Im(cstep)
@@ -238,7 +241,7 @@ __device__ __forceinline__ void adi_strip(const T2 *__restrict__ u, T2 *__restri
                     E.x *= sign;
                     E.y *= sign;
                 }
-                double2 v = mul(k.e[0], E), far = z2;
+                double2 v = fma2(k.e[0], E, E), far = z2;
                 if (!G::taps) {
                     v = fma2(k.e[1], beside(E), v);
                 } else {
@@ -253,7 +256,7 @@ __device__ __forceinline__ void adi_strip(const T2 *__restrict__ u, T2 *__restri
                     const int d = B << l;
                     *row[l] = v;
                     lds_order();
-                    v = fma2(k.s[l], sum(row[l][-d], row[l][d]), mul(k.c[l], v));
+                    v = fma2(k.s[l], sum(row[l][-d], row[l][d]), fma2(k.c[l], v, v));
                 }
                 if (X) v = fma2(k.x, far, v);
                 lds_order();

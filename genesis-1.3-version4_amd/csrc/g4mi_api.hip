@@ -40,6 +40,7 @@ struct AdiPlan {
     double2 *fac = nullptr, *band = nullptr;  // one allocation: c | cbet | cwet, the band, strip_k's tables
     int strip = -1;                           // the strip kernel's form; -1: none holds the step size
     StripCoef strip_k{};
+    LineCoef line{};                          // the line kernels' factors (levels 0: Thomas instead)
 };
 // The spectral solver's tables for one step size: the convolution's kernel
 // transform and, once a GEMM needs it, the propagator matrix.
@@ -118,7 +119,7 @@ struct Ctx {
     int ntiles = 0;                    // they are still per tile or strip in d_tilediag, this many a slice
     std::vector<int> zeroed_since_adi;
     // ADI kernel chosen by the autotuner (-1: not tuned yet) and its timings:
-    // 0 two-kernel Thomas, 1 fused recurrence, 2 fused recurrence with
+    // 0 line by line (wavefronts or Thomas), 1 fused recurrence, 2 fused recurrence with
     // prefetch, 3 banded inverse, 4 column strips
     int adi_kernel = -1;
     bool adi_fixed = false;               // set by g4mi_set_schedule("adi_kernel", k >= 0)
@@ -382,15 +383,38 @@ static int strip_coef(double a, double bar, StripCoef *k) {
     for (int m = 0; m < d.B; m++) {
         cld t = 0;
         for (int n = d.B - m; n-- > 0;) t = 1.0L + r.w * r.w * t;
-        k->e[m] = d2(r.g * (1.0L - r.w * r.w) * std::pow(r.w, m) * t);
+        k->e[m] = d2(r.g * (1.0L - r.w * r.w) * std::pow(r.w, m) * t - (m ? 0.0L : 1.0L));
     }
     cld wj = std::pow(r.w, d.B);
     for (int l = 0; l < d.L; l++, wj *= wj) {
-        k->c[l] = d2(1.0L + wj * wj);
+        k->c[l] = d2(wj * wj);
         k->s[l] = d2(wj);
     }
     k->x = d2(r.g * wj);  // at B 2^L
     return form;
+}
+
+// The line kernels' factors, 2^levels terms; levels 0 if more than
+// 2^kLineLevels are needed or the grid is wider than they take.
+static void line_coef(double a, int ng, double bar, LineCoef *k) {
+    const AdiRoot r = adi_root(a);
+    k->a = a;
+    if (ng > kLineMax) return;
+    int n = 1;
+    double w = (double)std::abs(r.w);
+    for (w *= w; n < kLineLevels && !(w < bar); n++) w *= w;
+    if (!(w < bar)) return;
+    k->levels = n;
+    typedef std::complex<long double> cld;
+    auto d2 = [](cld v) { return make_double2((double)v.real(), (double)v.imag()); };
+    const int per = 2 * (ng + 1);
+    cld wj = r.w, f = r.g * (1.0L - r.w * r.w);
+    for (int l = 0; l < n; l++, wj *= wj, f = 1.0L) {
+        const int d = (1 << l) % per;  // both directions are summed: d and per - d are one distance
+        k->d[l] = std::min(d, per - d);
+        k->c[l] = d2(f * (1.0L + wj * wj) - 1.0L);
+        k->s[l] = d2(f * wj);
+    }
 }
 
 // FieldSolverADI::init for one grid and step size, kept in `pc`.
@@ -447,6 +471,7 @@ static int adi_plan(Ctx *c, PlanCache<AdiPlan> &pc, int ng, double dgrid, double
         for (int i = 0; i < 2 * ng; i++) h.push_back(-h[4 * ng + i]);
         h.insert(h.end(), 2 * kStripPad, 0.0);
     }
+    line_coef(p.cstep, ng, std::ldexp(1.0, -58), &p.line);
     G4_TRY(plans_room(c, pc, h.size() * sizeof(double)));
     G4_HIP(hipMalloc(&p.fac, h.size() * sizeof(double)));
     if (hipMemcpy(p.fac, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
@@ -464,7 +489,7 @@ static int adi_plan(Ctx *c, PlanCache<AdiPlan> &pc, int ng, double dgrid, double
 
 // The most blocks of field sums that any ADI kernel writes per slice.
 static int adi_sum_blocks(int ng) {
-    int n = adi_band_tiles(ng);
+    int n = std::max(adi_band_tiles(ng), line_blocks(ng));
     for (int f = 0; f < kStripForms; f++) n = std::max(n, strip_dims(f).count(ng));
     return n;
 }
@@ -474,7 +499,7 @@ static int ensure_factors(Ctx *c, double delz) {
     c->adi_delz = std::nan("");  // until the new plan is there
     G4_TRY(adi_plan(c, c->adi_plans, c->ng, c->dgrid, c->xks, delz, &c->adi));
     c->adi_delz = delz;
-    if ((c->adi.band_m || c->adi.strip >= 0) && !c->d_tilediag)
+    if ((c->adi.band_m || c->adi.strip >= 0 || c->adi.line.levels) && !c->d_tilediag)
         G4_HIP(hipMalloc(&c->d_tilediag, (size_t)c->ns * adi_sum_blocks(c->ng) * 8 * sizeof(double)));
     if (!c->adi_fixed) {
         // the tuner's choice for this step size, or tune it at the next field step
@@ -648,34 +673,44 @@ static void adi_launch(Ctx *c, int kind, const AdiField &a, double2 *fin, double
                         p.klo, p.khi, a.tilediag, nullptr);
     else if (kind == 1 || kind == 2)
         launch_adi_fused(c->stream, c->ns, fin, fout, a.src, a.box, f, c->first, a.diag, p.tile, kind == 2);
+    else if (p.line.levels)
+        launch_adi_lines(c->stream, c->ns, fin, fout, a.src, a.box, p.line, a.ng, c->first, a.tilediag);
     else
         launch_adi(c->stream, c->ns, fin, fout, a.src, a.box, f, c->first);
 }
 
 // Autotuner of the ADI, before a field's first step of each step size; ms[5]
-// receives the timings, -1 for kernels not run.  Where the banded inverse or
-// the strips hold the step size, only these two are run: they always beat the
-// others (ms a launch, strips | band | recurrence | recurrence with prefetch |
-// Thomas, - not eligible: 509 slices of 255^2, 0.08 m 0.35 | 1.45 | 1.30 |
-// 0.79 | 2.7; 97 of 151^2 0.095 | 0.066 | 0.240 | 0.185 | 0.31; one of 255^2
-// 0.17 | 0.032 | - | - | 0.40), and they leave their input alone, so they run
-// on the field itself.  Few slices want the band's many tiles, many the strips'
-// fewer operations, and where they cross depends on the step size, so both are
-// timed, up to one strip for each of the 1024 SIMDs: from there the strips are
-// taken (0.26 | 0.54 for 509 slices of 255^2, 0.16 | 0.44 for 1024 of 151^2).
-// A single candidate is taken as it is.
+// receives the timings, -1 for kernels not run.  us a launch (with the timing
+// events' 5), lines | band | strips, - not eligible:
+//     slices   1              16             97             200
+//   151^2 M 7  12 |  13 |  59   24 | 17 | 66   60 |  52 | 74      | 91 | 73
+//   151^2 M 16 13 |  18 |  77   25 | 34 | 79   62 | 136 | 86      | 250 | 90
+//   255^2 M 8  14 |  16 | 108   33 | 29 | 116  160 | 122 | 131
+//   255^2 M -  15 |   - | 134   34 |  - | 140  165 |   - | 149
+// (Thomas' two sweeps: 400 for one slice of 255^2.)  Many slices want the
+// strips' fewer passes: from one strip for each of the 1024 SIMDs on they are
+// taken (0.26 ms for the band's 0.54 at 509 slices of 255^2).  Few want the
+// many wavefronts of the band or the lines: the band where 8 columns on a side
+// hold the step size (timed against the strips, on the field itself: both
+// leave it alone), else the lines, up to half as many strips as SIMDs.  The
+// window recurrences and Thomas remain for what none of these takes.
 static int tune_adi(Ctx *c, const AdiField &a, double2 *field, double2 *work, int *choice, float *ms) {
-    if (adi_eligible(a, 4) && (long long)c->ns * strip_dims(a.p->strip).count(a.ng) >= 1024) {
+    std::fill(ms, ms + 5, -1.f);
+    const AdiPlan &p = *a.p;
+    const long long strips = p.strip >= 0 ? (long long)c->ns * strip_dims(p.strip).count(a.ng) : 0;
+    const bool narrow = p.band_m && p.band_m <= 8;
+    if (strips >= (narrow ? 1024 : 512)) {
         *choice = 4;
-        std::fill(ms, ms + 5, -1.f);
+        return G4MI_OK;
+    }
+    if (!narrow && p.line.levels) {
+        *choice = 0;
         return G4MI_OK;
     }
     const bool out = adi_eligible(a, 3) || adi_eligible(a, 4);
     std::vector<int> kinds;
-    for (int kind = 0; kind < 5; kind++) {
-        ms[kind] = -1.f;
+    for (int kind = 0; kind < 5; kind++)
         if (adi_eligible(a, kind) && (kind >= 3) == out) kinds.push_back(kind);
-    }
     *choice = kinds[0];
     if (kinds.size() == 1) return G4MI_OK;
     const size_t bytes = (size_t)c->ns * a.ng * a.ng * sizeof(double2);
@@ -1027,9 +1062,10 @@ static int field_track(Ctx *c, const g4mi_step_params &st, double delz, bool dep
         c->adi_choice[c->adi_delz] = c->adi_kernel;
     }
     adi_launch(c, c->adi_kernel, a, c->d_field, c->d_work);
-    c->ntiles = c->adi_kernel == 3 ? adi_band_tiles(c->ng) : c->adi_kernel == 4 ? strip_dims(c->adi.strip).count(c->ng) : 0;
+    c->ntiles = c->adi_kernel == 4 ? strip_dims(c->adi.strip).count(c->ng) : c->adi_kernel == 3 ? adi_band_tiles(c->ng)
+                : c->adi_kernel == 0 && c->adi.line.levels ? line_blocks(c->ng) : 0;
     if (c->adi_kernel >= 3) std::swap(c->d_field, c->d_work);  // result is in the other buffer
-    c->field_diag_fresh = c->adi_kernel != 0;
+    c->field_diag_fresh = c->adi_kernel != 0 || c->ntiles;
     c->zeroed_since_adi.clear();
     G4_HIP(hipGetLastError());
     if (c->ev) G4_HIP(hipEventRecord(c->ev[7], c->stream));

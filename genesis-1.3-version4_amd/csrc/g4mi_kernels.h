@@ -96,6 +96,20 @@ void launch_deposit(hipStream_t s, int ns, const long long *off, const double *g
                     double2 *src, int4 *box, const DepositParams &p);
 void launch_adi(hipStream_t s, int ns, double2 *field, double2 *work, const double2 *src,
                 const int4 *box, const AdiFactors &f, int first);
+// The same with a wavefront per line and the lines' systems as a product of
+// log2 convolutions (grids up to kLineMax, coefficients from the host); the
+// field sums of every four columns to tilediag [ns][line_blocks(ng)][8] (null:
+// none).
+constexpr int kLineMax = 512, kLineLevels = 10;
+struct LineCoef {
+    double a;       // Im(cstep)
+    int levels;     // 2^levels terms on each side
+    int d[kLineLevels];
+    double2 c[kLineLevels], s[kLineLevels];  // factor at distance d: cell (less 1) and neighbours
+};
+inline int line_blocks(int ng) { return (ng + 3) / 4; }
+void launch_adi_lines(hipStream_t s, int ns, double2 *field, double2 *work, const double2 *src, const int4 *box,
+                      const LineCoef &k, int ng, int first, double *tilediag);
 // Fused two-sweep ADI (one workgroup per slice, ngrid <= 256) with
 // register-window back substitution of `tile` cells (8 or 16), tiles
 // prefetched into registers (prefetch=1) or loaded when needed (0), and the

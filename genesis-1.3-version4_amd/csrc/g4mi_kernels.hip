@@ -1585,6 +1585,111 @@ __global__ void __launch_bounds__(64) k_adi_y(double2 *__restrict__ field,
 }
 
 // ---------------------------------------------------------------------------
+// K5/K6 with a wavefront per line, C cells of the line in each lane.  The
+// inverse as the strips' convolution (g4mi_adi_strip.h: odd continuation about
+// the cells beside the ends, factors at distances 1, 2, 4, ..), here along a
+// line held in LDS, so that it reaches as far as any step size needs: 2^levels
+// terms, distances taken modulo the continuation's period.  A line's levels
+// depend on one another, its cells do not, and every line has a wavefront:
+// latency-bound at 5.1 + 7.7 us for one slice of 255^2, where the banded tiles
+// of 33 terms take 32 us and Thomas' dependent steps 207 + 189 us.  From about
+// 100 slices of 151^2 on its levels' LDS traffic is more than the strips' work
+// (the dispatch compares them).  k_adi_line_x leaves F = S + (1 + i a d_x^2) u'
+// in `work`, so the column pass reads one value a cell.  A wavefront's LDS
+// accesses are in order: no barrier.
+// ---------------------------------------------------------------------------
+template <int C>
+__device__ __forceinline__ void line_solve(double2 (&v)[C], double2 *row, int ng, const LineCoef &k) {
+    using namespace strip;
+    const int lane = threadIdx.x & 63, per = 2 * (ng + 1);
+    if (lane == 0) row[0] = row[ng + 1] = make_double2(0, 0);
+    for (int l = 0; l < k.levels; l++) {
+#pragma unroll
+        for (int c = 0; c < C; c++)
+            if (lane + 64 * c < ng) row[lane + 64 * c + 1] = v[c];
+        lds_order();
+        const int d = k.d[l];  // 0 .. ng + 1
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const int t = min(lane + 64 * c, ng - 1) + 1, n = t - d, m = t + d;
+            const double2 p = row[abs(n)], q = row[m > ng + 1 ? per - m : m];
+            const double sp = n < 0 ? -1.0 : 1.0, sq = m > ng + 1 ? -1.0 : 1.0;
+            const double2 b = make_double2(__builtin_fma(sq, q.x, sp * p.x), __builtin_fma(sq, q.y, sp * p.y));
+            v[c] = fma2(k.s[l], b, fma2(k.c[l], v[c], v[c]));
+        }
+        lds_order();
+    }
+}
+
+template <int C>
+__global__ void __launch_bounds__(64) k_adi_line_x(const double2 *__restrict__ field, double2 *__restrict__ work,
+                                                   const double2 *__restrict__ src, const int4 *__restrict__ box,
+                                                   LineCoef k, int ng, int first, int ns) {
+    extern __shared__ double2 line_lds[];
+    const int lane = threadIdx.x, r = blockIdx.x, ii = blockIdx.y;
+    const long long fs = (long long)((ii + first) % ns) * ng * ng + (long long)r * ng;
+    const double2 *u = field + fs, *S = src + (long long)ii * ng * ng;
+    const int4 bx = box[ii];
+    double2 s[C], e[C], v[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int x = min(lane + 64 * c, ng - 1);
+        const double2 z = make_double2(0, 0);
+        const double2 uc = u[x], un = r + 1 < ng ? u[x + ng] : z, um = r > 0 ? u[x - ng] : z;
+        s[c] = src_at(S, bx, x, r, ng);
+        const double dx = __builtin_fma(-2.0, uc.x, un.x) + um.x, dy = __builtin_fma(-2.0, uc.y, un.y) + um.y;
+        v[c] = e[c] = make_double2(__builtin_fma(-k.a, dy, s[c].x + uc.x), __builtin_fma(k.a, dx, s[c].y + uc.y));
+    }
+    line_solve<C>(v, line_lds, ng, k);
+#pragma unroll
+    for (int c = 0; c < C; c++)
+        if (lane + 64 * c < ng)
+            work[fs + lane + 64 * c] = make_double2(__builtin_fma(2.0, v[c].x, s[c].x - e[c].x),
+                                                    __builtin_fma(2.0, v[c].y, s[c].y - e[c].y));
+}
+
+template <int C>
+__global__ void __launch_bounds__(256) k_adi_line_y(double2 *__restrict__ field, const double2 *__restrict__ work,
+                                                    LineCoef k, int ng, int ns, double *__restrict__ tilediag) {
+    extern __shared__ double2 line_lds[];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, x = blockIdx.x * 4 + w, fi = blockIdx.y;
+    const long long fs = (long long)fi * ng * ng;
+    double dg[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (x < ng) {  // uniform per wavefront
+        double2 v[C];
+#pragma unroll
+        for (int c = 0; c < C; c++) v[c] = work[fs + (long long)min(lane + 64 * c, ng - 1) * ng + x];
+        line_solve<C>(v, line_lds + w * (ng + 2), ng, k);
+        const double shift = -0.5 * (double)(ng - 1), dx = (double)x + shift;
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const int r = lane + 64 * c;
+            if (r >= ng) continue;
+            field[fs + (long long)r * ng + x] = v[c];
+            const double wei = __builtin_fma(v[c].x, v[c].x, v[c].y * v[c].y), dy = (double)r + shift;
+            dg[0] += wei;
+            dg[3] += dy * wei;
+            dg[4] += dy * dy * wei;
+            dg[5] += v[c].x;
+            dg[6] += v[c].y;
+            if (r == ng / 2 && x == ng / 2) dg[7] = wei;
+        }
+        dg[1] = dx * dg[0];
+        dg[2] = dx * dx * dg[0];
+    }
+    if (!tilediag) return;
+    __syncthreads();  // the lines' rows are free
+    double *sum = (double *)line_lds;
+#pragma unroll
+    for (int c = 0; c < 8; c++) dg[c] = wave_sum(dg[c]);
+    if (lane == 0)
+        for (int c = 0; c < 8; c++) sum[w * 8 + c] = dg[c];
+    __syncthreads();
+    const int c = threadIdx.x;
+    if (c < 8) tilediag[((long long)fi * gridDim.x + blockIdx.x) * 8 + c] = sum[c] + sum[8 + c] + sum[16 + c] + sum[24 + c];
+}
+
+// ---------------------------------------------------------------------------
 // K5+K6 fused: both ADI half steps of one slice per workgroup.
 //
 // FieldSolverADI::ADI (:60-91) solves (1 - i a d_x^2) u' = S + (1 + i a d_y^2) u
@@ -2494,6 +2599,22 @@ void launch_adi(hipStream_t s, int ns, double2 *field, double2 *work, const doub
     dim3 grid(nblk(f.ngrid, 64), ns);
     hipLaunchKernelGGL(k_adi_x, grid, dim3(64), 0, s, field, work, src, box, f, first, ns);
     hipLaunchKernelGGL(k_adi_y, grid, dim3(64), 0, s, field, work, src, box, f, first, ns);
+}
+void launch_adi_lines(hipStream_t s, int ns, double2 *field, double2 *work, const double2 *src, const int4 *box,
+                      const LineCoef &k, int ng, int first, double *tilediag) {
+    const size_t lds = (size_t)(ng + 2) * sizeof(double2);
+    const size_t ldsy = std::max(4 * lds, 32 * sizeof(double));
+    auto go = [&](auto c) {
+        constexpr int C = decltype(c)::value;
+        hipLaunchKernelGGL(k_adi_line_x<C>, dim3(ng, ns), dim3(64), lds, s, field, work, src, box, k, ng, first, ns);
+        hipLaunchKernelGGL(k_adi_line_y<C>, dim3(line_blocks(ng), ns), dim3(256), ldsy, s, field, work, k, ng, ns,
+                           tilediag);
+    };
+    if (ng <= 64) go(StripInt<1>{});
+    else if (ng <= 128) go(StripInt<2>{});
+    else if (ng <= 192) go(StripInt<3>{});
+    else if (ng <= 256) go(StripInt<4>{});
+    else go(StripInt<8>{});
 }
 template <int T, int G, bool PREF>
 static void launch_adi_fused_t(hipStream_t s, int ns, double2 *field, double2 *work,

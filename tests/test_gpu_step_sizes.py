@@ -127,3 +127,33 @@ def test_column_strips_mixed(ngrid, delz):
     assert err < 2.5 * 2.0 ** -24
     assert np.max(np.abs(d["power"] / d["power"].sum() - w / w.sum())) < 1e-6
     ctx.close()
+
+
+@pytest.mark.parametrize("delz", [0.004, 0.2, 2.0, 40.0, 300.0])
+@pytest.mark.parametrize("ngrid", [3, 4, 31, 63, 64, 65, 128, 129, 192, 193, 256, 257, 300])
+def test_lines(ngrid, delz):
+    """The line kernels (adi_kernel 0) at the edges of a lane's cells (64, 128,
+    192, 256 columns) and of the blocks of four columns, for step sizes whose
+    convolution needs 8 terms to many times the line's length (its distances
+    taken modulo the period) and one that goes to Thomas' sweeps, against the
+    oracle: two steps of the single step's 1e-13 bar, and the field sums."""
+    gridmax = 0.5e-3 * (ngrid - 1) / 150
+    sim = H.make_state([256, 512, 0], ngrid=ngrid, gridmax=gridmax, timerun=False)
+    rng = np.random.default_rng(ngrid)
+    sim.theta += 0.3 * np.sin(sim.theta)
+    sim.field[:] = rng.normal(size=sim.field.shape) * 1e9
+    ctx = H.to_gpu(sim)
+    ctx.set_schedule("adi_kernel", 0)
+    st = H.steps(1, 2)
+    one = H.gsteps(st)[0]
+    for _ in range(2):
+        ctx.field_track(one, delz)
+        H.oracle_call("orc_field_advance", sim, C.byref(st[0]), C.c_double(delz))
+    f, _ = ctx.download_field()
+    err = np.max(np.abs(f - sim.field)) / np.max(np.abs(sim.field))
+    d = ctx.diag()
+    w = (sim.field ** 2).sum(axis=2).sum(axis=1)
+    print(f"  {ngrid}^2, delz {delz}: {err:.2e}", flush=True)
+    assert err < 2e-13
+    assert np.max(np.abs(d["power"] / d["power"].sum() - w / w.sum())) < 1e-12
+    ctx.close()
