@@ -155,8 +155,11 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm_bf16(GemmArgs g, int vecA
 
 // column sums of d [rows][ch] (ch <= 256): stage 1, block b sums rows
 // b, b + nblk, ... into part[b][ch] (coalesced: lane -> (row, channel));
-// stage 2 adds the nblk partials in block order
-constexpr int kColBlocks = 256;
+// stage 2 adds the nblk partials, a block per channel.  Bound by loads in
+// flight: four blocks a CU with eight rows under way in each (365 k rows of 32
+// channels 6 us, where one block a CU and a row at a time took 45), and in
+// stage 2 four partials for each of 256 lanes (4.8 us; one lane adding 256 took 10).
+constexpr int kColBlocks = 1024;
 __global__ void __launch_bounds__(256) k_colsum_part(const float *d, long long rows, int ch, double *part) {
     __shared__ double red[256];
     const int t = threadIdx.x;
@@ -164,8 +167,17 @@ __global__ void __launch_bounds__(256) k_colsum_part(const float *d, long long r
     double s = 0;
     if (t < rpb * ch) {
         const int c = t % ch;
-        for (long long r = (long long)blockIdx.x * rpb + t / ch; r < rows; r += (long long)kColBlocks * rpb)
-            s += d[r * ch + c];
+        const float *p = d + c;
+        const long long step = (long long)kColBlocks * rpb;
+        long long r = (long long)blockIdx.x * rpb + t / ch;
+        for (; r + 7 * step < rows; r += 8 * step) {
+            float v[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) v[q] = p[(r + q * step) * ch];
+#pragma unroll
+            for (int q = 0; q < 8; q++) s += v[q];
+        }
+        for (; r < rows; r += step) s += p[r * ch];
     }
     red[t] = s;
     __syncthreads();
@@ -175,22 +187,37 @@ __global__ void __launch_bounds__(256) k_colsum_part(const float *d, long long r
         part[(long long)blockIdx.x * ch + t] = acc;
     }
 }
-__global__ void k_colsum_fin(const double *part, int ch, float *out) {
-    const int c = blockIdx.x * 64 + threadIdx.x;
-    if (c >= ch) return;
-    double s = 0;
-    for (int b = 0; b < kColBlocks; b++) s += part[(long long)b * ch + c];
-    out[c] = (float)s;
+__global__ void __launch_bounds__(256) k_colsum_fin(const double *part, int ch, float *out) {
+    __shared__ double red[4];
+    const int c = blockIdx.x, t = threadIdx.x;
+    double v[kColBlocks / 256], s = 0;
+#pragma unroll
+    for (int q = 0; q < kColBlocks / 256; q++) v[q] = part[(long long)(t + 256 * q) * ch + c];
+#pragma unroll
+    for (int q = 0; q < kColBlocks / 256; q++) s += v[q];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if ((t & 63) == 0) red[t >> 6] = s;
+    __syncthreads();
+    if (t == 0) out[c] = (float)(red[0] + red[1] + red[2] + red[3]);
 }
 
 // sum of nz partial blocks of n floats: blockIdx.y = g adds blocks
-// [g zc, min((g + 1) zc, nz)) into out[g][n]
+// [g zc, min((g + 1) zc, nz)) into out[g][n].  Eight loads under way at a time
+// (4.9 us a launch, 12 and 9 with one).
 __global__ void k_reduce_parts(const float *parts, int nz, int zc, long long n, float *out) {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    const int z0 = blockIdx.y * zc, z1 = min(z0 + zc, nz);
+    int z = blockIdx.y * zc;
+    const int z1 = min(z + zc, nz);
     float s = 0;
-    for (int z = z0; z < z1; z++) s += parts[(long long)z * n + i];
+    for (; z + 8 <= z1; z += 8) {
+        float v[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = parts[(long long)(z + q) * n + i];
+#pragma unroll
+        for (int q = 0; q < 8; q++) s += v[q];
+    }
+    for (; z < z1; z++) s += parts[(long long)z * n + i];
     out[blockIdx.y * n + i] = s;
 }
 
@@ -601,7 +628,7 @@ void gemm_wgrad(Fno *f, const float *A, const float *B, float *dW, int M, int N,
 
 void colsum(Fno *f, const float *d, long long rows, int ch, float *out) {
     hipLaunchKernelGGL(k_colsum_part, dim3(kColBlocks), dim3(256), 0, f->s, d, rows, ch, f->colpart);
-    hipLaunchKernelGGL(k_colsum_fin, dim3((ch + 63) / 64), dim3(64), 0, f->s, f->colpart, ch, out);
+    hipLaunchKernelGGL(k_colsum_fin, dim3(ch), dim3(256), 0, f->s, f->colpart, ch, out);
 }
 
 void build_wreal(Fno *f) {
