@@ -509,7 +509,7 @@ def main():
     ap.add_argument("--adi-refine", type=int, default=None, choices=(0, 1),
                     help="mixed form: FP64 residual correction in the ADI (default: the library's)")
     ap.add_argument("--mixed-adi", type=int, default=None, choices=(0, 1, 2),
-                    help="mixed form: 0 tile ADI kernel, 1 streaming strips, 2 whole-width streaming "
+                    help="mixed form: 0 tile ADI kernel, 1 streaming strips, 2 FP64 column strips "
                          "(default: the library's)")
     ap.add_argument("--set", action="append", default=[], metavar="[FORM:]KEY=VAL",
                     help="a schedule entry (g4mi_set_schedule) for the measured contexts, e.g. "
