@@ -118,11 +118,11 @@ struct Ctx {
     bool field_diag_fresh = false;
     int ntiles = 0;                    // they are still per tile or strip in d_tilediag, this many a slice
     std::vector<int> zeroed_since_adi;
-    // ADI kernel chosen by the autotuner (-1: not tuned yet) and its timings:
+    // ADI kernel of the last field step (-1: none yet) and the tuner's timings:
     // 0 line by line (wavefronts or Thomas), 1 fused recurrence, 2 fused recurrence with
     // prefetch, 3 banded inverse, 4 column strips
     int adi_kernel = -1;
-    bool adi_fixed = false;               // set by g4mi_set_schedule("adi_kernel", k >= 0)
+    int adi_request = -1;                 // g4mi_set_schedule's "adi_kernel" (-1: the tuner's choice)
     std::map<double, int> adi_choice;     // the tuner's kernel per step size
     float adi_ms[5] = {-1.f, -1.f, -1.f, -1.f, -1.f};
     // spectral solver (FieldSolverFFT) instead of the ADI, with the source
@@ -501,17 +501,6 @@ static int ensure_factors(Ctx *c, double delz) {
     c->adi_delz = delz;
     if ((c->adi.band_m || c->adi.strip >= 0 || c->adi.line.levels) && !c->d_tilediag)
         G4_HIP(hipMalloc(&c->d_tilediag, (size_t)c->ns * adi_sum_blocks(c->ng) * 8 * sizeof(double)));
-    if (!c->adi_fixed) {
-        // the tuner's choice for this step size, or tune it at the next field step
-        auto it = c->adi_choice.find(delz);
-        c->adi_kernel = it != c->adi_choice.end() ? it->second : -1;
-    } else if (c->adi_kernel == 1 || c->adi_kernel == 2) {
-        if (!c->adi.tile) c->adi_kernel = -1;      // re-tune if no longer eligible
-    } else if (c->adi_kernel == 3 && !c->adi.band_m) {
-        c->adi_kernel = -1;
-    } else if (c->adi_kernel == 4 && c->adi.strip < 0) {
-        c->adi_kernel = -1;
-    }
     return G4MI_OK;
 }
 
@@ -746,6 +735,24 @@ static int tune_adi(Ctx *c, const AdiField &a, double2 *field, double2 *work, in
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (scratch) G4_HIP(hipFree(scratch));
+    return G4MI_OK;
+}
+
+// The kernel of this field step: the schedule's request where the step size's
+// tables hold it, else the tuner's choice.  Both are held against the tables of
+// this step, since a request may come between two steps of one size and a step
+// size that is no number finds any entry of `choice`.
+static int adi_pick(Ctx *c, const AdiField &a, double delz, std::map<double, int> &choice, double2 *field,
+                    double2 *work, float *ms, int *kind) {
+    *kind = c->adi_request;
+    if (*kind >= 0 && adi_eligible(a, *kind)) return G4MI_OK;
+    const auto it = choice.find(delz);
+    if (it != choice.end() && adi_eligible(a, it->second)) {
+        *kind = it->second;
+        return G4MI_OK;
+    }
+    G4_TRY(tune_adi(c, a, field, work, kind, ms));
+    if (delz == delz) choice[delz] = *kind;
     return G4MI_OK;
 }
 
@@ -1003,19 +1010,9 @@ static int harmonics_track(Ctx *c, const g4mi_step_params &st, double delz, bool
         d.ngrid = h.ng;
         deposit_field(c, split, d, h.d_src, h.d_box, h.split, false);
         const AdiField a{h.ng, &p, h.d_src, h.d_box, nullptr, nullptr};
-        // the fundamental's rules: a fixed kernel where it is eligible, the
-        // tuner's choice for the step size otherwise
-        int kind = c->adi_fixed && adi_eligible(a, c->adi_kernel) ? c->adi_kernel : -1;
-        if (kind < 0) {
-            auto it = h.choice.find(delz);
-            if (it == h.choice.end()) {
-                float ms[5];
-                G4_TRY(tune_adi(c, a, h.d_field, h.d_work, &kind, ms));
-                h.choice[delz] = kind;
-            } else {
-                kind = it->second;
-            }
-        }
+        int kind = 0;
+        float ms[5];
+        G4_TRY(adi_pick(c, a, delz, h.choice, h.d_field, h.d_work, ms, &kind));
         adi_launch(c, kind, a, h.d_field, h.d_work);
         if (kind >= 3) std::swap(h.d_field, h.d_work);  // result is in the other buffer
     }
@@ -1057,10 +1054,7 @@ static int field_track(Ctx *c, const g4mi_step_params &st, double delz, bool dep
         return G4MI_OK;
     }
     const AdiField a{c->ng, &c->adi, c->d_src, c->d_box, c->d_tilediag, c->d_diag_f};
-    if (c->adi_kernel < 0) {
-        G4_TRY(tune_adi(c, a, c->d_field, c->d_work, &c->adi_kernel, c->adi_ms));
-        c->adi_choice[c->adi_delz] = c->adi_kernel;
-    }
+    G4_TRY(adi_pick(c, a, delz, c->adi_choice, c->d_field, c->d_work, c->adi_ms, &c->adi_kernel));
     adi_launch(c, c->adi_kernel, a, c->d_field, c->d_work);
     c->ntiles = c->adi_kernel == 4 ? strip_dims(c->adi.strip).count(c->ng) : c->adi_kernel == 3 ? adi_band_tiles(c->ng)
                 : c->adi_kernel == 0 && c->adi.line.levels ? line_blocks(c->ng) : 0;
@@ -3394,8 +3388,7 @@ int g4mi_set_schedule(g4mi_ctx *h, const char *name, int value) {
     if (!h || !name) return G4MI_E_ARG;
     Ctx *c = &h->c;
     if (std::string(name) == "adi_kernel" && value >= -1 && value <= 4) {
-        c->adi_kernel = value;
-        c->adi_fixed = value >= 0;
+        c->adi_kernel = c->adi_request = value;
         if (value < 0) {
             c->adi_choice.clear();
             for (Ctx::HField &hf : c->hf) hf.choice.clear();

@@ -157,3 +157,50 @@ def test_lines(ngrid, delz):
     assert err < 2e-13
     assert np.max(np.abs(d["power"] / d["power"].sum() - w / w.sum())) < 1e-12
     ctx.close()
+
+
+@pytest.mark.parametrize("kernel", [1, 2, 3, 4])
+def test_request_between_steps_of_one_size(kernel):
+    """A kernel asked for between two steps of a size that it does not hold
+    leaves the tuner's choice there (with and without a harmonic field), and
+    is taken at the next step size that it does hold."""
+    sim = H.make_state([256] * 4, ngrid=151, seed_power=1e6, timerun=False)
+    # bunched at the harmonic: an unmodulated quiet beam's source is rounding noise
+    sim.theta[:] += 0.2 * np.sin(3 * sim.theta)
+    sim.add_harmonics([(3, 151, sim.s.gridmax)])
+    sim.hfields[0][:] = np.random.default_rng(kernel).normal(size=sim.hfields[0].shape) * 1e10
+    ctx = H.to_gpu(sim)
+    ctx.add_harmonic(3, 151, sim.s.gridmax)
+    ctx.upload_harmonic(0, sim.hfields[0])
+    st = H.steps(1, 2)
+    one = H.gsteps(st)[0]
+    for k, delz in enumerate((5.0, 5.0, 0.015)):
+        ctx.field_track(one, delz)
+        H.oracle_call("orc_field_advance", sim, C.byref(st[0]), C.c_double(delz))
+        if k == 0:
+            ctx.set_schedule("adi_kernel", kernel)
+        else:
+            assert (ctx.schedule()["adi_kernel"] == kernel) == (delz == 0.015)
+        f, _ = ctx.download_field()
+        assert np.max(np.abs(f - sim.field)) < 1e-13 * 3 * np.max(np.abs(sim.field))
+        e = np.max(np.abs(ctx.download_harmonic(0) - sim.hfields[0])) / np.max(np.abs(sim.hfields[0]))
+        assert e < 4e-13
+    ctx.close()
+
+
+def test_step_size_that_is_no_number():
+    """A step of NaN gives the oracle's NaN field, whatever step sizes came
+    before it, and leaves their choices alone."""
+    sim = H.make_state([256] * 3, ngrid=65, seed_power=1e6, timerun=False)
+    ctx = H.to_gpu(sim)
+    one = H.gsteps(H.steps(1, 2))[0]
+    for kernel in (-1, 3, 4):
+        ctx.set_schedule("adi_kernel", kernel)
+        ctx.upload_field(sim.field, 0)
+        for delz in (0.015, 0.03):
+            ctx.field_track(one, delz)
+        before = ctx.schedule()["adi_by_delz"]
+        ctx.field_track(one, float("nan"))
+        assert np.all(np.isnan(ctx.download_field()[0]))
+        assert ctx.schedule()["adi_by_delz"] == before
+    ctx.close()
