@@ -1679,6 +1679,8 @@ static int split_step(Ctx *c, const g4mi_step_params &st, double gamma0, double 
     if (f.chicane) f.r56 = chicane_r56(st.chic_angle, st.chic_lb, st.chic_ld, c->lambda0, gamma0);
     f.gamma0 = gamma0;
     f.d.enabled = st.aw > 0 ? 1 : 0;
+    f.d.gridmax = c->gridmax;
+    for (const Ctx::HField &h : c->hf) f.d.gridmax = std::max(f.d.gridmax, h.gridmax);
     f.d.ax = st.ax;
     f.d.ay = st.ay;
     f.d.kx = st.kx;

@@ -76,7 +76,7 @@ void launch_fp64_main(hipStream_t s, int ns, const long long *off, double *g, do
 struct TrackParams {
     PushParams p;
     TransParams t1, t2;
-    DepositParams d;               // the fundamental's (its enabled and faw2 terms)
+    DepositParams d;               // the fundamental's (its enabled and faw2 terms); gridmax: the widest field's
     double r56, gamma0;            // R56 (chicane != 0)
     int chicane, first;
 };

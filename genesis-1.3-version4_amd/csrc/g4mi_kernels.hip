@@ -1280,8 +1280,8 @@ __global__ void __launch_bounds__(kFuseNT, GEN ? 2 : 4) k_fp64_main(const long l
 // k_track: push (k_push), R56 (k_r56) and second transverse half step, before
 // them the first one where no space-charge pass needs its positions first;
 // the sums of DiagBeam per block (part[8 block]) and the slice's largest
-// sqrt(faw2) / gamma (pmax, the deposit's fixed-point scale: a maximum, so
-// the order of the atomics does not matter).
+// sqrt(faw2) / gamma on the widest grid (pmax, the deposit's fixed-point scale:
+// a maximum, so the order of the atomics does not matter).
 // k_deposit_part: the source of `chunk` particles in an LDS tile over their
 // own footprint, its cells then added to the slice's fixed-point plane with
 // integer atomics (any order, the same bits); particles spread over more cells
@@ -1331,7 +1331,7 @@ __global__ void __launch_bounds__(256) k_track(const int *__restrict__ blk_slice
         v[5] = yi * yi;
         v[6] = c;
         v[7] = s;
-        if (f.d.enabled) {
+        if (f.d.enabled && fabs(xi) < f.d.gridmax && fabs(yi) < f.d.gridmax) {  // some field takes its charge
             const double dx = xi - f.d.ax, dy = yi - f.d.ay;
             const double faw2 = (1 + f.d.kx * dx * dx + f.d.ky * dy * dy + 2 * (f.d.gradx * dx + f.d.grady * dy));
             m = fmax(0.0, sqrt(faw2) / fabs(gamma));

@@ -131,3 +131,33 @@ def test_one4one_records_across_sorts():
     assert np.array_equal(ctx.slices()[0], ref.slices()[0])
     ctx.close()
     ref.close()
+
+
+def test_slow_particle_leaving_the_grid():
+    """A slow particle that crosses the axis at the push and is 100 m away
+    after the second half step, in a strong gradient: sqrt(faw2) / gamma is a
+    million times the others' there, but it deposits nothing, so it takes
+    nothing from the resolution of the others' fixed-point sums."""
+    st = H.steps(1, 2)[:1]
+    s = st[0]
+    s.kx = s.ky = s.gradx = s.ax = s.ay = s.qf = 0.0
+    s.grady = 1e3
+    sim = H.make_state([1024, 512, 256], ngrid=63, gridmax=0.3e-3, timerun=False)
+    sim.theta[:] += 0.3 * np.sin(sim.theta)
+    sim.y *= 0.1
+    gamma, gz = 4.0, 2.6e-4
+    py = np.sqrt(gamma ** 2 - 1 - s.aw ** 2 - gz ** 2)
+    gz = np.sqrt(gamma * gamma - 1 - s.aw * s.aw - py * py)
+    for i in (5, 1030):
+        sim.gamma[i], sim.px[i], sim.py[i], sim.x[i] = gamma, 0.0, py, 0.0
+        sim.y[i] = -py * (0.5 * s.dz) / gz - 2e-4
+    ctx = H.to_gpu(sim)
+    ctx.run(H.gsteps(st), cases.GAMMA0, record=())
+    sim.run(st, cases.GAMMA0, record=("power",))
+    far = sim.y[[5, 1030]]
+    assert np.all(np.isfinite(sim.gamma[[5, 1030]])) and np.all(far > 50), far
+    f, _ = ctx.download_field()
+    e = np.max(np.abs(f - sim.field)) / np.max(np.abs(sim.field))
+    print(f"  field of the other particles: {e:.2e}", flush=True)
+    assert e < 1e-12
+    ctx.close()
