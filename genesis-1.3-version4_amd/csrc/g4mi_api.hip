@@ -180,10 +180,10 @@ struct Ctx {
     std::vector<PendingRecord> pend;
     // one4one beams: Beam::sort at sort markers, with its work buffers
     bool one4one = false;
-    // the step's particle passes as two fused kernels (schedule "fp64_fused":
-    // 1 on, 0 off, -1 on when the window has at least kFuseMinSlices slices,
-    // since the fused kernels run one workgroup per slice while the separate
-    // ones spread a slice's particles over blocks of 256)
+    // the step's particle passes (schedule "fp64_fused"): 1 as two fused kernels
+    // of one workgroup per slice, 0 as the separate kernels, -1 fused when the
+    // window has at least kFuseMinSlices slices and else over blocks of the
+    // particles (split_step)
     int fuse64 = -1;
     double *d_beamsum = nullptr;           // beam sums of the last fused step [8 ns]
     int4 *d_pbox = nullptr;                // in-grid footprint per slice after the first half step
@@ -1662,9 +1662,10 @@ static int split_alloc(Ctx *c) {
 
 // Whether a step takes the split path: a window too small to fill the chip
 // with a workgroup per slice (the fused kernels' rule), no energy kicks
-// between the push and R56, no sort between the beam and the field track.
+// between the push and R56, no sort between the beam and the field track, and
+// the separate kernels not asked for.
 static bool splittable(const Ctx *c, const g4mi_step_params &st) {
-    if (c->split_off || c->ns >= kFuseMinSlices || !c->has_beam || !c->has_field) return false;
+    if (c->split_off || c->fuse64 == 0 || c->ns >= kFuseMinSlices || !c->has_beam || !c->has_field) return false;
     if (c->incoh && st.aw > 0 && (c->incoh_loss || c->incoh_spread)) return false;
     return !c->d_wake && !((st.marker & 4) && c->one4one);
 }
@@ -3484,14 +3485,16 @@ int g4mi_get_schedule(g4mi_ctx *h, char *buf, int len) {
         snprintf(buf, (size_t)len, "%s", tmp);
         return G4MI_OK;
     }
+    const g4mi_step_params plain{};
+    const char *passes = fp64_fusable(c, plain) ? "fused" : splittable(c, plain) ? "split" : "separate";
     if (c->fft) {
         snprintf(tmp, sizeof(tmp),
                  "{\"field_solver\": \"fft\", \"source_filter\": %d, \"gemm_tile\": %d, \"gemm_variant\": %d, "
                  "\"gemm_tuned_ms\": [%.4f, %.4f, %.4f, %.4f], \"propagation\": \"%s\", "
-                 "\"conv_length\": %d, \"conv_tuned_ms\": %.4f, \"fp64_fused\": %d}",
+                 "\"conv_length\": %d, \"conv_tuned_ms\": %.4f, \"fp64_fused\": %d, \"particle_passes\": \"%s\"}",
                  c->fft_filter, cgemm_tile(c->ng), c->fft_variant, c->fft_ms[0], c->fft_ms[1], c->fft_ms[2],
                  c->fft_ms[3], c->fft_prop == 1 ? "fft-conv" : (c->fft_prop == 0 ? "gemm" : "untuned"),
-                 fft_conv_length(c->ng), c->fft_conv_ms, fp64_fuse_on(c) ? 1 : 0);
+                 fft_conv_length(c->ng), c->fft_conv_ms, fp64_fuse_on(c) ? 1 : 0, passes);
         snprintf(buf, (size_t)len, "%s", tmp);
         return G4MI_OK;
     }
@@ -3505,10 +3508,10 @@ int g4mi_get_schedule(g4mi_ctx *h, char *buf, int len) {
     snprintf(tmp, sizeof(tmp),
              "{\"field_solver\": \"adi\", \"adi_kernel\": %d, \"adi\": \"%s\", \"adi_window\": %d, "
              "\"adi_band_m\": %d, \"adi_tuned_ms\": [%.4f, %.4f, %.4f, %.4f, %.4f], \"adi_by_delz\": %s, "
-             "\"fp64_fused\": %d}",
+             "\"fp64_fused\": %d, \"particle_passes\": \"%s\"}",
              c->adi_kernel, c->adi_kernel >= 0 ? names[c->adi_kernel] : "untuned", c->adi.tile,
              c->adi.band_m, c->adi_ms[0], c->adi_ms[1], c->adi_ms[2], c->adi_ms[3], c->adi_ms[4], bydz.c_str(),
-             fp64_fuse_on(c) ? 1 : 0);
+             fp64_fuse_on(c) ? 1 : 0, passes);
     snprintf(buf, (size_t)len, "%s", tmp);
     return G4MI_OK;
 }

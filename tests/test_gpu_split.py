@@ -161,3 +161,49 @@ def test_slow_particle_leaving_the_grid():
     print(f"  field of the other particles: {e:.2e}", flush=True)
     assert e < 1e-12
     ctx.close()
+
+
+@pytest.mark.parametrize("counts,value,passes", [
+    ([256] * 10, -1, "split"), ([256] * 10, 1, "fused"), ([256] * 10, 0, "separate"),
+    ([64] * 256, -1, "fused"), ([64] * 256, 0, "separate")])
+def test_particle_passes_by_request(counts, value, passes):
+    """fp64_fused 0 runs the separate kernels on any window: a record's beam
+    sums are then k_diag_beam's bits, which g4mi_diag gives for the same
+    particles."""
+    st = H.steps(1, 2)[:2]
+    sim = H.make_state(counts, ngrid=41, gridmax=0.3e-3, seed_power=1e6)
+    ctx = H.to_gpu(sim)
+    ctx.set_schedule("fp64_fused", value)
+    assert ctx.schedule()["particle_passes"] == passes
+    keys = ("bunching", "energy", "xsize", "ysize")
+    g = ctx.run(H.gsteps(st), cases.GAMMA0, record=keys)
+    d = ctx.diag()
+    for k in keys:
+        if passes == "separate":
+            assert np.array_equal(g[k][-1], d[k]), k
+        else:
+            assert H.rel_err(g[k][-1], d[k]) < 1e-10, k
+    ctx.close()
+
+
+def test_separate_kernels_on_a_wide_window_with_a_harmonic():
+    """256 slices with a harmonic field run the separate kernels by
+    themselves: against the oracle, and the same bits twice."""
+    out = []
+    for _ in range(2):
+        sim = H.make_state([64, 0, 132, 64] * 64, ngrid=31, gridmax=0.3e-3, seed_power=1e6, timerun=False)
+        sim.theta[:] += 0.2 * np.sin(3 * sim.theta)
+        sim.add_harmonics([(3, 33, 0.25e-3)])
+        sim.hfields[0][:] = np.random.default_rng(2).normal(size=sim.hfields[0].shape) * 1e10
+        ctx = H.to_gpu(sim)
+        ctx.add_harmonic(3, 33, 0.25e-3)
+        ctx.upload_harmonic(0, sim.hfields[0])
+        assert ctx.schedule()["particle_passes"] == "separate"
+        _check(sim, ctx, H.steps(1, 4)[:4])
+        h = ctx.download_harmonic(0)
+        assert np.max(np.abs(h - sim.hfields[0])) <= 1e-12 * np.max(np.abs(sim.hfields[0]))
+        out.append((ctx.download_beam(), ctx.download_field()[0], h))
+        ctx.close()
+    for k in BEAM:
+        assert np.array_equal(out[0][0][k], out[1][0][k]), k
+    assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][2], out[1][2])
