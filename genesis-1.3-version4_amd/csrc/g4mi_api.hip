@@ -40,7 +40,7 @@ struct AdiPlan {
     double2 *fac = nullptr, *band = nullptr;  // one allocation: c | cbet | cwet, the band, strip_k's tables
     int strip = -1;                           // the strip kernel's form; -1: none holds the step size
     StripCoef strip_k{};
-    LineCoef line{};                          // the line kernels' factors (levels 0: Thomas instead)
+    LineCoef line{};                          // the line kernels' factors (levels 0: none hold the step size)
 };
 // The spectral solver's tables for one step size: the convolution's kernel
 // transform and, once a GEMM needs it, the propagator matrix.
@@ -119,8 +119,8 @@ struct Ctx {
     int ntiles = 0;                    // they are still per tile or strip in d_tilediag, this many a slice
     std::vector<int> zeroed_since_adi;
     // ADI kernel of the last field step (-1: none yet) and the tuner's timings:
-    // 0 line by line (wavefronts or Thomas), 1 fused recurrence, 2 fused recurrence with
-    // prefetch, 3 banded inverse, 4 column strips
+    // 0 two-kernel Thomas, 1 fused recurrence, 2 fused recurrence with prefetch,
+    // 3 banded inverse, 4 column strips, 5 line by line
     int adi_kernel = -1;
     int adi_request = -1;                 // g4mi_set_schedule's "adi_kernel" (-1: the tuner's choice)
     std::map<double, int> adi_choice;     // the tuner's kernel per step size
@@ -647,11 +647,15 @@ static bool adi_eligible(const AdiField &a, int kind) {
     if (kind == 1 || kind == 2) return a.p->tile != 0 && a.diag;
     if (kind == 3) return a.p->band_m != 0;
     if (kind == 4) return a.p->strip >= 0;
+    if (kind == 5) return a.p->line.levels != 0;
     return kind == 0;
 }
 
-// One ADI launch of kernel `kind` on field buffer `fin` (the banded kernels
-// write `fout`, the others work in place using `fout` as scratch).
+// The banded kernels and the strips write the other buffer, the others work in
+// place with it as scratch.
+static bool adi_swaps(int kind) { return kind == 3 || kind == 4; }
+
+// One ADI launch of kernel `kind` on field buffer `fin`.
 static void adi_launch(Ctx *c, int kind, const AdiField &a, double2 *fin, double2 *fout) {
     const AdiPlan &p = *a.p;
     const AdiFactors f{p.fac, p.fac + a.ng, p.fac + 2 * a.ng, p.cstep, a.ng};
@@ -662,7 +666,7 @@ static void adi_launch(Ctx *c, int kind, const AdiField &a, double2 *fin, double
                         p.klo, p.khi, a.tilediag, nullptr);
     else if (kind == 1 || kind == 2)
         launch_adi_fused(c->stream, c->ns, fin, fout, a.src, a.box, f, c->first, a.diag, p.tile, kind == 2);
-    else if (p.line.levels)
+    else if (kind == 5)
         launch_adi_lines(c->stream, c->ns, fin, fout, a.src, a.box, p.line, a.ng, c->first, a.tilediag);
     else
         launch_adi(c->stream, c->ns, fin, fout, a.src, a.box, f, c->first);
@@ -693,7 +697,7 @@ static int tune_adi(Ctx *c, const AdiField &a, double2 *field, double2 *work, in
         return G4MI_OK;
     }
     if (!narrow && p.line.levels) {
-        *choice = 0;
+        *choice = 5;
         return G4MI_OK;
     }
     const bool out = adi_eligible(a, 3) || adi_eligible(a, 4);
@@ -1014,7 +1018,7 @@ static int harmonics_track(Ctx *c, const g4mi_step_params &st, double delz, bool
         float ms[5];
         G4_TRY(adi_pick(c, a, delz, h.choice, h.d_field, h.d_work, ms, &kind));
         adi_launch(c, kind, a, h.d_field, h.d_work);
-        if (kind >= 3) std::swap(h.d_field, h.d_work);  // result is in the other buffer
+        if (adi_swaps(kind)) std::swap(h.d_field, h.d_work);  // result is in the other buffer
     }
     G4_HIP(hipGetLastError());
     return G4MI_OK;
@@ -1057,9 +1061,9 @@ static int field_track(Ctx *c, const g4mi_step_params &st, double delz, bool dep
     G4_TRY(adi_pick(c, a, delz, c->adi_choice, c->d_field, c->d_work, c->adi_ms, &c->adi_kernel));
     adi_launch(c, c->adi_kernel, a, c->d_field, c->d_work);
     c->ntiles = c->adi_kernel == 4 ? strip_dims(c->adi.strip).count(c->ng) : c->adi_kernel == 3 ? adi_band_tiles(c->ng)
-                : c->adi_kernel == 0 && c->adi.line.levels ? line_blocks(c->ng) : 0;
-    if (c->adi_kernel >= 3) std::swap(c->d_field, c->d_work);  // result is in the other buffer
-    c->field_diag_fresh = c->adi_kernel != 0 || c->ntiles;
+                : c->adi_kernel == 5 ? line_blocks(c->ng) : 0;
+    if (adi_swaps(c->adi_kernel)) std::swap(c->d_field, c->d_work);  // result is in the other buffer
+    c->field_diag_fresh = c->adi_kernel != 0;
     c->zeroed_since_adi.clear();
     G4_HIP(hipGetLastError());
     if (c->ev) G4_HIP(hipEventRecord(c->ev[7], c->stream));
@@ -3390,7 +3394,7 @@ int g4mi_sort_index_noalloc(g4mi_ctx *h, double slen, int *atar, long long *move
 int g4mi_set_schedule(g4mi_ctx *h, const char *name, int value) {
     if (!h || !name) return G4MI_E_ARG;
     Ctx *c = &h->c;
-    if (std::string(name) == "adi_kernel" && value >= -1 && value <= 4) {
+    if (std::string(name) == "adi_kernel" && value >= -1 && value <= 5) {
         c->adi_kernel = c->adi_request = value;
         if (value < 0) {
             c->adi_choice.clear();
@@ -3466,7 +3470,7 @@ int g4mi_get_schedule(g4mi_ctx *h, char *buf, int len) {
     if (!h || !buf || len < 1) return G4MI_E_ARG;
     Ctx *c = &h->c;
     char tmp[4096];
-    static const char *names[5] = {"thomas", "fused", "fused-prefetch", "band", "band-wide"};
+    static const char *names[6] = {"thomas", "fused", "fused-prefetch", "band", "band-wide", "lines"};
     if (c->precision == G4MI_FP32) {
         std::string bands = "[";
         for (size_t k = 0; k < c->h_binfo.size(); k++)

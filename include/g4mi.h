@@ -238,14 +238,14 @@ int g4mi_sort_index(g4mi_ctx *ctx, double slen, int *atar, long long *moved);
 int g4mi_sort_index_noalloc(g4mi_ctx *ctx, double slen, int *atar, long long *moved);
 
 /* Kernel schedule.  The first field step of each step size takes the ADI
- * kernel that suits its grid, step and number of slices: 0 two kernels over
- * the lines ("thomas": a wavefront per line, Thomas' algorithm where that does
- * not hold the step), 1 and 2 the fused recurrence without and with prefetch,
- * 3 banded inverse in 32x32 tiles, 4 strips of whole columns; 3 against 4
+ * kernel that suits its grid, step and number of slices: 0 Thomas' algorithm
+ * in two kernels, 1 and 2 the fused recurrence without and with prefetch,
+ * 3 banded inverse in 32x32 tiles, 4 strips of whole columns, 5 a wavefront
+ * per line; 3 against 4
  * where either can be the faster, and the recurrences where neither holds the
  * step, are timed (the library's autotuner).  g4mi_set_schedule
- * fixes an entry instead ("adi_kernel": 0..4, -1 re-enables tuning; a
- * kernel not eligible for a step size falls back to the tuner's choice);
+ * fixes an entry instead ("adi_kernel": 0..5, -1 re-enables tuning; a step
+ * size that the kernel does not hold takes the tuner's choice);
  * g4mi_get_schedule writes the current choice
  * and the measured timings as a JSON object into buf.  "fp64_fused": the step's
  * particle passes where the step allows them, 1 as two fused kernels (one

@@ -35,7 +35,7 @@ def test_more_step_sizes_than_kept(solver, ngrid):
     ctx.close()
 
 
-@pytest.mark.parametrize("kernel", [-1, 0, 3, 4])
+@pytest.mark.parametrize("kernel", [-1, 0, 3, 4, 5])
 @pytest.mark.parametrize("ngrid", [31, 32, 65, 97])
 def test_harmonic_field_in_each_adi_kernel(kernel, ngrid):
     """A third-harmonic field on its own grid (at, below and above the edges
@@ -129,26 +129,27 @@ def test_column_strips_mixed(ngrid, delz):
     ctx.close()
 
 
-@pytest.mark.parametrize("delz", [0.004, 0.2, 2.0, 40.0, 300.0])
+@pytest.mark.parametrize("delz", [0.004, 0.2, 2.0, 40.0, 300.0, 4000.0])
 @pytest.mark.parametrize("ngrid", [3, 4, 31, 63, 64, 65, 128, 129, 192, 193, 256, 257, 300])
 def test_lines(ngrid, delz):
-    """The line kernels (adi_kernel 0) at the edges of a lane's cells (64, 128,
+    """The line kernels (adi_kernel 5) at the edges of a lane's cells (64, 128,
     192, 256 columns) and of the blocks of four columns, for step sizes whose
     convolution needs 8 terms to many times the line's length (its distances
-    taken modulo the period) and one that goes to Thomas' sweeps, against the
-    oracle: two steps of the single step's 1e-13 bar, and the field sums."""
+    taken modulo the period) and one that they leave to Thomas' sweeps, against
+    the oracle: two steps of the single step's 1e-13 bar, and the field sums."""
     gridmax = 0.5e-3 * (ngrid - 1) / 150
     sim = H.make_state([256, 512, 0], ngrid=ngrid, gridmax=gridmax, timerun=False)
     rng = np.random.default_rng(ngrid)
     sim.theta += 0.3 * np.sin(sim.theta)
     sim.field[:] = rng.normal(size=sim.field.shape) * 1e9
     ctx = H.to_gpu(sim)
-    ctx.set_schedule("adi_kernel", 0)
+    ctx.set_schedule("adi_kernel", 5)
     st = H.steps(1, 2)
     one = H.gsteps(st)[0]
     for _ in range(2):
         ctx.field_track(one, delz)
         H.oracle_call("orc_field_advance", sim, C.byref(st[0]), C.c_double(delz))
+    assert ctx.schedule()["adi"] == ("lines" if delz < 1000 else "thomas" if ngrid > 8 else "band")
     f, _ = ctx.download_field()
     err = np.max(np.abs(f - sim.field)) / np.max(np.abs(sim.field))
     d = ctx.diag()
@@ -157,6 +158,40 @@ def test_lines(ngrid, delz):
     assert err < 2e-13
     assert np.max(np.abs(d["power"] / d["power"].sum() - w / w.sum())) < 1e-12
     ctx.close()
+
+
+@pytest.mark.parametrize("delz", [0.015, 0.4, 2.0])
+@pytest.mark.parametrize("ngrid", [31, 151, 255])
+def test_thomas_by_request(ngrid, delz):
+    """adi_kernel 0 runs the reference's recurrence, for the fundamental and a
+    harmonic field, whatever other kernels hold the step size: its fields
+    differ from the lines' by rounding, not by nothing."""
+    out = []
+    for kernel in (0, 5):
+        sim = H.make_state([256] * 2, ngrid=ngrid, gridmax=0.5e-3 * (ngrid - 1) / 150, timerun=False)
+        sim.theta[:] += 0.2 * np.sin(3 * sim.theta)
+        sim.add_harmonics([(3, ngrid, sim.s.gridmax)])
+        rng = np.random.default_rng(ngrid)
+        for f in (sim.field, sim.hfields[0]):
+            f[:] = rng.normal(size=f.shape) * 1e10
+        ctx = H.to_gpu(sim)
+        ctx.add_harmonic(3, ngrid, sim.s.gridmax)
+        ctx.upload_harmonic(0, sim.hfields[0])
+        ctx.set_schedule("adi_kernel", kernel)
+        st = H.steps(1, 2)
+        ctx.field_track(H.gsteps(st)[0], delz)
+        H.oracle_call("orc_field_advance", sim, C.byref(st[0]), C.c_double(delz))
+        assert ctx.schedule()["adi"] == ("thomas" if kernel == 0 else "lines")
+        got = (ctx.download_field()[0], ctx.download_harmonic(0))
+        d = ctx.diag()
+        ctx.close()
+        for f, ref in zip(got, (sim.field, sim.hfields[0])):
+            assert np.max(np.abs(f - ref)) < 1e-13 * np.max(np.abs(ref))
+        w = (sim.field ** 2).sum(axis=2).sum(axis=1)
+        assert np.max(np.abs(d["power"] / d["power"].sum() - w / w.sum())) < 1e-12
+        out.append(got)
+    for a, b in zip(*out):
+        assert not np.array_equal(a, b)
 
 
 @pytest.mark.parametrize("kernel", [1, 2, 3, 4])
@@ -182,7 +217,7 @@ def test_request_between_steps_of_one_size(kernel):
         else:
             assert (ctx.schedule()["adi_kernel"] == kernel) == (delz == 0.015)
         f, _ = ctx.download_field()
-        assert np.max(np.abs(f - sim.field)) < 1e-13 * 3 * np.max(np.abs(sim.field))
+        assert np.max(np.abs(f - sim.field)) < 1e-13 * 3 * np.max(np.abs(sim.field)), k
         e = np.max(np.abs(ctx.download_harmonic(0) - sim.hfields[0])) / np.max(np.abs(sim.hfields[0]))
         assert e < 4e-13
     ctx.close()
