@@ -172,12 +172,12 @@ def roofline(cfg, kt, ntot, precision=g4mi.FP64, schedule=None):
     gbs = per[name] / (ms * 1e-3) / 1e9
     dev = KERNEL_OF["fp64_fused" if fused else precision].get(name)
     if name == "adi" and precision == g4mi.FP32 and schedule:
-        dev = {"band32-wide": "k_mix_adi_strip", "band32-stream": "k_mix_adi_stream",
+        dev = {"strips": "k_mix_adi_strip", "band32-stream": "k_mix_adi_stream",
                "band32-tile": "k_mix_adi<"}.get(schedule.get("adi"), dev)
     if name == "adi" and precision == g4mi.FP64 and schedule:
         # the ADI kernel the tuner chose for the undulator step (the timed steps)
         und = (schedule.get("adi_by_delz") or {}).get(f"{W.DELZ:.6g}", schedule.get("adi"))
-        dev = {"band": "k_adi_band", "band-wide": "k_adi_strip"}.get(und)  # traffic rows: banded kernels
+        dev = {"band": "k_adi_band", "strips": "k_adi_strip"}.get(und)  # the kernels with traffic rows
     traffic = measured_traffic(cfg["name"], dev) if dev else None
     return name, dict(bound="hbm", achieved=round(gbs, 1), peak=HBM_PEAK_GBS, unit="GB/s",
                       frac=round(gbs / HBM_PEAK_GBS, 4),
@@ -502,14 +502,15 @@ def main():
     ap.add_argument("--cpu-steps", type=int, default=2)
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--adi-kernel", type=int, default=-1,
-                    help="fix the ADI kernel (0 Thomas, 1 fused, 2 fused+prefetch, 3 banded); "
+                    help="fix the ADI kernel (0 Thomas, 1 fused, 2 fused+prefetch, 3 banded, "
+                         "4 column strips, 5 lines); "
                          "default: autotuned")
     ap.add_argument("--field-solver", choices=("adi", "fft"), default="adi",
                     help="FP64 form: the ADI (default) or the spectral field solver")
     ap.add_argument("--adi-refine", type=int, default=None, choices=(0, 1),
-                    help="mixed form: FP64 residual correction in the ADI (default: the library's)")
+                    help="mixed form: FP64 residual correction of the FP32 band ADI (default: the library's)")
     ap.add_argument("--mixed-adi", type=int, default=None, choices=(0, 1, 2),
-                    help="mixed form: 0 tile ADI kernel, 1 streaming strips, 2 FP64 column strips "
+                    help="mixed form: 0 FP32 band in tiles, 1 streaming, 2 FP64 column strips "
                          "(default: the library's)")
     ap.add_argument("--set", action="append", default=[], metavar="[FORM:]KEY=VAL",
                     help="a schedule entry (g4mi_set_schedule) for the measured contexts, e.g. "
@@ -569,8 +570,13 @@ def main():
     if prec == g4mi.FP64:
         dtype = "f64"
     else:
-        refine = m["schedule"].get("adi_refine", 0)
-        dtype = "f32 (f64 slice phase base, f64 sums" + (", f64 ADI residual correction)" if refine else ")")
+        if m["schedule"].get("adi") == "strips":
+            adi = ("FP64 ADI arithmetic on the FP32 field", "f64 ADI arithmetic")
+        elif m["schedule"].get("adi_refine", 0):
+            adi = ("FP64 ADI residual correction", "f64 ADI residual correction")
+        else:
+            adi = ("no FP64 ADI residual correction", "f32 ADI")
+        dtype = f"f32 (f64 slice phase base, f64 sums, {adi[1]})"
     out = {
         "metric": "macroparticle-steps/s",
         "value": main_line["value"],
@@ -585,9 +591,7 @@ def main():
         "dtype": dtype,
         "data": "synthetic: Hammersley quiet loading + shot noise (seed 7), as LoadBeam",
         "config": {"workload": W.describe(cfg) +
-                   ("" if prec == g4mi.FP64 else
-                    (", FP64 ADI residual correction" if m["schedule"].get("adi_refine", 0)
-                     else ", no FP64 ADI residual correction")),
+                   ("" if prec == g4mi.FP64 else ", " + adi[0]),
                    "slices": cfg["nslice"], "macroparticles": m["ntot"], "ngrid": cfg["ngrid"],
                    "precision": cfg["precision"], "parallelism": "single GPU"},
         "field_cell_updates_per_s": main_line["field_cell_updates_per_s"],

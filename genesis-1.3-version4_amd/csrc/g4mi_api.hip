@@ -228,7 +228,7 @@ struct Ctx {
     double2 *m_strip = nullptr;            // the strip kernel's tables, kMixMaxBands of 2 ng + kStripPad
     bool m_refine = true;                  // FP64 residual correction in the ADI (schedule "adi_refine")
     bool m_graphs = true;                  // replay captured step graphs
-    int m_adi_mode = kAdiWide;             // mixed ADI kernel (schedule "mixed_adi"): tile 0, strips 1, wide 2
+    int m_adi_mode = kAdiWide;             // mixed ADI kernel (schedule "mixed_adi"): FP32 band in tiles 0, streaming 1, column strips 2
     int m_main_nt = 384;                   // threads per slice of the main kernel ("main_nt")
     int m_main_lds = 0;                    // its LDS region: 0 = 68 KiB, 1 = 44 KiB, 2 = 32 KiB ("main_lds")
     bool m_persistent = false;             // the whole step as one cooperative launch ("persistent")
@@ -2251,7 +2251,7 @@ static int mix_tune_step(Ctx *c, const MixKey &key) {
                      "{\"main_ms\": {\"384/68K\": %.4f, \"256/68K\": %.4f, \"512/68K\": %.4f, "
                      "\"384/44K\": %.4f, \"256/44K\": %.4f, \"512/44K\": %.4f, \"256/32K\": %.4f, "
                      "\"384/32K\": %.4f}, "
-                     "\"adi_ms\": {\"wide\": %.4f, \"strips\": %.4f, \"tile\": %.4f}, "
+                     "\"adi_ms\": {\"strips\": %.4f, \"band32-stream\": %.4f, \"band32-tile\": %.4f}, "
                      "\"step_ms\": {\"graph\": %.4f, \"persistent\": %.4f}}",
                      avg(mm[0], nm[0]), avg(mm[1], nm[1]), avg(mm[2], nm[2]), avg(mm[3], nm[3]),
                      avg(mm[4], nm[4]), avg(mm[5], nm[5]), avg(mm[6], nm[6]), avg(mm[7], nm[7]),
@@ -3470,19 +3470,21 @@ int g4mi_get_schedule(g4mi_ctx *h, char *buf, int len) {
     if (!h || !buf || len < 1) return G4MI_E_ARG;
     Ctx *c = &h->c;
     char tmp[4096];
-    static const char *names[6] = {"thomas", "fused", "fused-prefetch", "band", "band-wide", "lines"};
+    static const char *names[6] = {"thomas", "fused", "fused-prefetch", "band", "strips", "lines"};
     if (c->precision == G4MI_FP32) {
         std::string bands = "[";
         for (size_t k = 0; k < c->h_binfo.size(); k++)
             bands += (k ? ", " : "") + std::to_string(c->h_binfo[k].m) + "/" + std::to_string(c->band_tmpl[k]);
         bands += "]";
+        // the persistent launch streams the FP32 band whatever the other launches run
+        const int adi = c->m_adi_mode == kAdiWide && c->m_persistent ? kAdiStrips : c->m_adi_mode;
         snprintf(tmp, sizeof(tmp),
                  "{\"precision\": \"fp32\", \"adi\": \"%s\", \"adi_refine\": %d, "
                  "\"main_nt\": %d, \"main_lds_kib\": %d, \"persistent\": %d, \"autotune\": %d, \"tuned\": %d, "
                  "\"graphs\": %d, \"fuse_front\": %d, \"bands_m_over_template\": \"%s\", \"graphs_captured\": %d, "
                  "\"tuning\": %s, \"fno_skipped_steps\": %lld}",
-                 c->m_adi_mode == kAdiWide ? "band32-wide" : c->m_adi_mode == kAdiStrips ? "band32-stream" : "band32-tile",
-                 c->m_refine ? 1 : 0, c->m_main_nt,
+                 adi == kAdiWide ? "strips" : adi == kAdiStrips ? "band32-stream" : "band32-tile",
+                 c->m_refine && adi != kAdiWide ? 1 : 0, c->m_main_nt,
                  (c->m_main_lds == 2 && c->m_main_nt != 512) ? 32 : c->m_main_lds ? 44 : 68, c->m_persistent ? 1 : 0, c->m_autotune ? 1 : 0, c->m_tuned ? 1 : 0, c->m_graphs ? 1 : 0,
                  c->m_fuse_front ? 1 : 0, bands.c_str(), (int)c->m_graph.size(), c->m_tune_log.empty() ? "null" : c->m_tune_log.c_str(),
                  c->fno_skipped);

@@ -40,8 +40,8 @@ def _field_err(ctx, sim):
 def test_mixed_adi_against_oracle(st, refine, mode):
     """Field-only steps (zero current: no source) over undulator, quadrupole
     and drift step sizes (band half widths 3, 4, 6 on 151^2): the FP32 band
-    ADI, with and without the FP64 residual correction, in each kernel
-    (2: whole-width streaming, 1: streaming strips, 0: 32x32 tiles), against
+    ADI, with and without the FP64 residual correction, streaming (1) and in
+    32x32 tiles (0), and the FP64 column strips (2, no correction), against
     the FP64 Thomas ADI of the oracle.  Bound: the FP32 rounding of the
     stored field per step (2^-24 relative) times the step count, with
     margin."""
@@ -59,7 +59,8 @@ def test_mixed_adi_against_oracle(st, refine, mode):
         ctx.step(H.gsteps(st)[i], cases.GAMMA0)
         errs.append(_field_err(ctx, sim))
     sched = ctx.schedule()
-    assert sched["adi"] == {2: "band32-wide", 1: "band32-stream", 0: "band32-tile"}[mode]
+    assert sched["adi"] == {2: "strips", 1: "band32-stream", 0: "band32-tile"}[mode]
+    assert sched["adi_refine"] == (refine if mode < 2 else 0)
     _log(f"  dz {[round(st[i].dz, 3) for i in idx]}\n  field rel err per step {['%.2e' % e for e in errs]}"
          f"\n  schedule {sched}")
     bound = (2.0 if refine else 8.0) * 2.0 ** -24 * len(idx)
@@ -71,11 +72,10 @@ def test_mixed_adi_against_oracle(st, refine, mode):
 def test_mixed_adi_kernels_agree_with_source(st):
     """The three ADI kernels of the mixed form on a SASE window with a
     source, long-range space charge and slippage (10 slices x 1024, 131^2:
-    the whole-width kernel then has idle lanes and a partly filled last
-    wavefront) over 40 steps: records and final field of the whole-width
-    kernel and of the strips against the tile kernel.  All three round the
-    same FP32 band products in a different order only, so they agree to
-    a few FP32 ulps per step."""
+    the last column strip is partly filled) over 40 steps: records and final
+    field of the column strips (FP64 arithmetic) and of the streaming FP32 band
+    (FP64 residual correction) against the tiles.  Each rounds the field to
+    FP32 once a step, so they agree to a few FP32 ulps per step."""
     _log("mixed ADI kernels agree: 10 slices x 1024, 131^2, 40 steps, modes 2, 1, 0")
     out = {}
     for mode in (2, 1, 0):
@@ -332,8 +332,8 @@ def test_mixed_autotuner_picks_a_schedule(st):
     assert sched["tuned"] == 1
     tun = sched["tuning"]
     assert len(tun["main_ms"]) == 8 and all(v > 0 for v in tun["main_ms"].values())
-    assert tun["adi_ms"]["wide"] > 0 and tun["adi_ms"]["strips"] > 0 and tun["step_ms"]["graph"] > 0
-    assert sched["adi"] in ("band32-wide", "band32-stream", "band32-tile")
+    assert tun["adi_ms"]["strips"] > 0 and tun["adi_ms"]["band32-stream"] > 0 and tun["step_ms"]["graph"] > 0
+    assert sched["adi"] in ("strips", "band32-stream", "band32-tile")
     assert sched["main_nt"] in (256, 384, 512) and sched["main_lds_kib"] in (32, 44, 68)
     r = sim.run(st, cases.GAMMA0, record=("power", "bunching"), nsteps=n)
     pg, pr = g["power"][1:].sum(axis=1), r["power"][1:].sum(axis=1)

@@ -203,8 +203,8 @@ def test_deposit_corner_cell_and_mixed_groups(st):
 def test_adi_kernels_and_regimes(delz, kernel):
     """rtmp = dz/(4 ks dx^2) = 3e-3, 3e-2 and 1 on the 151^2 grid: the fused
     recurrence kernels use an 8-cell window, a 16-cell window, or are not
-    eligible; the banded-inverse kernels a half width 7 (tiles and the
-    whole-width stream), 12 (tiles only), or are not eligible.  Every
+    eligible; the banded inverse in tiles a half width 7, 12, or is not
+    eligible, the column strips 7 or 12 terms, or are not eligible.  Every
     eligible kernel agrees with the oracle's Thomas; an ineligible request
     falls back to the autotuner's choice."""
     _log(f"ADI regime delz={delz} kernel={kernel}")
@@ -224,7 +224,7 @@ def test_adi_kernels_and_regimes(delz, kernel):
     assert sch["adi_window"] == {0.015: 8, 0.15: 16, 5.0: 0}[delz]
     assert sch["adi_band_m"] == {0.015: 7, 0.15: 12, 5.0: 0}[delz]
     if kernel == 4 and delz == 0.015:
-        assert sch["adi"] == "band-wide"
+        assert sch["adi"] == "strips"
 
 
 @pytest.mark.parametrize("delz,m", [(0.35, 16), (0.8, 0)])
@@ -255,13 +255,12 @@ def test_adi_band_tiles_wide_halfwidths(delz, m):
 
 @pytest.mark.parametrize("ngrid", [151, 255, 63])
 def test_adi_wide_stream_matches_band_tiles(ngrid):
-    """The whole-width banded ADI evaluates the products of the 32x32-tile
-    banded kernel; a column or row takes the symmetric form of the central
-    band where its own wavefront (stream) or its whole tile (tiles) lies in
-    [klo, khi], so the two differ by the rounding of that choice only: over
-    6 undulator steps with a source the fields agree to 1e-14 and both
-    match the oracle's Thomas."""
-    _log(f"banded ADI: whole-width stream vs tiles, {ngrid}^2, 6 slices, 6 steps")
+    """The column strips (factored convolution in x, windowed Thomas in y)
+    against the 32x32-tile products with the banded inverse: two orders of the
+    same inverse, each within a few roundings of it, so over 6 undulator steps
+    with a source the fields agree to 1e-14 and both match the oracle's
+    Thomas."""
+    _log(f"ADI: column strips vs band tiles, {ngrid}^2, 6 slices, 6 steps")
     st = H.steps()
     out = []
     for kernel in (3, 4):
@@ -271,7 +270,7 @@ def test_adi_wide_stream_matches_band_tiles(ngrid):
         ctx.set_schedule("adi_kernel", kernel)
         r = ctx.run(H.gsteps(st[118:124]), cases.GAMMA0, record=("power",))
         sch = ctx.schedule()
-        assert sch["adi"] == ("band" if kernel == 3 else "band-wide"), sch
+        assert sch["adi"] == ("band" if kernel == 3 else "strips"), sch
         f, first = ctx.download_field()
         out.append((r, f, first))
         ctx.close()
@@ -280,11 +279,11 @@ def test_adi_wide_stream_matches_band_tiles(ngrid):
     assert qa == qb == sim.s.first
     ef = float(np.max(np.abs(fa - fb)) / np.max(np.abs(fa)))
     eo = float(np.max(np.abs(fb - sim.field)) / np.max(np.abs(fa)))
-    _log(f"  field stream vs tiles {ef:.3e}, stream vs oracle {eo:.3e}")
+    _log(f"  field strips vs tiles {ef:.3e}, strips vs oracle {eo:.3e}")
     assert ef < 1e-14 and eo < 1e-12
     ep = H.rel_err(rb["power"], ra["power"])
     eo = H.rel_err(rb["power"], rs["power"])
-    _log(f"  power stream vs tiles {ep:.3e}, stream vs oracle {eo:.3e}")
+    _log(f"  power strips vs tiles {ep:.3e}, strips vs oracle {eo:.3e}")
     assert ep < 1e-13 and eo < 1e-10
 
 

@@ -88,7 +88,7 @@ def test_column_strips(ngrid, delz):
     for _ in range(2):
         ctx.field_track(one, delz)
         H.oracle_call("orc_field_advance", sim, C.byref(st[0]), C.c_double(delz))
-    assert ctx.schedule()["adi"] == "band-wide"
+    assert ctx.schedule()["adi"] == "strips"
     f, _ = ctx.download_field()
     err = np.max(np.abs(f - sim.field)) / np.max(np.abs(sim.field))
     d = ctx.diag()
@@ -118,7 +118,7 @@ def test_column_strips_mixed(ngrid, delz):
     for _ in range(2):
         O.lib().orc_step_all(C.byref(sim.s), C.byref(st[0]), cases.GAMMA0)
         ctx.step(H.gsteps(st)[0], cases.GAMMA0)
-    assert ctx.schedule()["adi"] == "band32-wide"
+    assert ctx.schedule()["adi"] == "strips"
     f, _ = ctx.download_field()
     err = np.max(np.abs(f - sim.field)) / np.max(np.abs(sim.field))
     d = ctx.diag()
