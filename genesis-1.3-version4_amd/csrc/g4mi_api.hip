@@ -663,7 +663,7 @@ static void adi_launch(Ctx *c, int kind, const AdiField &a, double2 *fin, double
         launch_adi_strip(c->stream, c->ns, fin, fout, a.src, a.box, p.strip_k, p.strip, a.ng, c->first, a.tilediag);
     else if (kind == 3)
         launch_adi_band(c->stream, c->ns, fin, fout, a.src, a.box, p.band, p.cstep, a.ng, c->first, p.band_m,
-                        p.klo, p.khi, a.tilediag, nullptr);
+                        p.klo, p.khi, a.tilediag);
     else if (kind == 1 || kind == 2)
         launch_adi_fused(c->stream, c->ns, fin, fout, a.src, a.box, f, c->first, a.diag, p.tile, kind == 2);
     else if (kind == 5)
@@ -685,8 +685,13 @@ static void adi_launch(Ctx *c, int kind, const AdiField &a, double2 *fin, double
 // taken (0.26 ms for the band's 0.54 at 509 slices of 255^2).  Few want the
 // many wavefronts of the band or the lines: the band where 8 columns on a side
 // hold the step size (timed against the strips, on the field itself: both
-// leave it alone), else the lines, up to half as many strips as SIMDs.  The
-// window recurrences and Thomas remain for what none of these takes.
+// leave it alone), else the lines, up to half as many strips as SIMDs.  Where
+// no strip holds the step size the lines are taken for any number of slices
+// (lines | Thomas, ms: 1024 slices of 151^2 0.65 | 1.96, 4096 of 61^2 0.62 |
+// 1.42, 509 of 255^2 0.89 | 2.71).  Grids beyond the lines' 512 time a wider
+// band against the strips, and Thomas is left what none of these takes.  The
+// window recurrences, slower than the strips wherever they apply, run by
+// request only.
 static int tune_adi(Ctx *c, const AdiField &a, double2 *field, double2 *work, int *choice, float *ms) {
     std::fill(ms, ms + 5, -1.f);
     const AdiPlan &p = *a.p;
@@ -700,29 +705,19 @@ static int tune_adi(Ctx *c, const AdiField &a, double2 *field, double2 *work, in
         *choice = 5;
         return G4MI_OK;
     }
-    const bool out = adi_eligible(a, 3) || adi_eligible(a, 4);
-    std::vector<int> kinds;
-    for (int kind = 0; kind < 5; kind++)
-        if (adi_eligible(a, kind) && (kind >= 3) == out) kinds.push_back(kind);
-    *choice = kinds[0];
-    if (kinds.size() == 1) return G4MI_OK;
-    const size_t bytes = (size_t)c->ns * a.ng * a.ng * sizeof(double2);
-    double2 *scratch = nullptr;
-    if (!out) {
-        G4_HIP(hipMalloc(&scratch, bytes));
-        G4_HIP(hipMemcpyAsync(scratch, field, bytes, hipMemcpyDeviceToDevice, c->stream));
-    }
-    double2 *const fin = out ? field : scratch;
+    const bool band = adi_eligible(a, 3), strip = adi_eligible(a, 4);
+    *choice = band ? 3 : strip ? 4 : 0;
+    if (!(band && strip)) return G4MI_OK;
     hipEvent_t e0, e1;
     G4_HIP(hipEventCreate(&e0));
     G4_HIP(hipEventCreate(&e1));
     float best_ms = 1e30f;
-    for (int kind : kinds) {
-        adi_launch(c, kind, a, fin, work);  // warm-up
+    for (int kind : {3, 4}) {
+        adi_launch(c, kind, a, field, work);  // warm-up
         float best = 1e30f;
         for (int rep = 0; rep < 3; rep++) {
             G4_HIP(hipEventRecord(e0, c->stream));
-            adi_launch(c, kind, a, fin, work);
+            adi_launch(c, kind, a, field, work);
             G4_HIP(hipEventRecord(e1, c->stream));
             G4_HIP(hipEventSynchronize(e1));
             float t = 0;
@@ -738,7 +733,6 @@ static int tune_adi(Ctx *c, const AdiField &a, double2 *field, double2 *work, in
     G4_HIP(hipGetLastError());
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    if (scratch) G4_HIP(hipFree(scratch));
     return G4MI_OK;
 }
 

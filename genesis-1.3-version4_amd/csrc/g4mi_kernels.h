@@ -122,12 +122,12 @@ int launch_adi_fused(hipStream_t s, int ns, double2 *field, double2 *work, const
 // [ngrid][2M+1] complex rows of A^-1 around the diagonal, a = Im(cstep).
 // m: 7, 8 or 12.  Rows [klo, khi] of the band equal row (klo+khi)/2 to
 // 2^-60.  tilediag: scratch [ns][adi_band_tiles(ngrid)][8], or null: no
-// field sums; diag null: the tiles' sums are left for launch_tile_sums.
+// field sums; launch_tile_sums folds them.
 int adi_band_tiles(int ng);
 void launch_tile_sums(hipStream_t s, int ns, const double *tilediag, int ntiles, double *diag);
 int launch_adi_band(hipStream_t s, int ns, const double2 *fin, double2 *fout, const double2 *src,
                     const int4 *box, const double2 *band, double a, int ng, int first, int m,
-                    int klo, int khi, double *tilediag, double *diag);
+                    int klo, int khi, double *tilediag);
 // Both half steps in strips of columns, one wavefront each (any grid):
 // tilediag [ns][strip_dims(form).count(ng)][8] or null.
 void launch_adi_strip(hipStream_t s, int ns, const double2 *fin, double2 *fout, const double2 *src, const int4 *box,

@@ -2663,8 +2663,7 @@ void launch_adi_strip(hipStream_t s, int ns, const double2 *fin, double2 *fout, 
 template <int M>
 static void launch_adi_band_t(hipStream_t s, int ns, const double2 *fin, double2 *fout,
                               const double2 *src, const int4 *box, const double2 *band, double a,
-                              int ng, int first, int klo, int khi, double *tilediag,
-                              double *diag) {
+                              int ng, int first, int klo, int khi, double *tilediag) {
     constexpr int TS = BandGeom<M>::TS;
     static bool attr = false;
     const size_t lds = BandGeom<M>::lds_cells * sizeof(double2);
@@ -2677,7 +2676,6 @@ static void launch_adi_band_t(hipStream_t s, int ns, const double2 *fin, double2
     const unsigned nblocks = (unsigned)(((ns + 7) / 8) * 8) * (unsigned)(ntx * ntx);
     hipLaunchKernelGGL(k_adi_band<M>, dim3(nblocks), dim3(256), lds, s, fin, fout, src, box,
                        band, a, ng, first, ns, ntx, klo, khi, tilediag);
-    if (tilediag && diag) launch_tile_sums(s, ns, tilediag, ntx * ntx, diag);
 }
 
 int adi_band_tiles(int ng) {
@@ -2687,8 +2685,8 @@ int adi_band_tiles(int ng) {
 
 int launch_adi_band(hipStream_t s, int ns, const double2 *fin, double2 *fout, const double2 *src,
                     const int4 *box, const double2 *band, double a, int ng, int first, int m,
-                    int klo, int khi, double *tilediag, double *diag) {
-#define G4_BAND(MM) launch_adi_band_t<MM>(s, ns, fin, fout, src, box, band, a, ng, first, klo, khi, tilediag, diag)
+                    int klo, int khi, double *tilediag) {
+#define G4_BAND(MM) launch_adi_band_t<MM>(s, ns, fin, fout, src, box, band, a, ng, first, klo, khi, tilediag)
     if (m == 7) G4_BAND(7);
     else if (m == 8) G4_BAND(8);
     else if (m == 12) G4_BAND(12);

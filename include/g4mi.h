@@ -241,10 +241,9 @@ int g4mi_sort_index_noalloc(g4mi_ctx *ctx, double slen, int *atar, long long *mo
  * kernel that suits its grid, step and number of slices: 0 Thomas' algorithm
  * in two kernels, 1 and 2 the fused recurrence without and with prefetch,
  * 3 banded inverse in 32x32 tiles, 4 strips of whole columns, 5 a wavefront
- * per line; 3 against 4
- * where either can be the faster, and the recurrences where neither holds the
- * step, are timed (the library's autotuner).  g4mi_set_schedule
- * fixes an entry instead ("adi_kernel": 0..5, -1 re-enables tuning; a step
+ * per line; 3 and 4 are timed (the library's autotuner) where either can be
+ * the faster, the others follow a rule, and 1 and 2 run by request only.
+ * g4mi_set_schedule fixes an entry instead ("adi_kernel": 0..5, -1 re-enables tuning; a step
  * size that the kernel does not hold takes the tuner's choice);
  * g4mi_get_schedule writes the current choice
  * and the measured timings as a JSON object into buf.  "fp64_fused": the step's

@@ -239,3 +239,27 @@ def test_step_size_that_is_no_number():
         assert np.all(np.isnan(ctx.download_field()[0]))
         assert ctx.schedule()["adi_by_delz"] == before
     ctx.close()
+
+
+@pytest.mark.parametrize("ngrid,ns,delz,kernels", [
+    (151, 2, 0.015, ("band", "strips")), (61, 511, 0.015, ("band", "strips")), (61, 512, 0.015, ("strips",)),
+    (151, 2, 0.2, ("lines",)), (61, 255, 0.2, ("lines",)), (61, 256, 0.2, ("strips",)),
+    (151, 2, 5.0, ("lines",)), (31, 1024, 5.0, ("lines",)), (151, 2, 4000.0, ("thomas",)),
+    (521, 2, 0.2, ("band", "strips")), (521, 2, 0.6, ("strips",)), (521, 2, 5.0, ("thomas",))])
+def test_choice_of_kernel(ngrid, ns, delz, kernels):
+    """The rule on both sides of its lines (8 columns of the band, half a strip
+    and one strip per SIMD, the strips' and the lines' step sizes, grids of
+    512), and the kernel chosen against the oracle."""
+    sim = H.make_state([4] * ns, ngrid=ngrid, gridmax=0.5e-3 * (ngrid - 1) / 150, timerun=False)
+    sim.field[:] = np.random.default_rng(ns).normal(size=sim.field.shape) * 1e9
+    ctx = H.to_gpu(sim)
+    st = H.steps(1, 2)
+    st[0].aw = 0
+    ctx.field_track(H.gsteps(st)[0], delz)
+    sch = ctx.schedule()
+    assert sch["adi"] in kernels, sch
+    assert sum(m > 0 for m in sch["adi_tuned_ms"]) == (2 if len(kernels) == 2 else 0)
+    H.oracle_call("orc_field_advance", sim, C.byref(st[0]), C.c_double(delz))
+    f, _ = ctx.download_field()
+    assert np.max(np.abs(f - sim.field)) < 1e-13 * np.max(np.abs(sim.field))
+    ctx.close()
