@@ -62,14 +62,19 @@ __device__ __forceinline__ double2 cpow_int(double2 z, int n) {
 //
 // These kernels are bound by FP64 issue, and most of their instructions were
 // the compiler's general divide (12 of them), square root (21) and sincos
-// (~100 on its near path).  The operands here are normal numbers far from
-// overflow, so the scaling and fix-up steps of the general forms go:
+// (~100 on its near path).  On normal operands whose quotient is normal the
+// scaling and fix-up steps of the general forms can go:
 //  * quot(a, recip(b)) is the correctly rounded quotient of the general form
 //    (Newton on v_rcp_f64, then one correction with the exact remainder:
 //    Markstein, IBM J. Res. Dev. 34 (1990) 111), and one reciprocal serves
 //    every division by the same b;
 //  * root(a) is the correctly rounded square root (Goldschmidt on v_rsq_f64
-//    with two exact-remainder corrections) of a normal a > 0;
+//    with two exact-remainder corrections) of a normal a > 0.
+//    Both give NaN for operands that have overflowed or vanished, so their
+//    callers test one value in their place and go to the general forms: before
+//    (transverse_one) or after, where any such operand shows up as a NaN
+//    (Ode::eval).  A fix-up at each quotient and root took 15 us of
+//    k_fp64_main's 435 (1024 x 8192 particles, 151^2);
 //  * sincos64 reduces by Cody and Waite's two-part pi/2 (exact products by
 //    FMA), carries the remainder's rounding along, and evaluates degree-5
 //    polynomials in r^2 interpolated at the Chebyshev nodes of [0, (pi/4)^2]
@@ -107,6 +112,20 @@ __device__ __forceinline__ double root(double a) {
     g = __builtin_fma(__builtin_fma(-g, g, a), h, g);
     return __builtin_fma(__builtin_fma(-g, g, a), h, g);
 }
+// v_cmp_class masks
+constexpr int kPosNormal = 0x100, kFinite = 0x1f8;
+// The two ways to the same quotients and roots: on operands that are known to
+// be normal, and on any.
+struct NormalOps {
+    static __device__ __forceinline__ Recip over(double b) { return recip(b); }
+    static __device__ __forceinline__ double div(double a, const Recip &r) { return quot(a, r); }
+    static __device__ __forceinline__ double rt(double a) { return root(a); }
+};
+struct AnyOps {
+    static __device__ __forceinline__ Recip over(double b) { return {b, 0}; }
+    static __device__ __forceinline__ double div(double a, const Recip &r) { return a / r.b; }
+    static __device__ __forceinline__ double rt(double a) { return sqrt(a); }
+};
 __device__ __forceinline__ void sincos64(double x, double *s, double *c) {
     if (__builtin_expect(!(fabs(x) < 0x1p45), 0)) x = fmod(x, 0x1.921fb54442d18p+2);
     const double kb = x * 0x1.45f306dc9c883p-1 + 0x1.8p52;  // the multiple in the low bits
@@ -160,24 +179,24 @@ __device__ __forceinline__ void block_sum(double (&v)[K], double *lds) {
 // chicane matrix application (:223-236).
 // ---------------------------------------------------------------------------
 // DEFOC: lines that defocus (quadrupoles) are among them
-template <bool DEFOC = true>
+template <class Ops, bool DEFOC>
 __device__ __forceinline__ void line_map(int kind, double delz, double q, double &x, double &px,
                                          const Recip &gz, double d) {
     if (kind == 0) {
-        x += quot(px * delz, gz);
+        x += Ops::div(px * delz, gz);
     } else if (kind > 0) {
-        double foc = root(quot(q, gz)), omg = foc * delz;
+        double foc = Ops::rt(Ops::div(q, gz)), omg = foc * delz;
         double s, c;
         sincos64(omg, &s, &c);
-        double a1 = c, a2 = quot(s, recip(foc)), a3 = -a2 * foc * foc;
+        double a1 = c, a2 = Ops::div(s, Ops::over(foc)), a3 = -a2 * foc * foc;
         double xtmp = x - d;
-        x = a1 * xtmp + quot(a2 * px, gz) + d;
+        x = a1 * xtmp + Ops::div(a2 * px, gz) + d;
         px = a3 * xtmp * gz.b + a1 * px;
     } else if (DEFOC) {
-        double foc = root(quot(-q, gz)), omg = foc * delz;
-        double a1 = cosh(omg), a2 = quot(sinh(omg), recip(foc)), a3 = a2 * foc * foc;
+        double foc = Ops::rt(Ops::div(-q, gz)), omg = foc * delz;
+        double a1 = cosh(omg), a2 = Ops::div(sinh(omg), Ops::over(foc)), a3 = a2 * foc * foc;
         double xtmp = x - d;
-        x = a1 * xtmp + quot(a2 * px, gz) + d;
+        x = a1 * xtmp + Ops::div(a2 * px, gz) + d;
         px = a3 * xtmp * gz.b + a1 * px;
     }
 }
@@ -198,9 +217,16 @@ __device__ __forceinline__ void transverse_one(const TransParams &p, double gi, 
         yi = p.m22 * t + p.m23 * pyi / gz;
         pyi = p.m32 * t * gz + p.m33 * pyi;
     }
-    const Recip gammaz = recip(root(gi * gi - 1 - p.aw * p.aw - pxi * pxi - pyi * pyi));
-    line_map<DEFOC>(p.kindx, p.delz, p.qx, xi, pxi, gammaz, p.xoff);
-    line_map<DEFOC>(p.kindy, p.delz, p.qy, yi, pyi, gammaz, p.yoff);
+    const double gz2 = gi * gi - 1 - p.aw * p.aw - pxi * pxi - pyi * pyi;
+    auto lines = [&](auto ops) {
+        typedef decltype(ops) Ops;
+        const Recip gammaz = Ops::over(Ops::rt(gz2));
+        line_map<Ops, DEFOC>(p.kindx, p.delz, p.qx, xi, pxi, gammaz, p.xoff);
+        line_map<Ops, DEFOC>(p.kindy, p.delz, p.qy, yi, pyi, gammaz, p.yoff);
+    };
+    // finite and positive: so are gamma and the momenta
+    if (__builtin_expect(__builtin_amdgcn_class(gz2, kPosNormal), 1)) lines(NormalOps{});
+    else lines(AnyOps{});
 }
 
 __global__ void __launch_bounds__(256) k_transverse(long long n, const double *__restrict__ g,
@@ -484,8 +510,14 @@ struct Ode {
         double btper0 = btpar + ztemp1 * ctmp.x;
         const Recip rg = recip(tgam);
         const Recip rb = recip(root(1. - quot(btper0, recip_sq(rg))));
-        k2pp += xks * (1. - quot(1.0, rb)) + xku;
-        k2gg += quot(quot(ctmp.y, rb), rg) - ez;
+        double ib = quot(1.0, rb), dg = quot(quot(ctmp.y, rb), rg);
+        if (__builtin_expect(!__builtin_amdgcn_class(ib + dg, kFinite), 0)) {
+            const double btpar0 = sqrt(1. - btper0 / (tgam * tgam));
+            ib = 1. / btpar0;
+            dg = ctmp.y / btpar0 / tgam;
+        }
+        k2pp += xks * (1. - ib) + xku;
+        k2gg += dg - ez;
     }
 };
 
@@ -1175,7 +1207,8 @@ __global__ void __launch_bounds__(kFuseNT, GEN ? 2 : 4) k_fp64_main(const long l
             by1 = max(by1, iy + 1);
             const double ddx = xi - d.ax, ddy = yi - d.ay;
             const double faw2 = (1 + d.kx * ddx * ddx + d.ky * ddy * ddy + 2 * (d.gradx * ddx + d.grady * ddy));
-            const double part = quot(sqrt(faw2) * scl, recip(gamma));
+            const double num = sqrt(faw2) * scl;
+            const double part = __builtin_amdgcn_div_fixup(quot(num, recip(gamma)), gamma, num);
             v[8] += fabs(part);
             if (fused) {
                 if (ix >= tx0 && ix + 1 < tx0 + tw && iy >= ty0 && iy + 1 < ty0 + tht) {
