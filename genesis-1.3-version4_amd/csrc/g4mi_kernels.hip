@@ -79,9 +79,8 @@ __device__ __forceinline__ double2 cpow_int(double2 z, int n) {
 //    FMA), carries the remainder's rounding along, and evaluates degree-5
 //    polynomials in r^2 interpolated at the Chebyshev nodes of [0, (pi/4)^2]
 //    (errors 1.3e-17 and 5e-19).  At most 0.93 ulp off, 2.8e-17 rms (a
-//    correctly rounded result: 2.7e-17) over |x| up to 5e8.  From 2^45 on,
-//    where neighbouring doubles lie 0.008 rad apart, the phase is first
-//    taken modulo the double nearest 2 pi: off by less than that spacing.
+//    correctly rounded result: 2.7e-17) over |x| up to 5e8.  From 2^45 on the
+//    reduction multiplies by as many bits of 2/pi as the phase needs.
 // ---------------------------------------------------------------------------
 struct Recip {
     double b, y;  // y = 1/b to an ulp
@@ -126,13 +125,49 @@ struct AnyOps {
     static __device__ __forceinline__ double div(double a, const Recip &r) { return a / r.b; }
     static __device__ __forceinline__ double rt(double a) { return sqrt(a); }
 };
+// 2/pi: 64 zero bits, then its first 1216 (from Machin's formula in integers)
+__device__ const unsigned long long kTwoOverPi[20] = {
+    0x0000000000000000ull, 0xa2f9836e4e441529ull, 0xfc2757d1f534ddc0ull, 0xdb6295993c439041ull,
+    0xfe5163abdebbc561ull, 0xb7246e3a424dd2e0ull, 0x06492eea09d1921cull, 0xfe1deb1cb129a73eull,
+    0xe88235f52ebb4484ull, 0xe99c7026b45f7e41ull, 0x3991d639835339f4ull, 0x9c845f8bbdf9283bull,
+    0x1ff897ffde05980full, 0xef2f118b5a0a6d1full, 0x6d367ecf27cb09b7ull, 0x4f463f669e5fea2dull,
+    0x7527bac7ebe5f17bull, 0x3d0739f78a5292eaull, 0x6bfb5fb11f8d5d08ull, 0x56033046fc7b6babull
+};
+// x = n pi/2 + r + tail for |x| >= 2^45 (Payne and Hanek, ACM SIGNUM Newsl. 18
+// (1983) 19): the 53-bit integer of x times the 192 bits of 2/pi that decide
+// the quarter turns modulo 4 and the fraction to 2^-137.
+__device__ __forceinline__ void reduce_far(double x, int *n, double *r, double *tail) {
+    typedef unsigned long long u64;
+    const u64 bits = (u64)__double_as_longlong(x);
+    const int ex = (int)(bits >> 52) & 0x7ff;
+    const u64 m = (bits & 0xfffffffffffffull) | 0x10000000000000ull;
+    const int p = min(ex, 2046) - 1013;  // of the first bit that counts: weight 2 times the integer's unit
+    const u64 *t = kTwoOverPi + (p >> 6);
+    const int sh = p & 63;
+    auto word = [&](int q) -> u64 { return (t[q] << sh) | ((t[q + 1] >> 1) >> (63 - sh)); };
+    const u64 w1 = word(1), low = m * w1;
+    const u64 mid = low + __umul64hi(m, word(2));
+    const u64 top = m * word(0) + __umul64hi(m, w1) + (mid < low ? 1 : 0);
+    const long long f = (long long)((top << 2) | (mid >> 62));  // the fraction of a quarter turn, in [-1/2, 1/2)
+    const double fh = (double)(f & ~0x7ffll) * 0x1p-64;
+    const double fl = ((double)(f & 0x7ff) + (double)(mid << 2) * 0x1p-64) * 0x1p-64;
+    double a = fh + fl, b = fl - (a - fh);
+    int q = (int)(top >> 62) + (f < 0 ? 1 : 0);
+    if (__double2hiint(x) < 0) a = -a, b = -b, q = -q;
+    if (ex == 2047) a = __longlong_as_double(0x7ff8000000000000ll);
+    *n = q;
+    *r = a * 0x1.921fb54442d18p+0;
+    *tail = __builtin_fma(a, 0x1.921fb54442d18p+0, -*r) +
+            __builtin_fma(a, 0x1.1a62633145c07p-54, b * 0x1.921fb54442d18p+0);
+}
 __device__ __forceinline__ void sincos64(double x, double *s, double *c) {
-    if (__builtin_expect(!(fabs(x) < 0x1p45), 0)) x = fmod(x, 0x1.921fb54442d18p+2);
     const double kb = x * 0x1.45f306dc9c883p-1 + 0x1.8p52;  // the multiple in the low bits
     const double k = kb - 0x1.8p52;
     const double u = __builtin_fma(-k, 0x1.921fb54442d18p+0, x);
-    const double r = __builtin_fma(-k, 0x1.1a62633145c07p-54, u);
-    const double tail = __builtin_fma(-k, 0x1.1a62633145c07p-54, u - r);
+    double r = __builtin_fma(-k, 0x1.1a62633145c07p-54, u);
+    double tail = __builtin_fma(-k, 0x1.1a62633145c07p-54, u - r);
+    int n = __double2loint(kb);
+    if (__builtin_expect(!(fabs(x) < 0x1p45), 0)) reduce_far(x, &n, &r, &tail);
     const double z = r * r;
     double p = __builtin_fma(0x1.5e0b19ee56c63p-33, z, -0x1.ae600b0299686p-26);
     double q = __builtin_fma(-0x1.907da35d467bfp-37, z, 0x1.1eeb68e92d026p-29);
@@ -147,7 +182,6 @@ __device__ __forceinline__ void sincos64(double x, double *s, double *c) {
     const double sn = r + __builtin_fma(r * z, p, tail);
     const double w = __builtin_fma(-0.5, z, 1.0);
     const double cs = w + __builtin_fma(z * z, q, __builtin_fma(-r, tail, __builtin_fma(-0.5, z, 1.0 - w)));
-    const int n = __double2loint(kb);
     const double a = (n & 1) ? cs : sn, b = (n & 1) ? sn : cs;
     *s = __hiloint2double(__double2hiint(a) ^ ((n << 30) & (int)0x80000000), __double2loint(a));
     *c = __hiloint2double(__double2hiint(b) ^ (((n + 1) << 30) & (int)0x80000000), __double2loint(b));
@@ -859,7 +893,7 @@ constexpr int kFuseTile = kFuseDyn - kFuseModes;        // deposit tile cells
 static_assert(kFuseNW * kScMaxNg + 4 * kScMaxNg <= kFuseTile && kFuseNT >= kScMaxNg,
               "the short-range solver's scratch must fit in the tile region");
 
-__global__ void __launch_bounds__(kFrontNT) k_fp64_front(const long long *__restrict__ off,
+__global__ void __launch_bounds__(kFrontNT, 4) k_fp64_front(const long long *__restrict__ off,
                                                         const double *__restrict__ g, double *__restrict__ x,
                                                         double *__restrict__ y, double *__restrict__ px,
                                                         double *__restrict__ py, const double *__restrict__ cur,
