@@ -160,6 +160,11 @@ __device__ __forceinline__ void reduce_far(double x, int *n, double *r, double *
     *tail = __builtin_fma(a, 0x1.921fb54442d18p+0, -*r) +
             __builtin_fma(a, 0x1.1a62633145c07p-54, b * 0x1.921fb54442d18p+0);
 }
+// AHEAD: the near reduction is kept ahead of the branch to the far one.  Left to
+// itself the compiler makes it that branch's other arm, and in a short loop over
+// the particles the loads that follow wait for the phase (k_sc_solve 75 us, 91
+// without); k_fp64_main is the faster without (438 us, 445 with).
+template <bool AHEAD = false>
 __device__ __forceinline__ void sincos64(double x, double *s, double *c) {
     const double kb = x * 0x1.45f306dc9c883p-1 + 0x1.8p52;  // the multiple in the low bits
     const double k = kb - 0x1.8p52;
@@ -167,6 +172,7 @@ __device__ __forceinline__ void sincos64(double x, double *s, double *c) {
     double r = __builtin_fma(-k, 0x1.1a62633145c07p-54, u);
     double tail = __builtin_fma(-k, 0x1.1a62633145c07p-54, u - r);
     int n = __double2loint(kb);
+    if (AHEAD) asm volatile("" : "+v"(r), "+v"(tail), "+v"(n));
     if (__builtin_expect(!(fabs(x) < 0x1p45), 0)) reduce_far(x, &n, &r, &tail);
     const double z = r * r;
     double p = __builtin_fma(0x1.5e0b19ee56c63p-33, z, -0x1.ae600b0299686p-26);
@@ -477,7 +483,7 @@ __global__ void __launch_bounds__(256) k_sc_solve(
                 int bin = (int)floor(radi / dr);
                 bin = (bin >= 0 && bin < ngr) ? bin : (bin >= ngr ? ngr - 1 : 0);
                 double s, c;
-                sincos64(l * th[i], &s, &c);
+                sincos64<true>(l * th[i], &s, &c);
                 double2 v = make_double2(c, -s);
                 if (m != 0)  // cwork^0 is exactly 1: the azimuthal factor only for m != 0
                     v = cmul(cpow_int(make_double2(tx / radi, ty / radi), -m), v);
@@ -505,7 +511,7 @@ __global__ void __launch_bounds__(256) k_sc_solve(
                 int bin = (int)floor(radi / dr);
                 bin = (bin >= 0 && bin < ngr) ? bin : (bin >= ngr ? ngr - 1 : 0);
                 double s, c;
-                sincos64(l * th[i], &s, &c);
+                sincos64<true>(l * th[i], &s, &c);
                 double2 ct = make_double2(c, s);
                 if (m != 0) ct = cmul(cpow_int(make_double2(tx / radi, ty / radi), m), ct);
                 ez[i] += 2 * cmul(ct, celm[bin]).x;
@@ -1012,7 +1018,8 @@ __global__ void __launch_bounds__(kFrontNT, 4) k_fp64_front(const long long *__r
 // step takes, is small enough for four wavefronts per SIMD (two workgroups
 // per CU, what the LDS allows): 1024 x 8192 particles with space charge
 // 433 us against 498 us at the two its 170 registers would give by
-// themselves, and 678 us with the general divide, square root and sincos.
+// themselves, and 678 us with the general divide, square root and sincos;
+// 440 us since operands that overflowed and phases beyond 2^45 are looked for.
 template <bool GEN>
 __global__ void __launch_bounds__(kFuseNT, GEN ? 2 : 4) k_fp64_main(const long long *__restrict__ off, double *__restrict__ g,
                                                        double *__restrict__ th, double *__restrict__ x,

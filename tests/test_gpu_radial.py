@@ -16,13 +16,13 @@ COUNTS = [1024, 64, 256, 768]
 @pytest.mark.parametrize("nz,nphi", [(1, 0), (2, 1)])
 @pytest.mark.parametrize("ngr", [3, 4, 5, 63, 64, 65, 100, 129, 255, 256])
 def test_radial_grids(ngr, nz, nphi):
-    """FP64 form, separate and fused kernels: the on-axis field and the
+    """FP64 form, separate, fused and split kernels: the on-axis field and the
     energies after two steps (the oracle's recurrence and the reduction are
     two orders of the same eliminations: 1e-12)."""
     st = H.steps(1, 2)[:2]
     sim = H.make_state(COUNTS, ngrid=41, sc=(nz, nphi, ngr, 0.0), seed_power=1e6)
     ctxs = []
-    for fused in (0, 1):
+    for fused in (0, 1, -1):
         ctx = H.to_gpu(sim)
         ctx.set_schedule("fp64_fused", fused)
         ctx.run(H.gsteps(st), cases.GAMMA0, record=())
