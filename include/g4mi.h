@@ -243,15 +243,15 @@ int g4mi_sort_index_noalloc(g4mi_ctx *ctx, double slen, int *atar, long long *mo
  * 3 banded inverse in 32x32 tiles, 4 strips of whole columns, 5 a wavefront
  * per line; 3 and 4 are timed (the library's autotuner) where either can be
  * the faster, the others follow a rule, and 1 and 2 run by request only.
- * g4mi_set_schedule fixes an entry instead ("adi_kernel": 0..5, -1 re-enables tuning; a step
- * size that the kernel does not hold takes the tuner's choice);
- * g4mi_get_schedule writes the current choice
- * and the measured timings as a JSON object into buf.  "fp64_fused": the step's
- * particle passes where the step allows them, 1 as two fused kernels (one
- * workgroup per slice), 0 as the separate kernels, -1 (the default) fused for
- * windows of 256 slices or more and else over blocks of the particles with a
- * split deposit; "particle_passes" reports which a plain step takes.  The
- * spectral solver's first step likewise times its
+ * g4mi_set_schedule fixes an entry instead ("adi_kernel": 0..5, -1 re-enables
+ * tuning; a step size that the kernel does not hold takes the tuner's choice,
+ * and the next one that it does hold takes the kernel); g4mi_get_schedule
+ * writes the current choice and the measured timings as a JSON object into
+ * buf.  "fp64_fused": the step's particle passes where the step allows them, 1
+ * as two fused kernels (one workgroup per slice), 0 as the separate kernels, -1
+ * (the default) fused for windows of 256 slices or more and else over blocks of
+ * the particles with a split deposit; "particle_passes" reports which a plain
+ * step takes.  The spectral solver's first step likewise times its
  * complex-GEMM variants ("fft_variant": 0 four real products per complex
  * one and k chunks of 16, 1 three products, 2 four products with chunks of
  * 32, 3 three with 32; -1 tunes again) and its propagation by those GEMMs
@@ -262,7 +262,8 @@ int g4mi_sort_index_noalloc(g4mi_ctx *ctx, double slen, int *atar, long long *mo
  * (unless "fft_propagation" is 0) compute their DFTs as Bluestein chirp
  * convolutions on the same FFTs for ngrid <= 256.
  * Mixed form: its first 18 steps time the main kernel's shapes (4, 6 or 8
- * wavefronts per slice x 68 or 44 KiB of LDS, 4 or 6 x 32 KiB), the three ADI kernels,
+ * wavefronts per slice x 68 or 44 KiB of LDS, 4 or 6 x 32 KiB), the three ADI
+ * kernels (from 1024 column strips on these alone),
  * and the step as a graph of kernels against one persistent
  * cooperative launch, and keep the fastest.  Entries: "adi_refine" (FP64
  * residual correction of its FP32 band products, default 1), "mixed_adi" (2
